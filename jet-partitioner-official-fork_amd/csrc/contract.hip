@@ -24,6 +24,12 @@ constexpr int32_t T1_MAX = 128;   // hsize bound for the wave tier
 constexpr int32_t T1_CAP = 256;   // wave LDS table slots
 constexpr int32_t T2_MAX = 4096;  // hsize bound for the workgroup tier
 constexpr int32_t T2_CAP = 8192;  // workgroup LDS table slots
+// The workgroup tier runs in two sizes, so that its many short rows do not
+// hold the long rows' LDS: up to T2S_MAX fine edges a 256-thread workgroup
+// with 2048 slots (8 of them fit a CU), above that 1024 threads with 8192
+// slots (2 fit). One size of 256 threads and 8192 slots left 8 waves a CU.
+constexpr int32_t T2S_MAX = 1024;
+constexpr int32_t T2S_CAP = 2048;
 constexpr int32_t EMPTY = -1;
 
 __device__ inline uint32_t slot_hash(vid_t u) { return (uint32_t)u * 0x9E3779B1u; }
@@ -45,18 +51,20 @@ __global__ void k_members(vid_t n, const vid_t* map, const int32_t* moff, int32_
 }
 
 __global__ void __launch_bounds__(256)
-    k_tiers(vid_t nc, const eoff_t* hoff, vid_t* l1, vid_t* l2, vid_t* l3, int32_t* cnt, int32_t t1max,
+    k_tiers(vid_t nc, const eoff_t* hoff, vid_t* l1, vid_t* l2, vid_t* l3, vid_t* l4, int32_t* cnt, int32_t t1max,
             int32_t t2max) {
     __shared__ int32_t sh[256 / WAVE + 1];
     FOR_BLOCK_UNIFORM(c, nc) {
         const bool in = c < nc;
         const eoff_t hs = in ? hoff[c + 1] - hoff[c] : 0;
         int32_t a = block_append<256>(&cnt[0], in && hs <= t1max, sh);
-        int32_t b = block_append<256>(&cnt[1], in && hs > t1max && hs <= t2max, sh);
+        int32_t b = block_append<256>(&cnt[1], in && hs > t1max && hs <= t2max && hs <= T2S_MAX, sh);
+        int32_t e = block_append<256>(&cnt[3], in && hs > t1max && hs <= t2max && hs > T2S_MAX, sh);
         int32_t d = block_append<256>(&cnt[2], in && hs > t2max, sh);
         if (a >= 0) l1[a] = (vid_t)c;
         if (b >= 0) l2[b] = (vid_t)c;
         if (d >= 0) l3[d] = (vid_t)c;
+        if (e >= 0) l4[e] = (vid_t)c;
     }
 }
 
@@ -169,32 +177,33 @@ __global__ void __launch_bounds__(T1_WAVES* WAVE)
     }
 }
 
-constexpr int T2_BLOCK = 256;
-
-__global__ void __launch_bounds__(T2_BLOCK)
+// One workgroup per row: hash into LDS, compact the unique entries (they fill
+// at most half of the table), then bitonic-sort only those. Sorting the whole
+// table took four times the exchanges: 7.5 ms a call on R-MAT 22's levels.
+template <int BLOCK, int CAP>
+__global__ void __launch_bounds__(BLOCK)
     k_dedupe_block(DGraph g, const vid_t* map, const vid_t* members, const int32_t* moff, const eoff_t* hoff,
-                   const vid_t* list, const int32_t* cnt, vid_t* tkey, wgt_t* tval, int32_t* ucount) {
-    __shared__ int32_t keys[T2_CAP];
-    __shared__ int32_t vals[T2_CAP];
-    __shared__ int32_t ucnt;
-    const int32_t nrows = cnt[1];
+                   const vid_t* list, int32_t nrows, vid_t* tkey, wgt_t* tval, int32_t* ucount) {
+    __shared__ int32_t keys[CAP];
+    __shared__ int32_t vals[CAP];
+    __shared__ int32_t ws[BLOCK / WAVE + 1];
+    constexpr int PER = CAP / BLOCK;
     for (int32_t r = blockIdx.x; r < nrows; r += gridDim.x) {
         vid_t c = list[r];
         eoff_t hs = hoff[c];
         int32_t hsz = (int32_t)(hoff[c + 1] - hs);
         uint32_t cap = 256;
         while ((int32_t)cap < 2 * hsz) cap <<= 1;
-        for (uint32_t t = threadIdx.x; t < cap; t += T2_BLOCK) {
+        for (uint32_t t = threadIdx.x; t < cap; t += BLOCK) {
             keys[t] = EMPTY;
             vals[t] = 0;
         }
-        if (threadIdx.x == 0) ucnt = 0;
         __syncthreads();
         int32_t mb = moff[c], me = moff[c + 1];
         const int lane = threadIdx.x & (WAVE - 1);
         const int wid = threadIdx.x / WAVE;
         // members round-robin over waves; each wave walks its member's row
-        for (int32_t mi = mb + wid; mi < me; mi += T2_BLOCK / WAVE) {
+        for (int32_t mi = mb + wid; mi < me; mi += BLOCK / WAVE) {
             vid_t i = members[mi];
             for (eoff_t j = g.rowptr[i] + lane; j < g.rowptr[i + 1]; j += WAVE) {
                 vid_t u = map[g.col[j]];
@@ -202,13 +211,33 @@ __global__ void __launch_bounds__(T2_BLOCK)
             }
         }
         __syncthreads();
-        for (uint32_t t = threadIdx.x; t < cap; t += T2_BLOCK)
-            if (keys[t] != EMPTY) atomicAdd(&ucnt, 1);
-        // bitonic sort of (key as unsigned, EMPTY last) over cap slots
-        for (uint32_t size = 2; size <= cap; size <<= 1) {
+        // the unique entries, packed to the front through registers
+        int32_t rk[PER], rv[PER];
+        int32_t mine = 0;
+#pragma unroll
+        for (int q = 0; q < PER; q++) {
+            const uint32_t t = threadIdx.x + (uint32_t)q * BLOCK;
+            rk[q] = t < cap ? keys[t] : EMPTY;
+            rv[q] = t < cap ? vals[t] : 0;
+            mine += rk[q] != EMPTY ? 1 : 0;
+        }
+        int32_t U;
+        int32_t at = block_excl_scan<int32_t, BLOCK>(mine, U, ws);
+        uint32_t scap = 2;
+        while ((int32_t)scap < U) scap <<= 1;
+#pragma unroll
+        for (int q = 0; q < PER; q++)
+            if (rk[q] != EMPTY) {
+                keys[at] = rk[q];
+                vals[at++] = rv[q];
+            }
+        // scap <= cap: U <= hsz <= cap / 2
+        for (uint32_t t = (uint32_t)U + threadIdx.x; t < scap; t += BLOCK) keys[t] = EMPTY;
+        // bitonic sort by key as unsigned (EMPTY last)
+        for (uint32_t size = 2; size <= scap; size <<= 1) {
             for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
                 __syncthreads();
-                for (uint32_t t = threadIdx.x; t < cap / 2; t += T2_BLOCK) {
+                for (uint32_t t = threadIdx.x; t < scap / 2; t += BLOCK) {
                     uint32_t lo = 2 * t - (t & (stride - 1));
                     uint32_t hi = lo + stride;
                     bool up = (lo & size) == 0;
@@ -224,8 +253,7 @@ __global__ void __launch_bounds__(T2_BLOCK)
             }
         }
         __syncthreads();
-        const int32_t U = ucnt;
-        for (int32_t e = threadIdx.x; e < U; e += T2_BLOCK) {
+        for (int32_t e = threadIdx.x; e < U; e += BLOCK) {
             tkey[hs + e] = keys[e];
             tval[hs + e] = vals[e];
         }
@@ -280,18 +308,42 @@ __global__ void k_spill_heads(const uint64_t* skey, int64_t len, int32_t* head) 
     }
 }
 
-__global__ void k_spill_reduce(const uint64_t* skey, const uint32_t* sval, int64_t len, const int32_t* uid_ex,
-                               const vid_t* list, int32_t* ukey, wgt_t* uval, int32_t* urow, int32_t* rowfirst) {
-    FOR_THREAD(t, len) {
-        uint64_t k = skey[t];
-        if (k == ~0ull) continue;
-        int32_t uid = uid_ex[t + 1] - 1;
-        atomicAdd(&uval[uid], (wgt_t)sval[t]);
-        if (uid_ex[t + 1] != uid_ex[t]) {
-            int32_t r = (int32_t)(k >> 32);
+// Sums the runs of equal keys. A hub row's runs are long (one entry per fine
+// edge between two aggregates), so each wave first sums its stretch of every
+// run with a segmented scan and adds once per wave and run; a row's first
+// unique entry is found by its neighbour's key instead of a minimum over the
+// row. With an atomic per entry, the entries of the few hub rows met on a few
+// addresses: 11.1 ms per call on R-MAT 22's levels (spill_write, which
+// counted a row's uniques with an atomic each, 10.5 ms).
+__global__ void __launch_bounds__(256)
+    k_spill_reduce(const uint64_t* skey, const uint32_t* sval, int64_t len, const int32_t* uid_ex, int32_t* ukey,
+                   wgt_t* uval, int32_t* urow, int32_t* rowfirst) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    for (int64_t t0 = blockIdx.x * (int64_t)256 + (threadIdx.x - lane); t0 < len; t0 += (int64_t)gridDim.x * 256) {
+        const int64_t t = t0 + lane;
+        const uint64_t k = t < len ? skey[t] : ~0ull;
+        const uint64_t kp = t > 0 && t < len ? skey[t - 1] : ~0ull;
+        const uint64_t kn = t + 1 < len ? skey[t + 1] : ~0ull;
+        const bool valid = k != ~0ull;
+        const bool head = t == 0 || k != kp;
+        wgt_t v = valid ? (wgt_t)sval[t] : 0;
+        const int32_t uid = valid ? uid_ex[t + 1] - 1 : 0;
+        // inclusive sum since the run's first entry in this wave
+        const uint64_t starts = __ballot(head || lane == 0);
+        const uint64_t upto = lane == WAVE - 1 ? starts : starts & ((2ull << lane) - 1ull);
+        const int start = 63 - __clzll((long long)upto);
+#pragma unroll
+        for (int d = 1; d < WAVE; d <<= 1) {
+            const wgt_t o = __shfl_up(v, d, WAVE);
+            if (lane - d >= start) v += o;
+        }
+        const bool last = lane == WAVE - 1 || kn != k;  // of the wave's stretch of the run
+        if (valid && last) atomicAdd(&uval[uid], v);
+        if (valid && head) {
+            const int32_t r = (int32_t)(k >> 32);
             ukey[uid] = (int32_t)(k & 0xffffffffull);
             urow[uid] = r;
-            atomicMin(&rowfirst[r], uid);
+            if (t == 0 || (int32_t)(kp >> 32) != r) rowfirst[r] = uid;
         }
     }
 }
@@ -305,7 +357,8 @@ __global__ void k_spill_write(int32_t U, const int32_t* ukey, const wgt_t* uval,
         int32_t off = (int32_t)e - rowfirst[r];
         tkey[hoff[c] + off] = ukey[e];
         tval[hoff[c] + off] = uval[e];
-        atomicAdd(&ucount[c], 1);
+        // the row's last unique entry knows its count
+        if (e + 1 == U || urow[e + 1] != r) ucount[c] = off + 1;
     }
 }
 
@@ -341,7 +394,7 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
     int32_t* mfill = a.alloc<int32_t>(nc);
     int32_t* ucount = a.alloc<int32_t>((int64_t)nc + 1);
     vid_t* members = a.alloc<vid_t>(g.n);
-    vid_t* lists = a.alloc<vid_t>(3 * (int64_t)nc);
+    vid_t* lists = a.alloc<vid_t>(4 * (int64_t)nc);
     int32_t* cnt = a.alloc<int32_t>(4);
     fill_i64(hoff, 0, (int64_t)nc + 1, s);
     fill_i32(out.vw, 0, nc, s);
@@ -358,10 +411,11 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
     vid_t* l1 = lists;
     vid_t* l2 = lists + nc;
     vid_t* l3 = lists + 2 * (int64_t)nc;
+    vid_t* l4 = lists + 3 * (int64_t)nc;
     // the tuned tier bounds never exceed T1_MAX / T2_MAX (half of each table)
     const int32_t t1max = (int32_t)std::min<int64_t>(T1_MAX, tuning().ct_wave_max);
     const int32_t t2max = (int32_t)std::min<int64_t>(T2_MAX, std::max<int64_t>(t1max, tuning().ct_block_max));
-    k_tiers<<<grid_for(nc, 256, 8192), 256, 0, s>>>(nc, hoff, l1, l2, l3, cnt, t1max, t2max);
+    k_tiers<<<grid_for(nc, 256, 8192), 256, 0, s>>>(nc, hoff, l1, l2, l3, l4, cnt, t1max, t2max);
     JET_LAUNCH_CHECK();
     int32_t hcnt[4];
     read_i32_words(cnt, 4, hcnt, s);
@@ -374,8 +428,13 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
         JET_LAUNCH_CHECK();
     }
     if (hcnt[1] > 0) {
-        k_dedupe_block<<<std::min(hcnt[1], 4096), T2_BLOCK, 0, s>>>(g, map, members, moff, hoff, l2, cnt, tkey, tval,
-                                                                    ucount);
+        k_dedupe_block<256, T2S_CAP><<<std::min(hcnt[1], 8192), 256, 0, s>>>(g, map, members, moff, hoff, l2, hcnt[1],
+                                                                            tkey, tval, ucount);
+        JET_LAUNCH_CHECK();
+    }
+    if (hcnt[3] > 0) {
+        k_dedupe_block<1024, T2_CAP><<<std::min(hcnt[3], 2048), 1024, 0, s>>>(g, map, members, moff, hoff, l4, hcnt[3],
+                                                                             tkey, tval, ucount);
         JET_LAUNCH_CHECK();
     }
     if (hcnt[2] > 0) {
@@ -406,8 +465,7 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
         int32_t* urow = a.alloc<int32_t>(U);
         int32_t* rowfirst = a.alloc<int32_t>(n3);
         fill_i32(uval, 0, U, s);
-        fill_i32(rowfirst, ORD_MAX, n3, s);
-        k_spill_reduce<<<hb, 256, 0, s>>>(skey, sval, H3, uid, l3, ukey, uval, urow, rowfirst);
+        k_spill_reduce<<<hb, 256, 0, s>>>(skey, sval, H3, uid, ukey, uval, urow, rowfirst);
         JET_LAUNCH_CHECK();
         if (U > 0) {
             k_spill_write<<<grid_for(U, 256, 8192), 256, 0, s>>>(U, ukey, uval, urow, rowfirst, l3, hoff, tkey, tval,
