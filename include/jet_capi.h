@@ -389,8 +389,9 @@ int jet_partition_batch(jet_ctx_t* ctx, int32_t count, const jet_config_t* cfgs,
  *   wider afterburner lane groups, 128-thread rebalancer select workgroups);
  * "ab_lanes_small", "upd_lanes": lane-group multipliers (1-4) of the
  *   afterburner on small levels and of the update passes;
- * "upd_big_slices": waves (1-64) that share the edges of one move of degree
- *   above 64 in the update passes;
+ * "upd_big_slices": moves and candidates of degree above 128 times this (1-64)
+ *   are taken by a whole workgroup in the update passes and the afterburner,
+ *   others of degree above 64 by a wave;
  * "lp_one_pass_n": LP select runs one pass per wave up to this level size;
  * "ct_wave_max", "ct_block_max": contraction rows of up to this many fine
  *   entries take the one-wave (<= 128) or one-workgroup (<= 4096) LDS table;

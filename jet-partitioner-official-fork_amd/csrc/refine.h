@@ -134,11 +134,12 @@ class Refiner {
     part_t* cur_part_;
     vid_t* tier_mid_;
     vid_t* tier_big_;
-    // rows of degree > BIG_DEG ("hubs": tier_big_ and pull_mid_) take their
-    // update_small changes through k_update_hubs: flags per vertex for hub
-    // and hub with a moved neighbour
+    // rows of degree > BIG_DEG ("hubs": tier_big_ and pull_mid_) take a step's
+    // changes through k_pull_hubs: flags per vertex for hub and hub with a
+    // moved neighbour, and a bit per vertex that moves in the current step
     uint8_t* hub_;
     uint8_t* hub_dirty_;
+    uint32_t* moved_bits_;
     // stamp_[v] == gen_: v is in the current step's move list (the move-list
     // producers write it; every selection step takes a new generation)
     int32_t* stamp_;

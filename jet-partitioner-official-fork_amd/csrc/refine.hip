@@ -560,29 +560,85 @@ __global__ void __launch_bounds__(AB_WAVES* WAVE)
     st.flush_stamped(moves, &mcounters[2], &mcounters[3], nmax, sh, stamp, gen);
 }
 
-__global__ void k_afterburner_big(DGraph g, const vid_t* cand, const int32_t* counters, const part_t* part,
-                                  const part_t* dest, const int32_t* pregain, int32_t* lock, vid_t* moves,
-                                  int32_t* mcounters, vid_t nmax, int32_t* stamp, int32_t gen) {
+// A wave per candidate of degree > BIG_DEG, AB_UNROLL edges per lane in
+// flight. The neighbours' destinations are gathered first: a neighbour that is
+// no candidate (NO_MOVE) contributes nothing, so its pre-gain and part are not
+// read. Candidates of degree > long_deg are queued in LDS and taken by the
+// whole workgroup afterwards.
+constexpr int AB_UNROLL = 4;
+constexpr int AB_QUEUE = 1024;
+__global__ void __launch_bounds__(AB_WAVES* WAVE)
+    k_afterburner_big(DGraph g, const vid_t* cand, const int32_t* counters, const part_t* part, const part_t* dest,
+                      const int32_t* pregain, int32_t* lock, vid_t* moves, int32_t* mcounters, vid_t nmax,
+                      int32_t* stamp, int32_t gen, int32_t long_deg) {
+    __shared__ vid_t queue[AB_QUEUE];
+    __shared__ int32_t nqueue;
+    __shared__ int64_t red[AB_WAVES];
     const int lane = threadIdx.x & (WAVE - 1);
-    const int64_t wstride = ((int64_t)gridDim.x * blockDim.x) / WAVE;
-    const int64_t x0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / WAVE;
-    const vid_t c0 = x0 < nmax ? cand[nmax - 1 - x0] : 0;  // loaded together with the count
+    const int wv = threadIdx.x / WAVE;
     const int32_t nb = counters[1];
-    for (int64_t x = x0; x < nb; x += wstride) {
-        const vid_t i = x == x0 ? c0 : cand[nmax - 1 - x];
-        part_t p = part[i], best = dest[i];
-        int32_t ig = pregain[i];
+    if (nb == 0) return;
+    if (threadIdx.x == 0) nqueue = 0;
+    __syncthreads();
+    auto burn = [&](vid_t i, eoff_t rs, eoff_t re, int sub, int stride) -> int64_t {
+        const part_t p = part[i], best = dest[i];
+        const int32_t ig = pregain[i];
         int64_t change = 0;
-        eoff_t rs = g.rowptr[i], re = g.rowptr[i + 1];
-        for (eoff_t j = rs + lane; j < re; j += WAVE)
-            change += afterburn_edge(g.col[j], i, ig, g.ew[j], p, best, part, dest, pregain);
-        change = wave_reduce_sum(change);
-        if (lane == 0 && (int64_t)ig + change >= 0) {
-            lock[i] = 1;
-            stamp[i] = gen;
-            if (re - rs > BIG_DEG) moves[nmax - 1 - atomicAdd(&mcounters[3], 1)] = i;
-            else moves[atomicAdd(&mcounters[2], 1)] = i;
+        for (eoff_t b0 = rs; b0 < re; b0 += (eoff_t)AB_UNROLL * stride) {
+            vid_t v[AB_UNROLL];
+            part_t vd[AB_UNROLL];
+#pragma unroll
+            for (int q = 0; q < AB_UNROLL; q++) {
+                const eoff_t j = b0 + (eoff_t)q * stride + sub;
+                v[q] = j < re ? g.col[j] : -1;
+            }
+#pragma unroll
+            for (int q = 0; q < AB_UNROLL; q++) vd[q] = v[q] >= 0 ? dest[v[q]] : NO_MOVE;
+#pragma unroll
+            for (int q = 0; q < AB_UNROLL; q++) {
+                if (vd[q] == NO_MOVE) continue;
+                const int32_t vg = pregain[v[q]];
+                const part_t vq = part[v[q]];
+                const int32_t w = g.ew[b0 + (eoff_t)q * stride + sub];
+                if (vg > ig || (vg == ig && v[q] < i)) {  // afterburn_edge
+                    if (vd[q] == p) change -= w;
+                    else if (vd[q] == best) change += w;
+                    if (vq == p) change += w;
+                    else if (vq == best) change -= w;
+                }
+            }
         }
+        return change;
+    };
+    auto keep = [&](vid_t i, int64_t change) {  // one thread
+        if ((int64_t)pregain[i] + change < 0) return;
+        lock[i] = 1;
+        stamp[i] = gen;
+        moves[nmax - 1 - atomicAdd(&mcounters[3], 1)] = i;
+    };
+    // consecutive candidates go to different workgroups
+    for (int64_t x = (int64_t)wv * gridDim.x + blockIdx.x; x < nb; x += (int64_t)gridDim.x * AB_WAVES) {
+        const vid_t i = cand[nmax - 1 - x];
+        const eoff_t rs = g.rowptr[i], re = g.rowptr[i + 1];
+        if (re - rs > long_deg) {
+            int32_t slot = 0;
+            if (lane == 0) slot = atomicAdd(&nqueue, 1);
+            slot = __shfl(slot, 0, WAVE);
+            if (slot < AB_QUEUE) {
+                if (lane == 0) queue[slot] = i;
+                continue;
+            }
+        }
+        const int64_t change = wave_reduce_sum(burn(i, rs, re, lane, WAVE));
+        if (lane == 0) keep(i, change);
+    }
+    __syncthreads();
+    const int32_t nq = min(nqueue, AB_QUEUE);
+    for (int32_t q = 0; q < nq; q++) {
+        const vid_t i = queue[q];
+        const int64_t change = block_reduce_sum<int64_t, AB_WAVES * WAVE>(
+            burn(i, g.rowptr[i], g.rowptr[i + 1], threadIdx.x, AB_WAVES * WAVE), red);
+        if (threadIdx.x == 0) keep(i, change);
     }
 }
 
@@ -594,7 +650,9 @@ __global__ void k_afterburner_big(DGraph g, const vid_t* cand, const int32_t* co
 // pushing keeps a part whose connectivity falls to 0 in a table of k slots
 // (jet_refiner.hpp:806-810) and the rebalancers read such entries, so the
 // choice follows the reference exactly.
-__device__ inline bool update_by_rebuild(const int32_t* mc, vid_t n) { return mc[2] + mc[3] > n / 10; }
+// Every hub row is scanned for moved neighbours (k_pull_hubs) when more than
+// n / PULL_ALL_DIV vertices move, else only those the first pass flags.
+constexpr int32_t PULL_ALL_DIV = 512;
 
 // The cut change and the largest part (jet_refiner.hpp:937-948). For a moved
 // vertex v the reference adds conn(v, new part) - conn(v, old part) from its
@@ -744,45 +802,49 @@ struct MoveRec {
 
 // One move in either pass, or one slice of it: the edges rs + sub, rs + sub +
 // stride, ... before re.
+// One edge of a move, its neighbour v no hub: the cut change and the old
+// part's subtraction (first pass) or the new part's addition (second).
 template <bool ADD>
-__device__ inline void update_move(const DGraph& g, vid_t i, part_t pold, part_t pnew, eoff_t rs, eoff_t re, int sub,
-                                   int stride,
-                                   bool rebuild, const part_t* part, const part_t* dest, const eoff_t* conn_off,
-                                   int2* conn, int32_t* conn_size, part_t* dest_cache, int32_t k, int32_t* err,
-                                   int32_t* mark, const uint8_t* hub, uint8_t* hub_dirty, const int32_t* stamp,
+__device__ inline void update_edge(vid_t v, int32_t w, part_t pold, part_t pnew, bool rebuild, const part_t* part,
+                                   const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size,
+                                   part_t* dest_cache, int32_t k, int32_t* err, int32_t* mark, const int32_t* stamp,
                                    int32_t gen, int64_t& cc) {
+    if (!ADD) {
+        // loaded together: the neighbour's parts and table
+        const part_t pv = part[v], dv = dest[v];
+        const bool sv = stamp[v] == gen;
+        const eoff_t co = rebuild ? 0 : conn_off[v];
+        const int32_t cs = rebuild ? 0 : ld_rx(&conn_size[v]);
+        const part_t nv = sv ? dv : pv;
+        cc += (int64_t)w *
+              ((pv == pnew ? 1 : 0) - (pv == pold ? 1 : 0) + (nv == pnew ? 1 : 0) - (nv == pold ? 1 : 0));
+        if (rebuild) mark[v] = 1;
+        else conn_sub(conn + co, cs, pold, w, k, err);
+    } else {
+        const eoff_t co = conn_off[v], ce = conn_off[v + 1];
+        dest_cache[v] = NULL_PART;
+        conn_add(conn + co, &conn_size[v], (int32_t)(ce - co), pnew, w, err);
+    }
+}
+
+// A neighbour of degree > BIG_DEG (hub[v]; hub null: the level has none) is
+// left to k_pull_hubs, which takes its table update and its share of the cut
+// change; unless every hub row is scanned there (pull_all), it is flagged.
+template <bool ADD>
+__device__ inline void update_move(const DGraph& g, part_t pold, part_t pnew, eoff_t rs, eoff_t re, int sub,
+                                   int stride, bool rebuild, bool pull_all, const part_t* part, const part_t* dest,
+                                   const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
+                                   int32_t k, int32_t* err, int32_t* mark, const uint8_t* hub, uint8_t* hub_dirty,
+                                   const int32_t* stamp, int32_t gen, int64_t& cc) {
     for (eoff_t j = rs + sub; j < re; j += stride) {
         const vid_t v = g.col[j];
         const int32_t w = g.ew[j];
-        if (!ADD) {
-            // loaded together: the neighbour's parts and table
-            const part_t pv = part[v], dv = dest[v];
-            const bool sv = stamp[v] == gen;
-            if (rebuild) {
-                const part_t nv = sv ? dv : pv;
-                cc += (int64_t)w *
-                      ((pv == pnew ? 1 : 0) - (pv == pold ? 1 : 0) + (nv == pnew ? 1 : 0) - (nv == pold ? 1 : 0));
-                mark[v] = 1;
-                continue;
-            }
-            const uint8_t hv = hub[v];
-            const eoff_t co = conn_off[v];
-            const int32_t cs = ld_rx(&conn_size[v]);
-            const part_t nv = sv ? dv : pv;
-            cc += (int64_t)w *
-                  ((pv == pnew ? 1 : 0) - (pv == pold ? 1 : 0) + (nv == pnew ? 1 : 0) - (nv == pold ? 1 : 0));
-            if (hv) {  // updated by k_update_hubs
-                hub_dirty[v] = 1;
-                continue;
-            }
-            conn_sub(conn + co, cs, pold, w, k, err);
-        } else {
-            const uint8_t hv = hub[v];
-            const eoff_t co = conn_off[v], ce = conn_off[v + 1];
-            if (hv) continue;  // updated by k_update_hubs
-            dest_cache[v] = NULL_PART;
-            conn_add(conn + co, &conn_size[v], (int32_t)(ce - co), pnew, w, err);
+        if (hub && hub[v]) {
+            if (!ADD && !pull_all) hub_dirty[v] = 1;
+            continue;
         }
+        update_edge<ADD>(v, w, pold, pnew, rebuild, part, dest, conn_off, conn, conn_size, dest_cache, k, err, mark,
+                         stamp, gen, cc);
     }
 }
 
@@ -809,7 +871,7 @@ __global__ void __launch_bounds__(256)
                    const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
                    int32_t k, int32_t* err, int32_t* mark, const uint8_t* hub, uint8_t* hub_dirty,
                    const int32_t* deferred, const int32_t* stamp, int32_t gen, unsigned long long* sizes,
-                   int64_t* partials, Publish pb, RebalPrep prep) {
+                   int64_t* partials, uint32_t* bits, Publish pb, RebalPrep prep) {
     __shared__ int64_t red[256 / WAVE];
     __shared__ int32_t ws[ADD ? 256 / WAVE + 1 : 1];
     __shared__ unsigned long long ls[ADD ? 1 : LDS_K];
@@ -844,7 +906,8 @@ __global__ void __launch_bounds__(256)
         // current step's readers have all run before the first pass)
         for (int64_t i = (blk * blockDim.x) + threadIdx.x; i < prep.nb; i += nblk * blockDim.x) prep.buckets[i] = 0;
     }
-    const bool rebuild = ns + nbig > g.n / 10;  // update_by_rebuild
+    const bool rebuild = ns + nbig > g.n / 10;  // jet_refiner.hpp:933
+    const bool pull_all = ns + nbig > g.n / PULL_ALL_DIV;
     if (!ADD && rebuild && blockIdx.x == 0 && threadIdx.x == 0) mc[6] = 1;  // the tables are to be rebuilt
     const bool lds = !ADD && k <= LDS_K;
     if (lds) {
@@ -855,16 +918,20 @@ __global__ void __launch_bounds__(256)
     for (int64_t x = x0; x < ns; x += gstride) {
         if (ADD) {
             const MoveRec r = x == x0 ? r0 : rec[x];
-            if (sub == 0) part[r.v] = r.pnew;
+            if (sub == 0) {
+                part[r.v] = r.pnew;
+                if (bits) bits[r.v >> 5] = 0;
+            }
             if (rebuild) continue;
-            update_move<true>(g, r.v, 0, r.pnew, r.rs, r.rs + r.deg, sub, G, false, part, dest, conn_off, conn,
-                                 conn_size, dest_cache, k, err, mark, hub, hub_dirty, stamp, gen, cc);
+            update_move<true>(g, 0, r.pnew, r.rs, r.rs + r.deg, sub, G, false, pull_all, part, dest, conn_off, conn,
+                              conn_size, dest_cache, k, err, mark, hub, hub_dirty, stamp, gen, cc);
         } else {
             const vid_t i = x == x0 ? i0 : moves[x];
             const part_t pold = part[i], pnew = dest[i];
             const eoff_t rs = g.rowptr[i], re = g.rowptr[i + 1];
             if (sub == 0) {
                 dest_cache[i] = NULL_PART;
+                if (bits) atomicOr(&bits[i >> 5], 1u << (i & 31));
                 rec[x] = MoveRec{rs, (int32_t)(re - rs), i, pnew, 0};
                 const unsigned long long w = (unsigned long long)g.vw[i];
                 if (lds) {
@@ -875,8 +942,8 @@ __global__ void __launch_bounds__(256)
                     atomicAdd(&sizes[pnew], w);
                 }
             }
-            update_move<false>(g, i, pold, pnew, rs, re, sub, G, rebuild, part, dest, conn_off, conn, conn_size,
-                                  dest_cache, k, err, mark, hub, hub_dirty, stamp, gen, cc);
+            update_move<false>(g, pold, pnew, rs, re, sub, G, rebuild, pull_all, part, dest, conn_off, conn,
+                               conn_size, dest_cache, k, err, mark, hub, hub_dirty, stamp, gen, cc);
         }
     }
     if (!ADD) {
@@ -891,106 +958,357 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// The same for the moves of degree > BIG_DEG (the back of the list), one wave
-// per move.
+// The same for the moves of degree > BIG_DEG (the back of the list): a wave
+// per move, UB_UNROLL edges per lane in flight; moves of degree > long_deg are
+// queued in LDS and taken by the whole workgroup afterwards, so that one long
+// row does not serialise a wave. (Every move spread over 16 waves, whatever
+// its degree, loaded most moves' records to find no edge left: 525 us a first
+// pass and 508 us a second one on R-MAT 22, bound by those loads.)
+constexpr int UB_BLOCK = 1024;
+constexpr int UB_UNROLL = 4;
+constexpr int UB_QUEUE = 1024;
 template <bool ADD>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(UB_BLOCK)
     k_update_big(DGraph g, const vid_t* moves, MoveRec* rec, const int32_t* mc, vid_t nmax, part_t* part,
                  const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
                  int32_t k, int32_t* err, int32_t* mark, const uint8_t* hub, uint8_t* hub_dirty,
                  const int32_t* deferred, const int32_t* stamp, int32_t gen, unsigned long long* sizes,
-                 int64_t* partials, int32_t slices) {
-    __shared__ int64_t red[256 / WAVE];
+                 int64_t* partials, uint32_t* bits, int32_t long_deg) {
+    __shared__ int64_t queue[UB_QUEUE];
+    __shared__ int32_t nqueue;
     const int lane = threadIdx.x & (WAVE - 1);
-    // units: (move x, slice q) for q < slices; slice q of a move takes its
-    // edges q * WAVE + lane, stride slices * WAVE, so a hub's edges are
-    // spread over `slices` waves; slice 0 does the move's bookkeeping
-    const int64_t wstride = ((int64_t)gridDim.x * blockDim.x) / WAVE;
-    const int64_t u0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / WAVE;
-    const int64_t x0 = u0 / slices;
-    const bool have0 = x0 < nmax;
-    const vid_t i0 = !ADD && have0 ? moves[nmax - 1 - x0] : 0;
-    MoveRec r0{};
-    if (ADD && have0) r0 = rec[nmax - 1 - x0];
+    const int wv = threadIdx.x / WAVE;
+    constexpr int WAVES = UB_BLOCK / WAVE;
     const int32_t dfr = *deferred;
     const int32_t ns = mc[2], nb = mc[3];
-    if (dfr) return;
-    const bool rebuild = ns + nb > g.n / 10;  // update_by_rebuild
-    const int STRIDE = slices * WAVE;
+    if (dfr || nb == 0) return;
+    const bool rebuild = ns + nb > g.n / 10;  // jet_refiner.hpp:933
+    const bool pull_all = ns + nb > g.n / PULL_ALL_DIV;
+    if (threadIdx.x == 0) nqueue = 0;
+    __syncthreads();
     int64_t cc = 0;
-    for (int64_t u = u0; u < (int64_t)nb * slices; u += wstride) {
-        const int64_t x = u / slices;
-        const int q = (int)(u % slices);
+    auto edges = [&](vid_t v, part_t pold, part_t pnew, eoff_t rs, eoff_t re, int sub, int stride) {
+        // the hub flags of UB_UNROLL edges are loaded together; only the
+        // neighbours that are no hubs go on to the table updates
+        for (eoff_t b0 = rs; b0 < re; b0 += (eoff_t)UB_UNROLL * stride) {
+            vid_t u[UB_UNROLL];
+            uint8_t h[UB_UNROLL];
+#pragma unroll
+            for (int q = 0; q < UB_UNROLL; q++) {
+                const eoff_t j = b0 + (eoff_t)q * stride + sub;
+                u[q] = j < re ? g.col[j] : -1;
+            }
+#pragma unroll
+            for (int q = 0; q < UB_UNROLL; q++) h[q] = u[q] >= 0 && hub ? hub[u[q]] : 0;
+#pragma unroll
+            for (int q = 0; q < UB_UNROLL; q++) {
+                if (u[q] < 0) continue;
+                if (h[q]) {
+                    if (!ADD && !pull_all) hub_dirty[u[q]] = 1;
+                    continue;
+                }
+                update_edge<ADD>(u[q], g.ew[b0 + (eoff_t)q * stride + sub], pold, pnew, rebuild, part, dest, conn_off,
+                                 conn, conn_size, dest_cache, k, err, mark, stamp, gen, cc);
+            }
+        }
+    };
+    auto one = [&](int64_t x, bool longs) {
         const int64_t at = nmax - 1 - x;
+        const int sub = longs ? threadIdx.x : lane, stride = longs ? UB_BLOCK : WAVE;
         if (ADD) {
-            const MoveRec r = x == x0 ? r0 : rec[at];
-            if (q == 0 && lane == 0) part[r.v] = r.pnew;
-            if (rebuild) continue;
-            update_move<true>(g, r.v, 0, r.pnew, r.rs, r.rs + r.deg, q * WAVE + lane, STRIDE, false, part, dest,
-                              conn_off, conn, conn_size, dest_cache, k, err, mark, hub, hub_dirty, stamp, gen, cc);
+            const MoveRec r = rec[at];
+            if (!longs) {
+                if (lane == 0) {
+                    part[r.v] = r.pnew;
+                    if (bits) bits[r.v >> 5] = 0;
+                }
+                if (rebuild) return;
+                if (r.deg > long_deg) {
+                    int32_t slot = 0;
+                    if (lane == 0) slot = atomicAdd(&nqueue, 1);
+                    slot = __shfl(slot, 0, WAVE);
+                    if (slot < UB_QUEUE) {
+                        if (lane == 0) queue[slot] = x;
+                        return;
+                    }
+                }
+            }
+            edges(r.v, 0, r.pnew, r.rs, r.rs + r.deg, sub, stride);
         } else {
-            const vid_t i = x == x0 ? i0 : moves[at];
+            const vid_t i = moves[at];
             const part_t pold = part[i], pnew = dest[i];
             const eoff_t rs = g.rowptr[i], re = g.rowptr[i + 1];
-            if (q == 0 && lane == 0) {
-                dest_cache[i] = NULL_PART;
-                rec[at] = MoveRec{rs, (int32_t)(re - rs), i, pnew, 0};
-                const unsigned long long w = (unsigned long long)g.vw[i];
-                atomicAdd(&sizes[pold], (unsigned long long)(-(long long)w));
-                atomicAdd(&sizes[pnew], w);
+            if (!longs) {
+                if (lane == 0) {
+                    dest_cache[i] = NULL_PART;
+                    if (bits) atomicOr(&bits[i >> 5], 1u << (i & 31));
+                    rec[at] = MoveRec{rs, (int32_t)(re - rs), i, pnew, 0};
+                    const unsigned long long w = (unsigned long long)g.vw[i];
+                    atomicAdd(&sizes[pold], (unsigned long long)(-(long long)w));
+                    atomicAdd(&sizes[pnew], w);
+                }
+                if (re - rs > long_deg) {
+                    int32_t slot = 0;
+                    if (lane == 0) slot = atomicAdd(&nqueue, 1);
+                    slot = __shfl(slot, 0, WAVE);
+                    if (slot < UB_QUEUE) {
+                        if (lane == 0) queue[slot] = x;
+                        return;
+                    }
+                }
             }
-            update_move<false>(g, i, pold, pnew, rs, re, q * WAVE + lane, STRIDE, rebuild, part, dest, conn_off,
-                               conn, conn_size, dest_cache, k, err, mark, hub, hub_dirty, stamp, gen, cc);
+            edges(i, pold, pnew, rs, re, sub, stride);
         }
+    };
+    // consecutive moves go to different workgroups, and with them the long ones
+    for (int64_t x = (int64_t)wv * gridDim.x + blockIdx.x; x < nb; x += (int64_t)gridDim.x * WAVES) one(x, false);
+    __syncthreads();
+    const int32_t nq = min(nqueue, UB_QUEUE);
+    for (int32_t q = 0; q < nq; q++) one(queue[q], true);
+    if (!ADD) {
+        cc = wave_reduce_sum(cc);
+        if (lane == 0 && cc)
+            atomicAdd((unsigned long long*)&partials[(int64_t)(blockIdx.x % PUB_GROUPS) * PUB_STRIDE],
+                      (unsigned long long)cc);
     }
-    if (!ADD) add_cut_part2(partials, cc, red);
 }
 
-// update_small for rows of degree > BIG_DEG ("hubs": the workgroup-built tier
-// and the pull_mid rows), one workgroup per row with a moved neighbour: the
-// row's moved neighbours are found by a scan of its adjacency and their
-// weights summed per part in LDS, then each part's total is applied to the
-// table once, with the subtraction phase before the
-// addition phase as for the other rows. The resulting table equals the one
-// per-edge pushes leave: a part is reclaimed when its connectivity reaches 0
-// in a table of fewer than k slots (jet_refiner.hpp:806-810), new parts take
-// free or reclaimed slots and then overflow slots (:828-884). Pushing instead
-// would land every moved neighbour's atomics on the same few hub slots.
-template <bool ADD, int BLOCK>
-__global__ void __launch_bounds__(BLOCK)
-    k_update_hubs(DGraph g, const vid_t* list, int32_t nlist, const int32_t* mc, const int32_t* stamp, int32_t gen,
-                  uint8_t* hub_dirty, const part_t* part, const part_t* dest, const eoff_t* conn_off, int2* conn,
-                  int32_t* conn_size, part_t* dest_cache, int32_t k, int32_t* err, const int32_t* deferred) {
-    if (*deferred || update_by_rebuild(mc, g.n)) return;
-    extern __shared__ int32_t delta[];  // k
-    for (int32_t r = blockIdx.x; r < nlist; r += gridDim.x) {
-        const vid_t u = list[r];
-        if (!hub_dirty[u]) continue;
-        for (int32_t p = threadIdx.x; p < k; p += BLOCK) delta[p] = 0;
-        __syncthreads();
-        for (eoff_t j = g.rowptr[u] + threadIdx.x; j < g.rowptr[u + 1]; j += BLOCK) {
-            vid_t v = g.col[j];
-            // between the passes part[v] is still the old part; the new one is dest[v]
-            if (stamp[v] == gen) atomicAdd(&delta[ADD ? dest[v] : part[v]], g.ew[j]);
+// The step's effect on the rows of degree > BIG_DEG ("hubs": the
+// workgroup-built tier and the pull_mid rows), one kernel between the two
+// passes: a wave per row (a workgroup per row of the workgroup-built tier)
+// scans the row for neighbours that move and adds their share of the cut
+// change (the same term the first pass adds for its neighbours, seen from the
+// other end of the edge). The row's table is held dense in LDS, connectivity
+// by part, so a moved neighbour costs two LDS adds; when the scan has found
+// one, the table is written back in increasing part id. It has the content
+// and the size that per-edge pushes, subtractions before additions, leave:
+// in a table of fewer than k slots a part whose connectivity reaches 0 is
+// dropped (jet_refiner.hpp:806-810) and new parts take the free slots before
+// the table grows (:828-884); a table of k slots keeps its zero entries.
+// Nothing looks a hub row's part up by its slot: select kernels read all
+// slots, and only this kernel and the builds write them. When the step
+// rebuilds the tables (update_large), the rows with a moved neighbour are
+// marked instead.
+//
+// Bound: the scan streams 4 bytes per edge; which neighbours move is a bit
+// per vertex, set by the first pass and cleared by the second, which every
+// workgroup holds in LDS (EXACT), so an edge costs an LDS read instead of a
+// gather of the generation stamp from L2. On levels of more vertices than
+// PH_BITS_MAX bytes hold, an LDS bit stands for 2^shift consecutive vertices
+// and only the neighbours whose bit is set look their own bit up in memory
+// (n / 8 bytes, resident in L2). Two workgroups fit a CU. Probing and
+// updating the hashed table per moved neighbour instead (staged in LDS too)
+// was bound by its instructions, a few lanes of a wave active in each.
+// R-MAT 22 (k = 256), averages per step: two scans per step with global
+// tables 1.36 ms in four launches, one scan probing hashed LDS tables 2.4 ms,
+// this kernel 0.32 ms on the levels of up to 438,484 vertices and 0.67 ms
+// above (0.90 ms with the stamps gathered there).
+// Steps that move few vertices scan only the rows that the first pass
+// flagged; from n / PULL_ALL_DIV moves on, about a third of the rows of
+// average degree 190 have a moved neighbour and flagging costs a store per
+// edge, so every hub row is scanned.
+constexpr int PH_WAVES_MAX = 16;
+constexpr int PH_UNROLL = 4;
+constexpr size_t PH_BITS_MAX = 56 * 1024;
+constexpr size_t PH_LDS_MAX = 96 * 1024;  // tables (at most 34 KB) and bits
+
+// LDS words of one dense table: k connectivities, then a bit per part (the
+// part has a slot).
+__host__ __device__ inline int32_t ph_table_words(int32_t k) { return k + (k + 31) / 32; }
+
+// Loads the row's table (cap slots at conn) into the dense table, which is
+// all zero; lanes start, start + stride, ...
+__device__ inline void ph_load(const int2* conn, int32_t cap, int32_t k, int32_t* val, int start, int stride) {
+    uint32_t* has = reinterpret_cast<uint32_t*>(val + k);
+    for (int32_t q = start; q < cap; q += stride) {
+        const int2 e = conn[q];
+        if (e.x < 0) continue;
+        val[e.x] = e.y;
+        atomicOr(&has[e.x >> 5], 1u << (e.x & 31));
+    }
+}
+
+// Writes the dense table back as the row's table of vsz slots (a wave), and
+// zeroes it; returns the new size.
+__device__ inline int32_t ph_store(int2* conn, int32_t cap, int32_t vsz, int32_t k, int32_t* val, int lane,
+                                   int32_t* err) {
+    uint32_t* has = reinterpret_cast<uint32_t*>(val + k);
+    int32_t used = 0;
+    for (int32_t p0 = 0; p0 < k; p0 += WAVE) {
+        const int32_t p = p0 + lane;
+        const int32_t y = p < k ? val[p] : 0;
+        const bool keep = p < k && (y != 0 || (vsz == k && ((has[p >> 5] >> (p & 31)) & 1u)));
+        if (y < 0) atomicOr(err, 1);
+        const uint64_t mk = __ballot(keep);
+        const int32_t at = used + (int32_t)__popcll(mk & ((1ull << lane) - 1ull));
+        if (keep) {
+            if (at < cap) conn[at] = make_int2(p, y);
+            else atomicOr(err, 2);
         }
+        if (p < k) val[p] = 0;
+        used += (int32_t)__popcll(mk);
+    }
+    wave_sync();  // the presence bits are read before they are cleared
+    for (int32_t q = lane; q < (k + 31) / 32; q += WAVE) has[q] = 0;
+    for (int32_t q = used + lane; q < vsz; q += WAVE) conn[q] = make_int2(NULL_PART, 0);
+    return used > vsz ? min(used, cap) : vsz;
+}
+
+template <bool EXACT>
+__global__ void __launch_bounds__(PH_WAVES_MAX* WAVE)
+    k_pull_hubs(DGraph g, const vid_t* big, int32_t nbig, const vid_t* mid, int32_t nmid, const int32_t* mc,
+                const uint32_t* bits, int32_t shift, uint8_t* hub_dirty, const part_t* part,
+                const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
+                int32_t k, int32_t* err, int32_t* mark, const int32_t* deferred, int64_t* partials) {
+    extern __shared__ int32_t ph_lds[];  // a dense table per wave, then the bits
+    if (*deferred) return;
+    const int32_t nm = mc[2] + mc[3];
+    if (nm == 0) return;
+    const bool rebuild = nm > g.n / 10;  // jet_refiner.hpp:933
+    const bool all = nm > g.n / PULL_ALL_DIV;
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int wv = threadIdx.x / WAVE;
+    const int nwv = blockDim.x / WAVE;
+    const int32_t tw = ph_table_words(k);
+    uint32_t* lbits = reinterpret_cast<uint32_t*>(ph_lds + (size_t)nwv * tw);
+    for (int32_t t = threadIdx.x; t < nwv * tw; t += blockDim.x) ph_lds[t] = 0;
+    const int32_t words = (g.n + 31) >> 5;
+    if (EXACT) {
+        for (int32_t t = threadIdx.x; t < words; t += blockDim.x) lbits[t] = bits[t];
+    } else {
+        for (int32_t t = threadIdx.x; t < (int32_t)(((int64_t)g.n + (32ll << shift) - 1) >> (5 + shift));
+             t += blockDim.x)
+            lbits[t] = 0;
         __syncthreads();
-        int2* tab = conn + conn_off[u];
-        const int32_t cap = (int32_t)(conn_off[u + 1] - conn_off[u]);
+        const uint32_t group = shift >= 5 ? ~0u : (1u << (1 << shift)) - 1u;
+        for (int32_t t = threadIdx.x; t < words; t += blockDim.x) {
+            const uint32_t x = bits[t];
+            if (x == 0) continue;
+            uint32_t y = 0;  // the word's groups with a bit set, from its group's place in the LDS word
+            const int32_t g0 = shift >= 5 ? t >> (shift - 5) : t << (5 - shift);
+            for (int32_t q = 0; q < (shift >= 5 ? 1 : 32 >> shift); q++)
+                if ((x >> (q << shift)) & group) y |= 1u << q;
+            atomicOr(&lbits[g0 >> 5], y << (g0 & 31));
+        }
+    }
+    __syncthreads();
+    auto moved = [&](vid_t v) -> bool {
+        if (EXACT) return ((lbits[v >> 5] >> (v & 31)) & 1u) != 0;
+        return ((lbits[v >> (5 + shift)] >> ((v >> shift) & 31)) & 1u) != 0 && ((bits[v >> 5] >> (v & 31)) & 1u) != 0;
+    };
+    int64_t cc = 0;
+    // the row's edges rs + sub + q * stride by this thread, PH_UNROLL at a
+    // time; first() runs before the first moved neighbour of a round (of any
+    // lane of the wave) is added to val. Returns whether one was found.
+    auto scan = [&](eoff_t rs, eoff_t re, int sub, int stride, part_t pu, part_t nu, int32_t* val, auto&& first) {
+        bool any = false;
+        for (eoff_t b0 = rs; b0 < re; b0 += (eoff_t)PH_UNROLL * stride) {
+            vid_t v[PH_UNROLL];
+#pragma unroll
+            for (int q = 0; q < PH_UNROLL; q++) {
+                const eoff_t j = b0 + (eoff_t)q * stride + sub;
+                v[q] = j < re ? g.col[j] : -1;
+            }
+            uint32_t hits = 0;
+#pragma unroll
+            for (int q = 0; q < PH_UNROLL; q++)
+                if (v[q] >= 0 && moved(v[q])) hits |= 1u << q;
+            if (__ballot(hits != 0) == 0) continue;
+            int32_t w[PH_UNROLL];
+            part_t po[PH_UNROLL], pn[PH_UNROLL];
+#pragma unroll
+            for (int q = 0; q < PH_UNROLL; q++) {
+                const bool h = (hits >> q) & 1u;
+                w[q] = h ? g.ew[b0 + (eoff_t)q * stride + sub] : 0;
+                po[q] = h ? part[v[q]] : 0;
+                pn[q] = h ? dest[v[q]] : 0;
+            }
+            if (!any) first();
+            any = true;
+#pragma unroll
+            for (int q = 0; q < PH_UNROLL; q++) {
+                if (!((hits >> q) & 1u)) continue;
+                cc += (int64_t)w[q] * ((pu == pn[q] ? 1 : 0) - (pu == po[q] ? 1 : 0) + (nu == pn[q] ? 1 : 0) -
+                                       (nu == po[q] ? 1 : 0));
+                if (!rebuild) {
+                    atomicAdd(&val[po[q]], -w[q]);
+                    atomicAdd(&val[pn[q]], w[q]);
+                }
+            }
+        }
+        return any;
+    };
+    // rows of the workgroup-built tier first: they are the longest
+    for (int32_t r = blockIdx.x; r < nbig; r += gridDim.x) {
+        const vid_t u = big[r];
+        if (!all && !hub_dirty[u]) continue;  // the same for every thread
+        const eoff_t rs = g.rowptr[u], re = g.rowptr[u + 1];
+        const eoff_t co = conn_off[u];
+        const int32_t cap = (int32_t)(conn_off[u + 1] - co);
         const int32_t vsz = conn_size[u];
-        for (int32_t p = threadIdx.x; p < k; p += BLOCK) {
-            const int32_t w = delta[p];
-            if (w == 0) continue;
-            if (ADD) conn_add(tab, &conn_size[u], cap, p, w, err);
-            else conn_sub(tab, vsz, p, w, k, err);
-        }
-        if (ADD && threadIdx.x == 0) {
-            dest_cache[u] = NULL_PART;
-            hub_dirty[u] = 0;
+        const part_t pu = part[u], nu = moved(u) ? dest[u] : pu;
+        int32_t* val = ph_lds;
+        if (!rebuild) ph_load(conn + co, cap, k, val, threadIdx.x, blockDim.x);
+        __syncthreads();
+        const int any = __syncthreads_or(scan(rs, re, threadIdx.x, blockDim.x, pu, nu, val, [] {}) ? 1 : 0);
+        if (wv == 0) {
+            // an unchanged row's table is written back as it was (the dense
+            // table has to be zero again)
+            int32_t sz = vsz;
+            if (!rebuild) sz = ph_store(conn + co, cap, vsz, k, val, lane, err);
+            if (lane == 0) {
+                if (any) {
+                    if (rebuild) {
+                        mark[u] = 1;
+                    } else {
+                        conn_size[u] = sz;
+                        dest_cache[u] = NULL_PART;
+                    }
+                }
+                if (!all) hub_dirty[u] = 0;
+            }
         }
         __syncthreads();
     }
+    int32_t* val = ph_lds + (size_t)wv * tw;
+    for (int32_t r = blockIdx.x * nwv + wv; r < nmid; r += (int32_t)gridDim.x * nwv) {
+        const vid_t u = mid[r];
+        if (!all && !hub_dirty[u]) continue;
+        const eoff_t rs = g.rowptr[u], re = g.rowptr[u + 1];
+        const eoff_t co = conn_off[u];
+        const int32_t cap = (int32_t)(conn_off[u + 1] - co);
+        const int32_t vsz = conn_size[u];
+        const part_t pu = part[u], du = dest[u];
+        const part_t nu = moved(u) ? du : pu;
+        const bool any = scan(rs, re, lane, WAVE, pu, nu, val, [&] {
+            if (!rebuild) {
+                ph_load(conn + co, cap, k, val, lane, WAVE);
+                wave_sync();
+            }
+        });
+        int32_t sz = vsz;
+        if (any && !rebuild) {
+            wave_sync();
+            sz = ph_store(conn + co, cap, vsz, k, val, lane, err);
+        }
+        if (lane == 0) {
+            if (any) {
+                if (rebuild) {
+                    mark[u] = 1;
+                } else {
+                    conn_size[u] = sz;
+                    dest_cache[u] = NULL_PART;
+                }
+            }
+            if (!all) hub_dirty[u] = 0;
+        }
+        wave_sync();  // the dense table is zero before the next row
+    }
+    cc = wave_reduce_sum(cc);
+    if (lane == 0 && cc)
+        atomicAdd((unsigned long long*)&partials[(int64_t)(blockIdx.x % PUB_GROUPS) * PUB_STRIDE],
+                  (unsigned long long)cc);
 }
-
 
 // ---------------------------------------------------------------- rebalancing
 // Rebalancer minibuckets (jet_refiner.hpp:359-412, :449-481, :632-643).
@@ -1914,6 +2232,11 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     fill_i32(rd_mark_, 0, N, s);
     JET_HIP(hipMemsetAsync(hub_dirty_, 0, (size_t)N, s));
     fill_i32(stamp_, -1, N, s);
+    moved_bits_ = a.alloc<uint32_t>((N + 31) / 32);
+    fill_i32(reinterpret_cast<int32_t*>(moved_bits_), 0, (N + 31) / 32, s);
+    for (const void* f : {reinterpret_cast<const void*>(&k_pull_hubs<true>),
+                          reinterpret_cast<const void*>(&k_pull_hubs<false>)})
+        JET_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PH_LDS_MAX));
     fill_i32(counters_, 0, 32, s);
     fill_i64(acc_, 0, 8, s);
     wg_state_ = a.alloc<WgState>(1);
@@ -2026,8 +2349,9 @@ void Refiner::jet_lp(const Level& L, const part_t* part, double fr) {
     }
 #undef JET_AB
     if (has_big_)
-        family_launch(PF_AFTERBURNER, k_afterburner_big, dim3(grid_for((int64_t)g.n * WAVE, 256, 2048)), dim3(256), 0,
-                      s_, g, cand_, c, part, dest_, pregain_, lock_, moves_, c, nmax_, stamp_, gen_);
+        family_launch(PF_AFTERBURNER, k_afterburner_big, dim3(grid_for((int64_t)g.n * WAVE, AB_WAVES * WAVE, 512)),
+                      dim3(AB_WAVES * WAVE), 0, s_, g, cand_, c, part, dest_, pregain_, lock_, moves_, c, nmax_, stamp_,
+                      gen_, (int32_t)(tuning().upd_big_slices * 2 * WAVE));
     JET_LAUNCH_CHECK();
 }
 
@@ -2252,7 +2576,17 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
     }
     const RebalPrep no_prep{};
     prep_ready_ = false;
-    int nbb = grid_for((int64_t)g.n * WAVE, 256, 512);
+    int nbb = grid_for((int64_t)g.n * WAVE, UB_BLOCK, 512);
+    // k_pull_hubs: a dense table of k parts per wave (about 32 KB of them) and
+    // the moved bits, 2^ph_shift vertices each
+    const bool hubs = ntier_big_ > 0 || npull_mid_ > 0;
+    const int ph_waves = std::max(1, std::min<int>(PH_WAVES_MAX, 8192 / k));
+    const size_t ph_tables = sizeof(int32_t) * (size_t)ph_table_words(k) * ph_waves;
+    int32_t ph_shift = 0;
+    auto bits_bytes = [&] { return 4 * (size_t)(((int64_t)g.n + (32ll << ph_shift) - 1) >> (5 + ph_shift)); };
+    while (bits_bytes() > PH_BITS_MAX) ph_shift++;
+    uint32_t* bits = hubs ? moved_bits_ : nullptr;
+    const uint8_t* hub = hubs ? hub_ : nullptr;
     for (int add = 0; add < 2; add++) {
         if (unsigned long long* pc = prof_counters(PF_UPDATE)) {
             // counting runs only: move degrees, once per pass (nothing when
@@ -2262,10 +2596,10 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
 #define JET_UPD(GG)                                                                                                   \
     if (add) family_launch(PF_UPDATE, k_update_small<true, GG>, dim3(nbs + 1), dim3(256), 0, s_, g, moves_, mrec_, c, \
                            nmax_, part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k, misc_ + 1, swap_bit_,    \
-                           hub_, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, pb, prep);                           \
+                           hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, pb, prep);                      \
     else family_launch(PF_UPDATE, k_update_small<false, GG>, dim3(nbs), dim3(256), 0, s_, g, moves_, mrec_, c, nmax_, \
-                       part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k, misc_ + 1, swap_bit_, hub_,         \
-                       hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, pb, no_prep);
+                       part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k, misc_ + 1, swap_bit_, hub,          \
+                       hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, pb, no_prep);
         switch (G) {
             case 4: JET_UPD(4) break;
             case 8: JET_UPD(8) break;
@@ -2275,25 +2609,18 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
         }
 #undef JET_UPD
         if (has_big_) {
-            const int32_t slices = (int32_t)tuning().upd_big_slices;
-            family_launch(PF_UPDATE, add ? k_update_big<true> : k_update_big<false>, dim3(nbb), dim3(256), 0, s_, g,
+            const int32_t long_deg = (int32_t)(tuning().upd_big_slices * 2 * WAVE);
+            family_launch(PF_UPDATE, add ? k_update_big<true> : k_update_big<false>, dim3(nbb), dim3(UB_BLOCK), 0, s_, g,
                           moves_, mrec_, c, nmax_, part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k,
-                          misc_ + 1, swap_bit_, hub_, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, slices);
+                          misc_ + 1, swap_bit_, hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, long_deg);
         }
-        // pulled rows: big-tier rows by a 256-thread workgroup, rows of
-        // degree (BIG_DEG, HEAVY_DEG_REFINE] by a single-wave workgroup
-        const uint32_t lds = (uint32_t)(sizeof(int32_t) * (size_t)k);
-        if (ntier_big_ > 0) {
-            const int hb = std::min(ntier_big_, 2048);
-            family_launch(PF_UPDATE, add ? k_update_hubs<true, 256> : k_update_hubs<false, 256>, dim3(hb), dim3(256),
-                          lds, s_, g, tier_big_, ntier_big_, c, stamp_, gen_, hub_dirty_, part, dest_, conn_off_,
-                          conn_, conn_size_, dest_cache_, k, misc_ + 1, misc_ + 2);
-        }
-        if (npull_mid_ > 0) {
-            const int hb = std::min(npull_mid_, 8192);
-            family_launch(PF_UPDATE, add ? k_update_hubs<true, WAVE> : k_update_hubs<false, WAVE>, dim3(hb),
-                          dim3(WAVE), lds, s_, g, pull_mid_, npull_mid_, c, stamp_, gen_, hub_dirty_, part, dest_,
-                          conn_off_, conn_, conn_size_, dest_cache_, k, misc_ + 1, misc_ + 2);
+        if (!add && hubs) {
+            const int want = std::max(ntier_big_, (int)ceil_div(npull_mid_, ph_waves));
+            const int pb = std::max(1, std::min(want, 512));
+            family_launch(PF_UPDATE, ph_shift == 0 ? k_pull_hubs<true> : k_pull_hubs<false>, dim3(pb),
+                          dim3(ph_waves * WAVE), (uint32_t)(ph_tables + bits_bytes()), s_, g, tier_big_, ntier_big_,
+                          pull_mid_, npull_mid_, c, moved_bits_, ph_shift, hub_dirty_, part, dest_, conn_off_, conn_,
+                          conn_size_, dest_cache_, k, misc_ + 1, swap_bit_, misc_ + 2, pub_);
         }
         JET_LAUNCH_CHECK();
     }
