@@ -94,6 +94,13 @@ void prof_bytes(int fam, double host_bytes) {
 
 int prof_timed_family() { return P().timed; }
 
+bool prof_active() {
+    const Prof& p = P();
+    bool on = p.timed >= 0;
+    for (int f = 0; f < PF_FAMILIES; f++) on = on || p.counting[f];
+    return on;
+}
+
 bool prof_enable(const std::string& spec) {
     Prof& p = P();
     std::string name = spec;

@@ -57,6 +57,8 @@ bool prof_enable(const std::string& name);
 bool prof_read(int fam, int64_t& units, double& ms, double& bytes);
 // The family enabled for timing, or -1.
 int prof_timed_family();
+// Whether any family is timed or counted.
+bool prof_active();
 
 // A launch of a kernel of family `fam` on stream s: with its own start and
 // end events when the family is timed, counted when it is counted.

@@ -6,6 +6,7 @@
 #include "arena.h"
 #include "contract.h"
 #include "jet_types.h"
+#include "refine_team.h"
 #include "refine_wg.h"
 
 namespace jet {
@@ -75,7 +76,11 @@ class Refiner {
     const int64_t* best_sizes_dev() const { return best_sizes_; }
 
   private:
-    // jet_refine on one level by the one-workgroup kernel (small levels)
+    // jet_refine on one level by a team of workgroups of one XCD (small
+    // levels); false when no team could start (nothing was changed)
+    bool refine_team(const Level& L, part_t* best_part, const std::vector<double>& temps, LevelRecord& rec);
+    // jet_refine on one level by the graph-tagged one-workgroup kernel (the
+    // batched and served layer's collector)
     LevelRecord refine_wg(const Level& L, part_t* best_part, const std::vector<double>& temps);
     void init_conn(const Level& L, const part_t* part, const int32_t* mark);
     void build_tiers(const Level& L);
@@ -182,6 +187,14 @@ class Refiner {
     WgState* wg_state_ = nullptr;  // the one-workgroup kernel's controller state
     vid_t* wg_list_ = nullptr;     // its ranked-member list (n)
     int32_t* wg_runb_ = nullptr;   // its per-bucket running weights (WG_MAX_NBK)
+    // the team kernel's tables (rows at their adjacency's offset), control
+    // words and scratch
+    int2* team_conn_ = nullptr;
+    TeamCtl* team_ctl_ = nullptr;
+    int32_t* team_buckets_ = nullptr;
+    uint64_t* team_rkey_ = nullptr;
+    int32_t* team_rweight_ = nullptr;
+    bool team_irregular_ = false;  // a level was too irregular for a team (so are the finer ones)
     int64_t* res_host_ = nullptr;  // thread mailbox: (cut change, largest part) of the last iteration
     int64_t* res_dev_ = nullptr;
     // refine_data mirror on the host

@@ -2242,6 +2242,11 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     wg_state_ = a.alloc<WgState>(1);
     wg_list_ = a.alloc<vid_t>(N);
     wg_runb_ = a.alloc<int32_t>(WG_MAX_NBK + 1);
+    team_conn_ = a.alloc<int2>(TEAM_MAX_M);
+    team_ctl_ = a.alloc<TeamCtl>(1);
+    team_buckets_ = a.alloc<int32_t>(TEAM_MAX_NBK + 1);
+    team_rkey_ = a.alloc<uint64_t>(std::min<int64_t>(N, TEAM_MAX_N));
+    team_rweight_ = a.alloc<int32_t>(std::min<int64_t>(N, TEAM_MAX_N));
     pub_ = a.alloc<int64_t>((int64_t)PUB_GROUPS * PUB_STRIDE);
     fill_i64(pub_, 0, (int64_t)PUB_GROUPS * PUB_STRIDE, s);
     szc_ = a.alloc<int64_t>((int64_t)SIZE_COPIES_MAX * p.k);
@@ -2664,8 +2669,7 @@ LevelRecord Refiner::refine(const Level& L, part_t* best_part) {
     best_due_ = false;
     DGraph g = L.view();
     const int32_t k = p_.k;
-    fill2_i32(misc_, 0, 8, counters_, 0, 16, s_);
-    par_ = 0;
+    int64_t first_max = 0;
     if (!init_) {
         cut_ = total_cut2(g, best_part, a_, s_);
         part_sizes(g, best_part, k, best_sizes_, s_);
@@ -2673,25 +2677,17 @@ LevelRecord Refiner::refine(const Level& L, part_t* best_part) {
         JET_HIP(hipMemcpyAsync(hs.data(), best_sizes_, sizeof(int64_t) * k, hipMemcpyDeviceToHost, s_));
         JET_HIP(hipStreamSynchronize(s_));
         total_size_ = 0;
-        for (int64_t v : hs) total_size_ += v;
+        for (int64_t v : hs) {
+            total_size_ += v;
+            first_max = std::max(first_max, v);
+        }
     }
     opt_ = (int32_t)(((int32_t)total_size_ + k - 1) / k);
     size_max_ = (int32_t)(opt_ * p_.imb);
     if (!init_) {
         init_ = true;
-        std::vector<int64_t> hs(k);
-        JET_HIP(hipMemcpyAsync(hs.data(), best_sizes_, sizeof(int64_t) * k, hipMemcpyDeviceToHost, s_));
-        JET_HIP(hipStreamSynchronize(s_));
-        int64_t mx = 0;
-        for (int64_t v : hs) mx = std::max(mx, v);
-        total_imb_ = mx > opt_ ? mx - opt_ : 0;
+        total_imb_ = first_max > opt_ ? first_max - opt_ : 0;
     }
-    int64_t curr_cut = cut_, curr_imb = total_imb_;
-    copy_i64(curr_sizes_, best_sizes_, k, s_);
-    const int64_t imb_max = (int64_t)size_max_ - opt_;
-    copy_i32(cur_part_, best_part, g.n, s_);
-    build_tiers(L);
-    init_conn(L, cur_part_, nullptr);
     std::vector<double> temps;
     if (p_.ultra) {
         for (double t = 0.85; t > 0; t -= 0.05) temps.push_back(t);
@@ -2700,13 +2696,32 @@ LevelRecord Refiner::refine(const Level& L, part_t* best_part) {
     } else {
         temps.push_back(0.75);
     }
-    {
-        const RebalanceShape wr = rebalance_shape(g.n, false);
-        if (!trace && wg_fits(g.n, k, wr.nbk, wg_threshold()) && (int)temps.size() <= WG_MAX_TEMPS) {
-            LevelRecord rec = refine_wg(L, best_part, temps);
+    const RebalanceShape wr = rebalance_shape(g.n, false);
+    const bool tagged = !trace && wg_collector() && wg_fits(g.n, k, wr.nbk, tuning().batch_wg_max_n) &&
+                        (int)temps.size() <= WG_MAX_TEMPS;
+    // the kernel families are measured, and iterations traced, on the
+    // multi-kernel path
+    const int64_t team_n = wg_collector() ? std::min<int64_t>(tuning().wg_max_n, TEAM_BATCH_N) : tuning().wg_max_n;
+    if (!tagged && !trace && !prof_active() && team_fits(g.n, g.m, k, wr.nbk, team_n) &&
+        (int)temps.size() <= WG_MAX_TEMPS && !(team_irregular_ && g.m > TEAM_REGULAR_M)) {
+        LevelRecord rec;
+        if (refine_team(L, best_part, temps, rec)) {
             rec.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
             return rec;
         }
+    }
+    fill2_i32(misc_, 0, 8, counters_, 0, 16, s_);
+    par_ = 0;
+    int64_t curr_cut = cut_, curr_imb = total_imb_;
+    copy_i64(curr_sizes_, best_sizes_, k, s_);
+    const int64_t imb_max = (int64_t)size_max_ - opt_;
+    copy_i32(cur_part_, best_part, g.n, s_);
+    build_tiers(L);
+    init_conn(L, cur_part_, nullptr);
+    if (tagged) {
+        LevelRecord rec = refine_wg(L, best_part, temps);
+        rec.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+        return rec;
     }
     LevelRecord rec;
     int balance_counter = 0;
@@ -2776,10 +2791,92 @@ LevelRecord Refiner::refine(const Level& L, part_t* best_part) {
     return rec;
 }
 
-// The level's iterations in the one-workgroup kernel (csrc/refine_wg.hip),
-// from the tables init_conn built. The kernel stops early only when a step
-// chose update_large: the marked rows are then rebuilt here, by the same
-// multi-workgroup build as flush_rebuild, and the kernel continues.
+// The whole level in one launch (csrc/refine_team.hip).
+bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<double>& temps, LevelRecord& rec) {
+    DGraph g = L.view();
+    const int32_t k = p_.k;
+    const RebalanceShape weak = rebalance_shape(g.n, false), strong = rebalance_shape(g.n, true);
+    TeamParams P{};
+    P.g = g;
+    P.k = k;
+    P.sections = weak.sections;
+    P.nbk = (int32_t)weak.nbk;
+    P.big_deg = (int32_t)tuning().wg_big_deg;
+    P.lanes = group_for_avg(g);
+    P.opt = opt_;
+    P.size_max = size_max_;
+    P.imb_max = (int64_t)size_max_ - opt_;
+    P.max_dest_weak = weak.max_dest;
+    P.max_dest_strong = strong.max_dest;
+    P.tol = p_.tol;
+    P.ntemps = (int32_t)temps.size();
+    for (size_t i = 0; i < temps.size(); i++) P.temps[i] = temps[i];
+    P.cut = cut_;
+    P.imb = total_imb_;
+    P.part = cur_part_;
+    P.best_part = best_part;
+    P.conn = team_conn_;
+    P.conn_size = conn_size_;
+    P.dest_cache = dest_cache_;
+    P.lock = lock_;
+    P.gain_p = gain_p_;
+    P.pregain = pregain_;
+    P.dest = dest_;
+    P.bid = bid_;
+    P.stamp = stamp_;
+    P.gen0 = gen_;
+    P.mark = swap_bit_;
+    P.score = score_;
+    P.rkey = team_rkey_;
+    P.rweight = team_rweight_;
+    P.redraw = redraw_;
+    P.buckets = team_buckets_;
+    P.sizes = curr_sizes_;
+    P.best_sizes = best_sizes_;
+    P.evict_adjust = evict_adjust_;
+    P.ctl = team_ctl_;
+    P.host_out = mailbox_->dev + 16;
+    volatile int64_t* out = mailbox_->host + 16;
+    P.seq = ++mailbox_->seq;
+    P.team = team_size(g.n, g.m);
+    TeamSlot slot(P.team);
+    P.xcd = slot.xcd();
+    launch_refine_team(P, s_);
+    for (uint64_t spins = 1; out[TEAM_OUT_WORDS] != P.seq; spins++) {
+        __builtin_ia32_pause();
+        if (spins >= (1u << 14) && spins % 64 == 0) sched_yield();
+        if (spins % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(s_);
+            if (e == hipSuccess) {
+                if (out[TEAM_OUT_WORDS] == P.seq) break;
+                return false;  // no workgroup ran on the wanted XCD
+            }
+            if (e != hipErrorNotReady) JET_HIP(e);
+        }
+    }
+    const int64_t status = out[5], err = out[6];
+    if (status == WG_IRREGULAR) team_irregular_ = true;
+    if (status == WG_ABANDONED || status == WG_IRREGULAR) return false;
+    if (err) throw DeviceError(refine_error_text((int32_t)err));
+    if (status != WG_DONE) throw DeviceError("team refinement made no progress");
+    cut_ = out[0];
+    total_imb_ = out[1];
+    rec.iterations = (int32_t)out[2];
+    rec.lp_iterations = (int32_t)out[3];
+    gen_ += rec.iterations;
+    if (out[4]) changed_ = true;
+    rec.cut2 = cut_;
+    rec.total_imb = total_imb_;
+    rec.n = g.n;
+    rec.m = g.m;
+    return true;
+}
+
+// The level's iterations in the graph-tagged one-workgroup kernel
+// (csrc/refine_wg.hip), from the tables init_conn built. The kernel stops
+// early only when a step chose update_large: the marked rows are then rebuilt
+// here, by the same multi-workgroup build as flush_rebuild, and the kernel
+// continues.
 LevelRecord Refiner::refine_wg(const Level& L, part_t* best_part, const std::vector<double>& temps) {
     DGraph g = L.view();
     const int32_t k = p_.k;
@@ -2823,13 +2920,7 @@ LevelRecord Refiner::refine_wg(const Level& L, part_t* best_part, const std::vec
     WgState h{};
     for (int launches = 0;; launches++) {
         if (launches > 100000) throw DeviceError("one-workgroup refinement made no progress");
-        if (WgCollector* col = wg_collector()) {
-            col->run(P, s_, h);  // graph-tagged with the levels of other jobs
-        } else {
-            launch_refine_wg(P, s_);
-            JET_HIP(hipMemcpyAsync(&h, wg_state_, sizeof(h), hipMemcpyDeviceToHost, s_));
-            JET_HIP(hipStreamSynchronize(s_));
-        }
+        wg_collector()->run(P, s_, h);  // graph-tagged with the levels of other jobs
         if (h.err) throw DeviceError(refine_error_text(h.err));
         if (h.status == WG_STALLED) throw DeviceError("one-workgroup refinement exceeded its iteration bound");
         if (h.status != WG_REBUILD) break;

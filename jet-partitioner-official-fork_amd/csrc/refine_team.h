@@ -1,0 +1,108 @@
+// Whole-level refinement by a team of workgroups on one XCD (host side).
+#pragma once
+#include <hip/hip_runtime.h>
+
+#include "jet_types.h"
+#include "refine_wg.h"
+
+namespace jet {
+
+constexpr int TEAM_MAX = 32;          // workgroups of a team: one per CU of an XCD
+constexpr int32_t TEAM_OWN = 2048;    // vertices a workgroup owns at most
+constexpr int32_t TEAM_MAX_N = TEAM_MAX * TEAM_OWN;
+constexpr int64_t TEAM_MAX_M = 600000;
+// Jobs of contexts of many workers use teams on levels of up to this many
+// vertices: a team kernel holds one of the process's four hardware queues for
+// the whole level, and the workgroups of its launch that fall on an XCD where
+// another team runs wait for a free CU. 60 mixed graphs on 16 workers: 298-312
+// ms without teams, 284 up to 512 vertices, 275 up to 2048, 268-273 up to
+// 4096, 287 up to 8192, 342 up to 65,536.
+constexpr int32_t TEAM_BATCH_N = 4096;
+constexpr int32_t TEAM_MAX_K = 256;
+constexpr int32_t TEAM_MAX_NBK = 16384;
+
+// Device words the team shares: start-up, the barrier, and the step's sums.
+// Each group of words that is polled or added to has a 128-byte line.
+struct TeamCtl {
+    int32_t arrived, pad0[31];
+    int32_t members, pad1[31];
+    int32_t state, pad2[31];  // 0 undecided, 1 go, 2 abandoned
+    uint32_t bar, pad3[31];
+    int32_t moves[2], ranked, redraws, err, fail, max_deg, pad4[25];
+    int64_t cut[2], pad5[14];
+};
+
+struct TeamParams {
+    DGraph g;
+    int32_t k, sections, nbk;
+    int32_t big_deg;  // items of higher degree are taken by a whole wave
+    int32_t lanes;    // lanes per smaller item: a power of two up to a wave
+    int32_t team;     // workgroups wanted
+    int32_t xcd;      // the XCD they run on
+    int32_t own;      // consecutive vertices of a workgroup's chunks (launch_refine_team sets it)
+    int64_t opt, size_max, imb_max, max_dest_weak, max_dest_strong;
+    double tol;
+    int32_t ntemps;
+    double temps[WG_MAX_TEMPS];
+    int64_t cut, imb;  // of the partition the level starts from
+    part_t* part;
+    part_t* best_part;  // in: the level's partition; out: the best one
+    int2* conn;         // m slots: the table of row i starts at slot rowptr[i]
+    int32_t* conn_size;
+    part_t* dest_cache;
+    int32_t* lock;
+    int32_t* gain_p;
+    int32_t* pregain;
+    part_t* dest;
+    int32_t* bid;
+    int32_t* stamp;
+    int32_t gen0;  // the level's steps stamp gen0 + 1, gen0 + 2, ...
+    int32_t* mark;     // n zeros
+    int64_t* score;    // n
+    uint64_t* rkey;    // n
+    int32_t* rweight;  // n
+    vid_t* redraw;     // n
+    int32_t* buckets;  // nbk + 1 zeros
+    int64_t* sizes;
+    int64_t* best_sizes;
+    int64_t* evict_adjust;
+    TeamCtl* ctl;
+    int64_t* host_out;  // TEAM_OUT_WORDS mapped host words, then the sequence word
+    int64_t seq;
+};
+
+constexpr int TEAM_OUT_WORDS = 7;  // best cut, best imbalance, iterations, LP iterations, changed, status, error bits
+// Levels of more edges are refined by a team only when no row is longer.
+constexpr int64_t TEAM_REGULAR_M = 100000;
+constexpr int32_t TEAM_MAX_DEG = 128;
+
+// Whether a level fits the team kernel's limits.
+bool team_fits(int64_t n, int64_t m, int32_t k, int64_t nbk, int64_t max_n);
+// Workgroups for a level of n vertices and m edges.
+int32_t team_size(int64_t n, int64_t m);
+// Clears the control words and the bucket sums and copies the best part sizes
+// to the current ones, then runs the level, on stream s. The result words are
+// published to p.host_out; status WG_ABANDONED (or a finished stream without a
+// result) means that no team could start: the level's arrays are untouched.
+// WG_IRREGULAR: the level has rows of more than TEAM_MAX_DEG edges, and too
+// many edges (likewise nothing has changed).
+enum : int32_t { WG_ABANDONED = 3, WG_IRREGULAR = 4 };
+void launch_refine_team(TeamParams p, hipStream_t s);
+
+// A place for `team` workgroups on an XCD of the device, held while a team
+// kernel runs there: the teams in flight on an XCD never need more CUs than
+// it has, so that every team finds room for all of its workgroups. Waits
+// until one is free.
+class TeamSlot {
+  public:
+    explicit TeamSlot(int32_t team);
+    ~TeamSlot();
+    TeamSlot(const TeamSlot&) = delete;
+    TeamSlot& operator=(const TeamSlot&) = delete;
+    int32_t xcd() const { return xcd_; }
+
+  private:
+    int32_t dev_ = 0, xcd_ = 0, team_ = 0;
+};
+
+}  // namespace jet

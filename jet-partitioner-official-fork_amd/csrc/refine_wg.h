@@ -61,8 +61,6 @@ constexpr int32_t WG_MAX_NBK = 16384;
 bool wg_fits(int64_t n, int32_t k, int64_t nbk, int64_t max_n);
 // Fresh controller state for a level: current and best cut / imbalance.
 void wg_init_state(WgState* st, int64_t cut, int64_t imb, hipStream_t s);
-// One launch of the kernel on stream s.
-void launch_refine_wg(const WgParams& p, hipStream_t s);
 // Gathers the one-workgroup level runs of concurrent jobs into graph-tagged
 // launches (the batched and served layer has one per context). run() first
 // waits for the job's stream (the level's tables and state are built there),

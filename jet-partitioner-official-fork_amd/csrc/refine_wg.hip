@@ -730,8 +730,6 @@ __device__ __forceinline__ void refine_wg_body(const WgParams& P, WgState* mirro
     }
 }
 
-__global__ void __launch_bounds__(WG_BLOCK) k_refine_wg(WgParams P) { refine_wg_body(P, nullptr); }
-
 // Graph-tagged: workgroup b runs the level that ps[b] describes (levels of
 // different graphs, each with its own arrays), and copies its final state to
 // states[b].
@@ -753,17 +751,17 @@ void wg_init_state(WgState* st, int64_t cut, int64_t imb, hipStream_t s) {
 
 // The dynamic LDS of the bucket array may take the kernels past 64 KB
 // (gfx950 has 160 KB per workgroup): allowed once per device and kernel.
-static void allow_wg_lds(const void* kernel, int which) {
-    static std::once_flag once[2][64];
-    static hipError_t attr_rc[2][64];
+static void allow_wg_lds(const void* kernel) {
+    static std::once_flag once[64];
+    static hipError_t attr_rc[64];
     int dev = 0;
     JET_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64) throw DeviceError("device index beyond 64");
-    std::call_once(once[which][dev], [&] {
-        attr_rc[which][dev] = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+    std::call_once(once[dev], [&] {
+        attr_rc[dev] = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                                   (int)(sizeof(int32_t) * (WG_MAX_NBK + 1)));
     });
-    JET_HIP(attr_rc[which][dev]);
+    JET_HIP(attr_rc[dev]);
 }
 
 static void check_wg_params(const WgParams& p) {
@@ -771,18 +769,10 @@ static void check_wg_params(const WgParams& p) {
         throw DeviceError("one-workgroup refinement: level outside the kernel's limits");
 }
 
-void launch_refine_wg(const WgParams& p, hipStream_t s) {
-    allow_wg_lds(reinterpret_cast<const void*>(&k_refine_wg), 0);
-    check_wg_params(p);
-    const size_t dyn = sizeof(int32_t) * (size_t)(p.nbk + 1);
-    k_refine_wg<<<1, WG_BLOCK, dyn, s>>>(p);
-    JET_LAUNCH_CHECK();
-}
-
 void launch_refine_wg_multi(const WgParams* host_ps, const WgParams* dev_ps, WgState* dev_states, int count,
                             hipStream_t s) {
     if (count <= 0) return;
-    allow_wg_lds(reinterpret_cast<const void*>(&k_refine_wg_multi), 1);
+    allow_wg_lds(reinterpret_cast<const void*>(&k_refine_wg_multi));
     int32_t nbk = 1;
     for (int i = 0; i < count; i++) {
         check_wg_params(host_ps[i]);

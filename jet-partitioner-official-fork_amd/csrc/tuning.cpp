@@ -22,14 +22,6 @@ Tuning& tuning() {
 }
 
 namespace {
-thread_local bool t_batch_thread = false;
-}
-
-void set_batch_thread(bool on) { t_batch_thread = on; }
-
-int64_t wg_threshold() { return t_batch_thread ? tuning().batch_wg_max_n : tuning().wg_max_n; }
-
-namespace {
 struct Field {
     const char* name;
     int64_t Tuning::*member;

@@ -9,16 +9,17 @@
 namespace jet {
 
 struct Tuning {
-    // levels of up to this many vertices are refined by the one-workgroup
-    // kernel (0: never)
-    int64_t wg_max_n = 0;
-    // the same threshold for jobs of the batched and served layer on contexts
-    // of at least BATCH_WG_MIN_WORKERS workers, whose many concurrent small
-    // jobs are bound by kernel launches more than by kernel time (their
-    // one-workgroup levels are launched together, one launch per round)
+    // levels of up to this many vertices (at most 65536, 256 parts, and not
+    // too many edges: team_fits) are refined in one launch by a team of
+    // workgroups on one XCD (0: never)
+    int64_t wg_max_n = 65536;
+    // jobs of the batched and served layer on contexts of at least
+    // BATCH_WG_MIN_WORKERS workers: levels of up to this many vertices are
+    // refined by one workgroup each, the levels of concurrent jobs in one
+    // launch (0: never)
     int64_t batch_wg_max_n = 0;
-    // in that kernel, candidates and moves of higher degree are taken by a
-    // whole wave instead of one thread
+    // in both kernels, candidates and moves of higher degree are taken by a
+    // whole wave instead of a group of lanes
     int64_t wg_big_deg = 32;
     // "small" levels: every connectivity row is built by a wave, the
     // afterburner takes ab_lanes_small times its lanes per candidate, and the
@@ -54,12 +55,6 @@ Tuning& tuning();
 // Contexts with fewer workers gather too few levels per launch for the
 // one-workgroup kernel to pay: their jobs refine as single calls do.
 constexpr int BATCH_WG_MIN_WORKERS = 8;
-// Marks the calling thread as a worker of the batched and served layer.
-void set_batch_thread(bool on);
-// The one-workgroup refinement threshold for the calling thread: wg_max_n,
-// or batch_wg_max_n on batch worker threads.
-int64_t wg_threshold();
-
 // Applies a tuning table (lines "name value"; '#' starts a comment). Returns
 // the number of settings applied, or -1 when the file cannot be read or holds
 // an unknown name or a value out of range (nothing is applied then).

@@ -30,7 +30,7 @@ SPACE = {
     "lp_one_pass_n": [131072, 524288, 2097152],
     "ct_wave_max": [32, 64, 128],
     "ct_block_max": [1024, 4096],
-    "wg_max_n": [0, 1024, 4096, 16384],
+    "wg_max_n": [0, 1024, 4096, 16384, 65536],
     "wg_big_deg": [0, 8, 32],
     "redraw_lds_max": [0, 8192],
     "sel_max_blocks": [512, 1024, 2048, 4096, 8192],
