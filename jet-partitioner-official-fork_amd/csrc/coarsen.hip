@@ -11,6 +11,8 @@
 //  * matchHash: candidates with equal digest pair two at a time in increasing
 //    vertex id (a stable sort by digest groups them).
 #include "coarsen.h"
+#include "coarsen_rules.h"
+#include "coarsen_team.h"
 #include "prims.h"
 #include "wave.h"
 
@@ -376,16 +378,6 @@ __global__ void k_match_init_uniform(DGraph g, uint64_t seed, uint32_t level, vi
     }
 }
 
-// pickMatch choice: lexicographic max of (weight, xorshift32(v + r)) over
-// eligible neighbours with weight >= 0 (weight ignored when UNIFORM).
-__device__ inline void pick_better(int64_t& bw, uint32_t& bh, vid_t& bv, int64_t w, uint32_t h, vid_t v) {
-    if (bv == ORD_MAX || w > bw || (w == bw && h > bh)) {
-        bw = w;
-        bh = h;
-        bv = v;
-    }
-}
-
 template <bool INITIAL>
 __device__ inline bool pick_skip(vid_t u, const vid_t* vcmap, const vid_t* hn) {
     if (INITIAL) return false;
@@ -692,6 +684,10 @@ int32_t coarsen_match(const DGraph& g, bool uniform, uint64_t seed, int32_t leve
                       Arena& a, hipStream_t s) {
     vid_t n = g.n;
     if (n <= 0) return 0;
+    if (team_match_fits(n, g.m)) {
+        const int32_t nc = coarsen_match_team(g, uniform, seed, level, two_hop, map, a, s);
+        if (nc >= 0) return nc;
+    }
     ArenaScope sc(a);
     vid_t* hn = a.alloc<vid_t>(n);
     vid_t* vcmap = a.alloc<vid_t>(n);

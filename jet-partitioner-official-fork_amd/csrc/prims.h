@@ -36,6 +36,13 @@ void peek_to_mailbox(const void* src, int bytes, int slot, hipStream_t s);
 // per-iteration results.
 void read_i32_words(const int32_t* src, int count, int32_t* out, hipStream_t s);
 
+// Waits until *word (a mailbox word a kernel on stream s writes last) holds
+// seq: a poll of host memory returns within a microsecond or two of the write,
+// where a stream synchronisation sleeps and wakes. Every few thousand polls
+// the stream is queried: false when it finished without the word, an exception
+// on an error.
+bool wait_mailbox(volatile int64_t* word, int64_t seq, hipStream_t s);
+
 // out[i] = in[0] + ... + in[i-1] for i in [0, n]; out has n + 1 entries
 // (out[n] is the total). `in` and `out` may alias when the types match.
 void excl_scan_i32_i32(const int32_t* in, int32_t* out, int64_t n, Arena& a, hipStream_t s);

@@ -1,6 +1,8 @@
 // Device-wide primitives for the Jet hot path on gfx950.
 #include "prims.h"
 
+#include <sched.h>
+
 #include <algorithm>
 #include <stdexcept>
 #include "wave.h"
@@ -56,6 +58,21 @@ Mailbox& thread_mailbox() {
         JET_HIP(hipHostGetDevicePointer(reinterpret_cast<void**>(&mb.dev), mb.host, 0));
     }
     return mb;
+}
+
+bool wait_mailbox(volatile int64_t* word, int64_t seq, hipStream_t s) {
+    for (uint64_t spins = 1;; spins++) {
+        if (*word == seq) return true;
+        __builtin_ia32_pause();
+        // a wait longer than about half a millisecond (the device is busy with
+        // other work, e.g. concurrent jobs) gives the CPU to other threads
+        if (spins >= (1u << 14) && spins % 64 == 0) sched_yield();
+        if (spins % 4096 == 0) {
+            const hipError_t e = hipStreamQuery(s);
+            if (e == hipSuccess) return *word == seq;
+            if (e != hipErrorNotReady) JET_HIP(e);
+        }
+    }
 }
 
 void peek_to_mailbox(const void* src, int bytes, int slot, hipStream_t s) {

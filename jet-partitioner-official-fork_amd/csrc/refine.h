@@ -190,7 +190,7 @@ class Refiner {
     // the team kernel's tables (rows at their adjacency's offset), control
     // words and scratch
     int2* team_conn_ = nullptr;
-    TeamCtl* team_ctl_ = nullptr;
+    RefineCtl* team_ctl_ = nullptr;
     int32_t* team_buckets_ = nullptr;
     uint64_t* team_rkey_ = nullptr;
     int32_t* team_rweight_ = nullptr;

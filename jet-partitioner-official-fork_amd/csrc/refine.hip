@@ -21,7 +21,6 @@
 #include <algorithm>
 #include <chrono>
 #include <cmath>
-#include <sched.h>
 
 #include "prims.h"
 #include "prof.h"
@@ -2243,7 +2242,7 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     wg_list_ = a.alloc<vid_t>(N);
     wg_runb_ = a.alloc<int32_t>(WG_MAX_NBK + 1);
     team_conn_ = a.alloc<int2>(TEAM_MAX_M);
-    team_ctl_ = a.alloc<TeamCtl>(1);
+    team_ctl_ = a.alloc<RefineCtl>(1);
     team_buckets_ = a.alloc<int32_t>(TEAM_MAX_NBK + 1);
     team_rkey_ = a.alloc<uint64_t>(std::min<int64_t>(N, TEAM_MAX_N));
     team_rweight_ = a.alloc<int32_t>(std::min<int64_t>(N, TEAM_MAX_N));
@@ -2534,29 +2533,9 @@ void Refiner::rebalance(const Level& L, const part_t* part, const int64_t* sizes
     if (strong) strong_tail(L, part, sizes, r, true);
 }
 
-// Waits for the step's sequence word in the mapped mailbox: a poll of host
-// memory returns within a microsecond or two of the write, where a stream
-// synchronisation sleeps and wakes. Every few thousand polls the stream is
-// queried, so an error or a stream that finished without the word ends the
-// wait.
+// Waits for the step's results in the mapped mailbox.
 void Refiner::wait_published(volatile int64_t* res, int64_t seq) {
-    for (uint64_t spins = 1;; spins++) {
-        if (res[5] == seq) return;
-        __builtin_ia32_pause();
-        // a wait longer than about half a millisecond (the device is busy with
-        // other work, e.g. concurrent jobs) gives the CPU to other threads
-        if (spins >= (1u << 14) && spins % 64 == 0) sched_yield();
-        if (spins % 4096 == 0) {
-            hipError_t e = hipStreamQuery(s_);
-            if (e == hipSuccess) {
-                if (res[5] == seq) return;
-                throw DeviceError("refinement step finished without publishing its results");
-            }
-            if (e != hipErrorNotReady) {
-                JET_HIP(e);
-            }
-        }
-    }
+    if (!wait_mailbox(&res[5], seq, s_)) throw DeviceError("refinement step finished without publishing its results");
 }
 
 bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_t& cut_change, int64_t& max_size,
@@ -2842,18 +2821,7 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
     TeamSlot slot(P.team);
     P.xcd = slot.xcd();
     launch_refine_team(P, s_);
-    for (uint64_t spins = 1; out[TEAM_OUT_WORDS] != P.seq; spins++) {
-        __builtin_ia32_pause();
-        if (spins >= (1u << 14) && spins % 64 == 0) sched_yield();
-        if (spins % 4096 == 0) {
-            const hipError_t e = hipStreamQuery(s_);
-            if (e == hipSuccess) {
-                if (out[TEAM_OUT_WORDS] == P.seq) break;
-                return false;  // no workgroup ran on the wanted XCD
-            }
-            if (e != hipErrorNotReady) JET_HIP(e);
-        }
-    }
+    if (!wait_mailbox(&out[TEAM_OUT_WORDS], P.seq, s_)) return false;  // no workgroup ran on the wanted XCD
     const int64_t status = out[5], err = out[6];
     if (status == WG_IRREGULAR) team_irregular_ = true;
     if (status == WG_ABANDONED || status == WG_IRREGULAR) return false;

@@ -4,13 +4,10 @@
 
 #include "jet_types.h"
 #include "refine_wg.h"
+#include "team.h"
 
 namespace jet {
 
-constexpr int TEAM_MAX = 32;          // workgroups of a team: one per CU of an XCD
-constexpr int32_t TEAM_OWN = 2048;    // vertices a workgroup owns at most
-constexpr int32_t TEAM_MAX_N = TEAM_MAX * TEAM_OWN;
-constexpr int64_t TEAM_MAX_M = 600000;
 // Jobs of contexts of many workers use teams on levels of up to this many
 // vertices: a team kernel holds one of the process's four hardware queues for
 // the whole level, and the workgroups of its launch that fall on an XCD where
@@ -18,17 +15,14 @@ constexpr int64_t TEAM_MAX_M = 600000;
 // ms without teams, 284 up to 512 vertices, 275 up to 2048, 268-273 up to
 // 4096, 287 up to 8192, 342 up to 65,536.
 constexpr int32_t TEAM_BATCH_N = 4096;
+constexpr int64_t TEAM_MAX_M = 600000;
 constexpr int32_t TEAM_MAX_K = 256;
 constexpr int32_t TEAM_MAX_NBK = 16384;
 
-// Device words the team shares: start-up, the barrier, and the step's sums.
-// Each group of words that is polled or added to has a 128-byte line.
-struct TeamCtl {
-    int32_t arrived, pad0[31];
-    int32_t members, pad1[31];
-    int32_t state, pad2[31];  // 0 undecided, 1 go, 2 abandoned
-    uint32_t bar, pad3[31];
-    int32_t moves[2], ranked, redraws, err, fail, max_deg, pad4[25];
+// Device words the level's team shares: the team's own, and the step's sums.
+struct RefineCtl {
+    TeamCtl team;
+    int32_t moves[2], ranked, redraws, err, max_deg, pad4[26];
     int64_t cut[2], pad5[14];
 };
 
@@ -66,7 +60,7 @@ struct TeamParams {
     int64_t* sizes;
     int64_t* best_sizes;
     int64_t* evict_adjust;
-    TeamCtl* ctl;
+    RefineCtl* ctl;
     int64_t* host_out;  // TEAM_OUT_WORDS mapped host words, then the sequence word
     int64_t seq;
 };
@@ -88,21 +82,5 @@ int32_t team_size(int64_t n, int64_t m);
 // many edges (likewise nothing has changed).
 enum : int32_t { WG_ABANDONED = 3, WG_IRREGULAR = 4 };
 void launch_refine_team(TeamParams p, hipStream_t s);
-
-// A place for `team` workgroups on an XCD of the device, held while a team
-// kernel runs there: the teams in flight on an XCD never need more CUs than
-// it has, so that every team finds room for all of its workgroups. Waits
-// until one is free.
-class TeamSlot {
-  public:
-    explicit TeamSlot(int32_t team);
-    ~TeamSlot();
-    TeamSlot(const TeamSlot&) = delete;
-    TeamSlot& operator=(const TeamSlot&) = delete;
-    int32_t xcd() const { return xcd_; }
-
-  private:
-    int32_t dev_ = 0, xcd_ = 0, team_ = 0;
-};
 
 }  // namespace jet

@@ -8,22 +8,7 @@
 // iteration's four to nine kernels and a host round trip for the controller.
 // Here one launch runs the level: it builds the connectivity tables, iterates
 // and keeps the controller (step choice, best state, counters, temperatures),
-// with barriers between the steps. A device-wide barrier costs 5 us and more,
-// because the XCDs' L2s are made coherent by writing them back; the CUs of one
-// XCD share its L2, so a team of workgroups of one XCD needs no cache
-// maintenance at all: stores are written through to the L2 and waited for
-// (s_waitcnt) before the barrier, and everything another workgroup may have
-// changed is read with agent-scope loads, which pass by the CU's own cache.
-// Measured: 0.6 us per barrier and exchange for 8 workgroups, 0.9 us for 32,
-// against 4.4 and 8.8 us for a device-wide barrier; an L2 hit takes about
-// 0.1 us where a load after a kernel boundary takes 0.5 us.
-//
-// The launch starts eight workgroups (one per XCD in dispatch order) for each
-// one wanted; each reads the number of its XCD, and those elsewhere end at
-// once. The first member waits until every workgroup of the launch has
-// arrived, with a bound, and then starts the team or abandons it (the host
-// then takes the multi-kernel path): nothing waits for a workgroup that might
-// not run, and every later wait is bounded too.
+// with the team's barriers (team_dev.h) between the steps.
 //
 // Vertices are owned by workgroups (8 to 64 consecutive ones in turn). A workgroup
 // selects among its vertices, keeps its candidates and moves in LDS lists, and
@@ -34,12 +19,11 @@
 // directly or scanned over the chunks, instead of by sorting.
 #include "refine_team.h"
 
-#include <sched.h>
-
 #include <algorithm>
 #include <mutex>
 
 #include "conn_table.h"
+#include "team_dev.h"
 #include "wave.h"
 
 namespace jet {
@@ -49,8 +33,6 @@ namespace jet {
 constexpr int TM_BLOCK = 1024;
 constexpr int TM_WAVES = TM_BLOCK / WAVE;
 constexpr int32_t TM_ITER_CAP = 1 << 16;
-constexpr int32_t TM_START_SPINS = 1 << 19;  // some 0.1 s for every workgroup to arrive
-constexpr int32_t TM_SPINS = 1 << 24;        // seconds: the members are resident
 constexpr int32_t TM_LANES = 16;             // lanes that build a row of at most TM_SMALL edges
 constexpr int32_t TM_SMALL = 64;
 constexpr int32_t TM_TABLE = 256;            // table slots of a wave: WAVE / TM_LANES * TM_SMALL, and TEAM_MAX_K
@@ -90,12 +72,6 @@ struct TeamShared {
     WgState S;
 };
 
-__device__ inline int64_t ldr64(const int64_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ inline uint64_t ldr64(const uint64_t* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
 __device__ inline int2 ldr_slot(const int2* p) {
     const uint64_t x = ldr64(reinterpret_cast<const uint64_t*>(p));
     return make_int2((int32_t)(uint32_t)x, (int32_t)(uint32_t)(x >> 32));
@@ -113,37 +89,6 @@ __device__ inline void for_slots_rx(const int2* tab, int32_t sz, F&& f) {
             if (s0 + u < sz) f(e[u]);
     }
 }
-
-__device__ inline int32_t xcd_id() {
-    return (int32_t)(__builtin_amdgcn_s_getreg(20 | (3 << 11)) & 15);  // HW_REG_XCC_ID, bits 0-3
-}
-
-// Barrier of the team's workgroups; false when a wait ran out (never, unless
-// an invariant is broken: all members are resident).
-struct Team {
-    TeamCtl* c;
-    int32_t size, me;
-    uint32_t target = 0;
-    int32_t* ok;  // LDS
-    __device__ bool sync() {
-        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // stores and atomics have reached the L2
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            target += (uint32_t)size;
-            __hip_atomic_fetch_add(&c->bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            int32_t spins = 0;
-            while ((int32_t)(__hip_atomic_load(&c->bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - target) < 0) {
-                if (++spins > TM_SPINS) {
-                    *ok = 0;
-                    atomicOr(&c->fail, 1);
-                    break;
-                }
-            }
-        }
-        __syncthreads();
-        return *ok != 0;
-    }
-};
 
 // Appends to an LDS list of TEAM_OWN items: small items from the front, big
 // ones from the back.
@@ -239,12 +184,6 @@ __device__ inline void tm_build_row(const TeamParams& P, const part_t* part, vid
     wave_sync();
 }
 
-// The workgroup's x-th own vertex: chunks of `own` consecutive vertices go to
-// the team's workgroups in turn.
-__device__ inline int64_t own_vertex(int32_t x, int32_t own, int32_t team, int32_t me) {
-    return ((int64_t)(x / own) * team + me) * own + x % own;
-}
-
 // Tables of the workgroup's own rows (marked: only those with a mark, which
 // is cleared), from the parts in `part`: 64 vertices at a time, four by each
 // wave (16 lanes a row, or one row after another when they are longer).
@@ -327,10 +266,10 @@ __device__ inline void tm_publish(const TeamParams& P, const WgState& S, int32_t
 
 }  // namespace
 
-__global__ void __launch_bounds__(256) k_team_prep(TeamCtl* ctl, int32_t* buckets, int32_t nb, int64_t* sizes,
+__global__ void __launch_bounds__(256) k_team_prep(RefineCtl* ctl, int32_t* buckets, int32_t nb, int64_t* sizes,
                                                   const int64_t* best_sizes, int32_t k) {
     const int32_t t = blockIdx.x * 256 + threadIdx.x;
-    constexpr int32_t W = sizeof(TeamCtl) / 4;
+    constexpr int32_t W = sizeof(RefineCtl) / 4;
     if (t < W) reinterpret_cast<int32_t*>(ctl)[t] = 0;
     for (int32_t x = t; x < nb; x += gridDim.x * 256) buckets[x] = 0;
     for (int32_t x = t; x < k; x += gridDim.x * 256) sizes[x] = best_sizes[x];
@@ -347,44 +286,17 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
     const int t = threadIdx.x;
     const int lane = t & (WAVE - 1);
     const int wv = t / WAVE;
-    TeamCtl* C = P.ctl;
+    RefineCtl* C = P.ctl;
     int32_t* err = &C->err;
 
     // ------------------------------------------------------------ start-up
     if (t == 0) {
-        L.go = 0;
-        const bool here = xcd_id() == P.xcd;
-        int32_t me = P.team;
-        if (here) me = __hip_atomic_fetch_add(&C->members, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        // ordered after the registration: a wait for the returned value
-        asm volatile("s_waitcnt vmcnt(0)" ::"v"(me) : "memory");
-        __hip_atomic_fetch_add(&C->arrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (here && me < P.team) {
-            int32_t st = 0;
-            if (me == 0) {
-                int32_t spins = 0;
-                while (ld_rx(&C->arrived) < (int32_t)gridDim.x && ++spins <= TM_START_SPINS) {
-                }
-                const int32_t size = min(ld_rx(&C->members), P.team);
-                const bool enough = (int64_t)size * TEAM_OWN >= n;
-                st = ld_rx(&C->arrived) >= (int32_t)gridDim.x && enough ? 1 : 2;
-                __hip_atomic_store(&C->state, st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            } else {
-                int32_t spins = 0;
-                while ((st = ld_rx(&C->state)) == 0 && ++spins <= TM_SPINS) {
-                }
-            }
-            if (st == 1) {
-                L.go = 1;
-                L.size = min(ld_rx(&C->members), P.team);
-                L.me = me;
-            } else if (me == 0) {
-                WgState S{};
-                S.status = WG_ABANDONED;
-                tm_publish(P, S, 0);
-            }
-        }
+        const int32_t st = team_start(C->team, P.xcd, P.team, ceil_div_dev(n, TEAM_OWN), L.go, L.size, L.me);
         WgState S{};
+        if (st == TEAM_ABANDON) {
+            S.status = WG_ABANDONED;
+            tm_publish(P, S, 0);
+        }
         S.curr_cut = S.best_cut = P.cut;
         S.curr_imb = S.best_imb = P.imb;
         S.status = WG_DONE;
@@ -393,7 +305,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
     __syncthreads();
     if (!L.go) return;
     const int32_t T = L.size, me = L.me;
-    Team team{C, T, me, 0, &L.go};
+    Team team{&C->team, T, me, 0, &L.go};
     // this workgroup's vertices, a wave 64 of them at a time
     auto for_own = [&](auto&& f) {
         for (int32_t x0 = WAVE * wv;; x0 += WAVE * TM_WAVES) {
@@ -1058,7 +970,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
     }
     __syncthreads();
     if (me == 0 && t == 0) {
-        if (!alive || ld_rx(&C->fail)) L.S.status = WG_STALLED;
+        if (!alive || ld_rx(&C->team.fail)) L.S.status = WG_STALLED;
         tm_publish(P, L.S, ld_rx(err));
     }
 }
@@ -1118,37 +1030,6 @@ void launch_refine_team(TeamParams p, hipStream_t s) {
                                                                                     p.sizes, p.best_sizes, p.k);
     k_refine_team<<<8 * p.team, TM_BLOCK, team_lds(p), s>>>(p);
     JET_LAUNCH_CHECK();
-}
-
-namespace {
-constexpr int XCDS = 8;
-std::mutex g_slot_mu;
-int32_t g_slot_load[64][XCDS];
-}  // namespace
-
-TeamSlot::TeamSlot(int32_t team) : team_(team) {
-    int dev = 0;
-    JET_HIP(hipGetDevice(&dev));
-    dev_ = dev & 63;
-    for (;;) {
-        {
-            std::lock_guard<std::mutex> lk(g_slot_mu);
-            int best = 0;
-            for (int x = 1; x < XCDS; x++)
-                if (g_slot_load[dev_][x] < g_slot_load[dev_][best]) best = x;
-            if (g_slot_load[dev_][best] + team_ <= TEAM_MAX) {
-                g_slot_load[dev_][best] += team_;
-                xcd_ = best;
-                return;
-            }
-        }
-        sched_yield();
-    }
-}
-
-TeamSlot::~TeamSlot() {
-    std::lock_guard<std::mutex> lk(g_slot_mu);
-    g_slot_load[dev_][xcd_] -= team_;
 }
 
 }  // namespace jet

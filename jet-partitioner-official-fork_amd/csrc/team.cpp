@@ -1,0 +1,44 @@
+// Places for teams of workgroups on the device's XCDs (team.h).
+#include "team.h"
+
+#include <hip/hip_runtime.h>
+#include <sched.h>
+
+#include <mutex>
+
+#include "jet_types.h"
+
+namespace jet {
+
+namespace {
+constexpr int XCDS = 8;
+std::mutex g_slot_mu;
+int32_t g_slot_load[64][XCDS];
+}  // namespace
+
+TeamSlot::TeamSlot(int32_t team) : team_(team) {
+    int dev = 0;
+    JET_HIP(hipGetDevice(&dev));
+    dev_ = dev & 63;
+    for (;;) {
+        {
+            std::lock_guard<std::mutex> lk(g_slot_mu);
+            int best = 0;
+            for (int x = 1; x < XCDS; x++)
+                if (g_slot_load[dev_][x] < g_slot_load[dev_][best]) best = x;
+            if (g_slot_load[dev_][best] + team_ <= TEAM_MAX) {
+                g_slot_load[dev_][best] += team_;
+                xcd_ = best;
+                return;
+            }
+        }
+        sched_yield();
+    }
+}
+
+TeamSlot::~TeamSlot() {
+    std::lock_guard<std::mutex> lk(g_slot_mu);
+    g_slot_load[dev_][xcd_] -= team_;
+}
+
+}  // namespace jet
