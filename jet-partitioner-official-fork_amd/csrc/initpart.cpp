@@ -583,8 +583,8 @@ constexpr int32_t ML_MIN_N = 2000;
 constexpr int32_t ML_COARSEST = 1000;
 // graphs with at least this many adjacency entries are matched by
 // handshakes on host threads instead of the serial greedy pass
-constexpr int64_t PAR_MATCH_EDGES = int64_t(1) << 21;
-constexpr int HANDSHAKE_ROUNDS = 6;
+using jet_init::HANDSHAKE_ROUNDS;
+using jet_init::PAR_MATCH_EDGES;
 
 static void shuffle_ids(std::vector<int32_t>& p, uint64_t seed) {
     for (int32_t i = (int32_t)p.size() - 1; i > 0; i--) {
@@ -652,7 +652,7 @@ static void handshake_matching(const Sub& s, uint64_t seed, int64_t cap, int par
 
 static Sub coarsen_once(const Sub& s, uint64_t seed, int par, std::vector<int32_t>& cmap) {
     const int32_t n = s.n;
-    const int64_t cap = std::max<int64_t>(1, (int64_t)(1.5 * (double)s.total_w / ML_COARSEST));
+    const int64_t cap = jet_init::match_weight_cap(s.total_w);
     std::vector<int32_t> mate(n, -1);
     if ((int64_t)s.adj.size() >= PAR_MATCH_EDGES) {
         handshake_matching(s, seed, cap, par, mate);
@@ -678,53 +678,16 @@ static Sub coarsen_once(const Sub& s, uint64_t seed, int par, std::vector<int32_
             }
         }
     }
-    // leaves sharing a neighbour, and isolated vertices, in increasing id
-    std::vector<std::pair<int32_t, int32_t>> keyed;
-    int32_t last_isolated = -1;
-    for (int32_t v = 0; v < n; v++) {
-        if (mate[v] >= 0) continue;
-        if (s.xadj[v + 1] == s.xadj[v]) {
-            if (last_isolated >= 0 && (int64_t)s.vw[v] + s.vw[last_isolated] <= cap) {
-                mate[v] = last_isolated;
-                mate[last_isolated] = v;
-                last_isolated = -1;
-            } else {
-                last_isolated = v;
-            }
-            continue;
-        }
-        keyed.push_back({s.adj[s.xadj[v]], v});
-    }
-    std::sort(keyed.begin(), keyed.end());
-    for (size_t i = 0; i + 1 < keyed.size();) {
-        int32_t a = keyed[i].second, b = keyed[i + 1].second;
-        if (keyed[i].first == keyed[i + 1].first && (int64_t)s.vw[a] + s.vw[b] <= cap) {
-            mate[a] = b;
-            mate[b] = a;
-            i += 2;
-        } else {
-            i += 1;
-        }
-    }
-    cmap.assign(n, -1);
-    int32_t nc = 0;
-    for (int32_t v = 0; v < n; v++) {
-        if (cmap[v] >= 0) continue;
-        cmap[v] = nc;
-        if (mate[v] >= 0) cmap[mate[v]] = nc;
-        nc++;
-    }
+    std::vector<int32_t> first_adj(n);
+    for (int32_t v = 0; v < n; v++) first_adj[v] = s.xadj[v + 1] > s.xadj[v] ? s.adj[s.xadj[v]] : -1;
+    jet_init::CoarseMap cm = jet_init::finish_matching(n, mate, first_adj.data(), s.vw.data(), cap);
+    cmap = std::move(cm.map);
+    const int32_t nc = cm.n;
+    const std::vector<int32_t>&first = cm.first, &second = cm.second;
     Sub c;
     c.n = nc;
-    c.vw.assign(nc, 0);
+    c.vw.assign(cm.vw.data(), cm.vw.data() + nc);
     c.gid.resize(nc);
-    std::vector<int32_t> first(nc, -1), second(nc, -1);
-    for (int32_t v = 0; v < n; v++) {
-        int32_t cv = cmap[v];
-        c.vw[cv] += s.vw[v];
-        if (first[cv] < 0) first[cv] = v;
-        else second[cv] = v;
-    }
     c.total_w = s.total_w;
     for (int32_t cv = 0; cv < nc; cv++) c.gid[cv] = cv;
     // Rows are built in contiguous chunks of coarse ids, one per thread, each
@@ -934,8 +897,65 @@ namespace jet_init {
 
 void set_thread_budget(int threads) { t_thread_budget = threads > 0 ? threads : 0; }
 
+int32_t hierarchy_target(int32_t k) { return std::max<int32_t>(ML_COARSEST, 8 * k); }
+uint64_t level_seed(uint64_t seed, int lvl) { return seed + 0x1A17ULL * (uint64_t)(lvl + 1); }
+int64_t match_weight_cap(int64_t total_w) {
+    return std::max<int64_t>(1, (int64_t)(1.5 * (double)total_w / ML_COARSEST));
+}
+bool shrinks_enough(int32_t nc, int32_t n) { return !((double)nc > 0.9 * (double)n); }
+
+CoarseMap finish_matching(int32_t n, std::vector<int32_t>& mate, const int32_t* first_adj, const int32_t* vw,
+                          int64_t cap) {
+    // leaves sharing a neighbour, and isolated vertices, in increasing id
+    std::vector<std::pair<int32_t, int32_t>> keyed;
+    int32_t last_isolated = -1;
+    for (int32_t v = 0; v < n; v++) {
+        if (mate[v] >= 0) continue;
+        if (first_adj[v] < 0) {
+            if (last_isolated >= 0 && (int64_t)vw[v] + vw[last_isolated] <= cap) {
+                mate[v] = last_isolated;
+                mate[last_isolated] = v;
+                last_isolated = -1;
+            } else {
+                last_isolated = v;
+            }
+            continue;
+        }
+        keyed.push_back({first_adj[v], v});
+    }
+    std::sort(keyed.begin(), keyed.end());
+    for (size_t i = 0; i + 1 < keyed.size();) {
+        int32_t a = keyed[i].second, b = keyed[i + 1].second;
+        if (keyed[i].first == keyed[i + 1].first && (int64_t)vw[a] + vw[b] <= cap) {
+            mate[a] = b;
+            mate[b] = a;
+            i += 2;
+        } else {
+            i += 1;
+        }
+    }
+    CoarseMap c;
+    c.map.assign(n, -1);
+    for (int32_t v = 0; v < n; v++) {
+        if (c.map[v] >= 0) continue;
+        c.map[v] = c.n;
+        if (mate[v] >= 0) c.map[mate[v]] = c.n;
+        c.n++;
+    }
+    c.vw.assign(c.n, 0);
+    c.first.assign(c.n, -1);
+    c.second.assign(c.n, -1);
+    for (int32_t v = 0; v < n; v++) {
+        const int32_t cv = c.map[v];
+        c.vw[cv] += vw[v];
+        if (c.first[cv] < 0) c.first[cv] = v;
+        else c.second[cv] = v;
+    }
+    return c;
+}
+
 std::vector<HostLevel> init_hierarchy(int32_t n, const int64_t* xadj, const int32_t* adj, const int32_t* adjw,
-                                      const int32_t* vw, int32_t k, uint64_t seed) {
+                                      const int32_t* vw, int32_t k, uint64_t seed, int first_lvl) {
     std::vector<HostLevel> out;
     if (n <= 0) return out;
     Sub cur;
@@ -952,12 +972,12 @@ std::vector<HostLevel> init_hierarchy(int32_t n, const int64_t* xadj, const int3
         cur.gid[v] = v;
         cur.total_w += cur.vw[v];
     }
-    const int32_t target = std::max<int32_t>(ML_COARSEST, 8 * k);
+    const int32_t target = hierarchy_target(k);
     const int par = host_threads();
-    for (int lvl = 0; cur.n > target && lvl < 64; lvl++) {
+    for (int lvl = first_lvl; cur.n > target && lvl < MAX_LEVELS; lvl++) {
         std::vector<int32_t> cmap;
-        Sub c = coarsen_once(cur, seed + 0x1A17ULL * (uint64_t)(lvl + 1), par, cmap);
-        if ((double)c.n > 0.9 * (double)cur.n) break;
+        Sub c = coarsen_once(cur, level_seed(seed, lvl), par, cmap);
+        if (!shrinks_enough(c.n, cur.n)) break;
         HostLevel L;
         L.n = c.n;
         L.xadj.assign(c.xadj.begin(), c.xadj.end());

@@ -21,6 +21,7 @@
 #include "coarsen.h"
 #include "engine.h"
 #include "hierarchy.h"
+#include "init_dev.h"
 #include "contract.h"
 #include "jet_capi.h"
 #include "misc.h"
@@ -401,47 +402,93 @@ static void uncoarsen_levels(Context& C, const jet_config_t& cfg, const std::vec
     R.t_refine = secs(t_start, clk::now());
 }
 
+// A level's graph on the host.
+struct HostGraph {
+    std::vector<int64_t> rp;
+    std::vector<int32_t> col, ew, vw;
+};
+static HostGraph fetch_graph(Context& C, const Level& L) {
+    HostGraph h;
+    h.rp.resize((size_t)L.n + 1);
+    h.col.resize(L.m);
+    h.ew.resize(L.m);
+    h.vw.resize(L.n);
+    hipStream_t s = C.stream;
+    JET_HIP(hipMemcpyAsync(h.rp.data(), L.rowptr, sizeof(int64_t) * (L.n + 1), hipMemcpyDeviceToHost, s));
+    if (L.m > 0) {
+        JET_HIP(hipMemcpyAsync(h.col.data(), L.col, sizeof(int32_t) * L.m, hipMemcpyDeviceToHost, s));
+        JET_HIP(hipMemcpyAsync(h.ew.data(), L.ew, sizeof(int32_t) * L.m, hipMemcpyDeviceToHost, s));
+    }
+    JET_HIP(hipMemcpyAsync(h.vw.data(), L.vw, sizeof(int32_t) * L.n, hipMemcpyDeviceToHost, s));
+    JET_HIP(hipStreamSynchronize(s));
+    return h;
+}
+
+static void host_initpart(const jet_config_t& cfg, int32_t n, const int64_t* rp, const int32_t* col, const int32_t* ew,
+                          const int32_t* vw, uint64_t seed, int32_t* part) {
+    if (jet_host_initpart(n, rp, col, ew, vw, cfg.num_parts, cfg.max_imb_ratio, seed, part) != 0)
+        throw InitFailure("initial partitioner could not partition the coarsest graph");
+}
+
 // The initial partition of a large coarsest graph `cs`, multilevel k-way
-// (initpart.h): the host coarsens it further, partitions the smallest level
-// by recursive bisection, and each level of that hierarchy is refined on the
-// device with Jet refinement (its own refine_data) before its partition is
-// projected to the next finer one; the partition of `cs` itself is left to
-// the uncoarsening that follows. Levels live in `persist`, the refinement
-// state in `scratch`.
-static void initial_partition_multilevel(Context& C, const jet_config_t& cfg, const Level& cs,
-                                         const std::vector<int64_t>& h_rp, const std::vector<int32_t>& h_col,
-                                         const std::vector<int32_t>& h_ew, const std::vector<int32_t>& h_vw,
-                                         uint64_t seed, part_t* cs_part) {
+// (initpart.h): it is coarsened further (levels of at least PAR_MATCH_EDGES
+// entries on the device, smaller ones on the host), the smallest level is
+// partitioned by recursive bisection on the host, and each level of that
+// hierarchy is refined on the device with Jet refinement (its own refine_data)
+// before its partition is projected to the next finer one; the partition of
+// `cs` itself is left to the uncoarsening that follows. Levels live in
+// `persist`, the refinement state in `scratch`.
+static void initial_partition_multilevel(Context& C, const jet_config_t& cfg, const Level& cs, uint64_t seed,
+                                         part_t* cs_part) {
     hipStream_t s = C.stream;
     const int32_t k = cfg.num_parts;
-    std::vector<jet_init::HostLevel> H =
-        jet_init::init_hierarchy(cs.n, h_rp.data(), h_col.data(), h_ew.data(), h_vw.data(), k, seed);
+    // the hierarchy's levels, with the maps from the next finer one
+    std::vector<Level> D;
+    bool ended = false;  // by a level that would not shrink enough
+    {
+        std::vector<int32_t> vw = to_host(C, cs.vw, cs.n);
+        for (;;) {
+            const Level& fine = D.empty() ? cs : D.back();
+            if (fine.n <= jet_init::hierarchy_target(k) || (int)D.size() >= jet_init::MAX_LEVELS ||
+                fine.m < jet_init::PAR_MATCH_EDGES)
+                break;
+            Level next;
+            if (!init_coarsen_device(fine.view(), vw, seed, (int)D.size(), C.persist, C.scratch, s, next)) {
+                ended = true;
+                break;
+            }
+            D.push_back(next);
+        }
+    }
+    const HostGraph last = fetch_graph(C, D.empty() ? cs : D.back());
+    const int32_t last_n = D.empty() ? cs.n : D.back().n;
+    std::vector<jet_init::HostLevel> H;
+    if (!ended)
+        H = jet_init::init_hierarchy(last_n, last.rp.data(), last.col.data(), last.ew.data(), last.vw.data(), k, seed,
+                                     (int)D.size());
     std::vector<int32_t> hp;
-    if (H.empty()) {  // no coarser level: the recursive bisection alone
-        hp.resize(cs.n);
-        if (jet_host_initpart(cs.n, h_rp.data(), h_col.data(), h_ew.data(), h_vw.data(), k, cfg.max_imb_ratio, seed,
-                              hp.data()) != 0)
-            throw InitFailure("initial partitioner could not partition the coarsest graph");
+    if (H.empty()) {
+        hp.resize(last_n);
+        host_initpart(cfg, last_n, last.rp.data(), last.col.data(), last.ew.data(), last.vw.data(), seed, hp.data());
+    } else {
+        const jet_init::HostLevel& h = H.back();
+        hp.resize(h.n);
+        host_initpart(cfg, h.n, h.xadj.data(), h.adj.data(), h.adjw.data(), h.vw.data(), seed, hp.data());
+    }
+    if (D.empty() && H.empty()) {  // no coarser level: the recursive bisection alone
         JET_HIP(hipMemcpyAsync(cs_part, hp.data(), sizeof(int32_t) * cs.n, hipMemcpyHostToDevice, s));
+        JET_HIP(hipStreamSynchronize(s));
         return;
     }
-    const jet_init::HostLevel& last = H.back();
-    hp.resize(last.n);
-    if (jet_host_initpart(last.n, last.xadj.data(), last.adj.data(), last.adjw.data(), last.vw.data(), k,
-                          cfg.max_imb_ratio, seed, hp.data()) != 0)
-        throw InitFailure("initial partitioner could not partition the coarsest graph");
-    // the hierarchy's levels and maps on the device
-    std::vector<Level> D(H.size());
-    for (size_t i = 0; i < H.size(); i++) {
-        const jet_init::HostLevel& h = H[i];
-        Level& d = D[i];
+    for (const jet_init::HostLevel& h : H) {
+        Level d;
+        const int64_t nf = D.empty() ? cs.n : D.back().n;
         d.n = h.n;
         d.m = h.xadj[h.n];
         d.rowptr = C.persist.alloc<eoff_t>((int64_t)h.n + 1);
         d.col = C.persist.alloc<vid_t>(std::max<int64_t>(d.m, 1));
         d.ew = C.persist.alloc<wgt_t>(std::max<int64_t>(d.m, 1));
         d.vw = C.persist.alloc<wgt_t>(std::max<int64_t>(h.n, 1));
-        const int64_t nf = i == 0 ? cs.n : H[i - 1].n;
         d.map = C.persist.alloc<vid_t>(std::max<int64_t>(nf, 1));
         d.uniform = false;
         JET_HIP(hipMemcpyAsync(d.rowptr, h.xadj.data(), sizeof(int64_t) * (h.n + 1), hipMemcpyHostToDevice, s));
@@ -451,6 +498,7 @@ static void initial_partition_multilevel(Context& C, const jet_config_t& cfg, co
         }
         JET_HIP(hipMemcpyAsync(d.vw, h.vw.data(), sizeof(int32_t) * h.n, hipMemcpyHostToDevice, s));
         JET_HIP(hipMemcpyAsync(d.map, h.map.data(), sizeof(int32_t) * nf, hipMemcpyHostToDevice, s));
+        D.push_back(d);
     }
     RefineParams rp;
     rp.k = k;
@@ -460,14 +508,15 @@ static void initial_partition_multilevel(Context& C, const jet_config_t& cfg, co
     ArenaScope rscope(C.scratch);
     int64_t cap = conn_capacity(D[0].n, D[0].rowptr, k, C.scratch, s);
     Refiner ref(C.scratch, s, D[0].n, cap, rp);
-    part_t* cur = C.persist.alloc<part_t>(last.n);
-    JET_HIP(hipMemcpyAsync(cur, hp.data(), sizeof(int32_t) * last.n, hipMemcpyHostToDevice, s));
+    part_t* cur = C.persist.alloc<part_t>(D.back().n);
+    JET_HIP(hipMemcpyAsync(cur, hp.data(), sizeof(int32_t) * D.back().n, hipMemcpyHostToDevice, s));
     for (size_t L = D.size(); L-- > 0;) {
         ref.refine(D[L], cur);
-        part_t* fp = L == 0 ? cs_part : C.persist.alloc<part_t>(H[L - 1].n);
-        project(L == 0 ? cs.n : H[L - 1].n, D[L].map, cur, fp, s);
+        part_t* fp = L == 0 ? cs_part : C.persist.alloc<part_t>(D[L - 1].n);
+        project(L == 0 ? cs.n : D[L - 1].n, D[L].map, cur, fp, s);
         cur = fp;
     }
+    JET_HIP(hipStreamSynchronize(s));  // the host arrays above end here
 }
 
 // partitioner.hpp:61-125. part_out: device buffer of fine.n entries.
@@ -534,22 +583,14 @@ static AttemptResult partition_once(Context& C, const jet_config_t& cfg, const L
 
     // initial partition of the coarsest graph on the host
     const Level& cs = levels.back();
-    std::vector<int64_t> h_rp(cs.n + 1);
-    std::vector<int32_t> h_col(cs.m), h_ew(cs.m), h_vw(cs.n), h_part(cs.n);
-    JET_HIP(hipMemcpyAsync(h_rp.data(), cs.rowptr, sizeof(int64_t) * (cs.n + 1), hipMemcpyDeviceToHost, s));
-    if (cs.m > 0) {
-        JET_HIP(hipMemcpyAsync(h_col.data(), cs.col, sizeof(int32_t) * cs.m, hipMemcpyDeviceToHost, s));
-        JET_HIP(hipMemcpyAsync(h_ew.data(), cs.ew, sizeof(int32_t) * cs.m, hipMemcpyDeviceToHost, s));
-    }
-    JET_HIP(hipMemcpyAsync(h_vw.data(), cs.vw, sizeof(int32_t) * cs.n, hipMemcpyDeviceToHost, s));
-    JET_HIP(hipStreamSynchronize(s));
+    std::vector<int32_t> h_part;
     part_t* cur = (levels.size() == 1) ? part_out : C.persist.alloc<part_t>(cs.n);
     if (jet_init::wants_hierarchy(cs.n, cs.m, k)) {
-        initial_partition_multilevel(C, cfg, cs, h_rp, h_col, h_ew, h_vw, seed, cur);
+        initial_partition_multilevel(C, cfg, cs, seed, cur);
     } else {
-        if (jet_host_initpart(cs.n, h_rp.data(), h_col.data(), h_ew.data(), h_vw.data(), k, cfg.max_imb_ratio, seed,
-                              h_part.data()) != 0)
-            throw InitFailure("initial partitioner could not partition the coarsest graph");
+        const HostGraph h = fetch_graph(C, cs);
+        h_part.resize(cs.n);
+        host_initpart(cfg, cs.n, h.rp.data(), h.col.data(), h.ew.data(), h.vw.data(), seed, h_part.data());
         JET_HIP(hipMemcpyAsync(cur, h_part.data(), sizeof(int32_t) * cs.n, hipMemcpyHostToDevice, s));
     }
     JET_HIP(hipStreamSynchronize(s));
