@@ -97,35 +97,45 @@ __device__ inline void conn_sub(int2* tab, int32_t vsz, part_t p, int32_t w, int
     if (vsz < k && x == w) __hip_atomic_store(&tab[po].x, HASH_RECLAIM, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// update_small add (jet_refiner.hpp:815-886).
+// update_small add (jet_refiner.hpp:815-886). Slots are only filled during an
+// addition pass, so a slot read as another part's stays that part's and the
+// first free slot seen is where the insertion starts: slots before it need no
+// second look. FRESH: earlier writes of the same launch may have touched the
+// table (the one-launch kernels), so the search reads past the caches; a pass
+// of its own launch starts from clean caches, and a slot that another
+// workgroup fills meanwhile is at worst seen free, which the compare-and-swap
+// finds out.
+template <bool FRESH = true>
 __device__ inline void conn_add(int2* tab, int32_t* vsize, int32_t cap, part_t best, int32_t w, int32_t* err) {
-    int32_t vsz = ld_rx(vsize);
+    const int32_t vsz = ld_rx(vsize);
     int32_t po = best % vsz;
     bool success = false;
-    // the search for best or an empty slot, four slots per round trip (the
-    // values are those a one-at-a-time probe could read: other threads only
-    // fill empty or reclaimed slots meanwhile)
-    for (int32_t q = 0, s0 = po; q < vsz; q += 4) {
-        int32_t sl[4], e[4];
+    int32_t free_at = -1;
+    constexpr int P = 4;  // slots per round trip
+    for (int32_t q = 0, s0 = po; q < vsz; q += P) {
+        int32_t sl[P], e[P];
         sl[0] = s0;
-        for (int j = 1; j < 4; j++) sl[j] = next_slot(sl[j - 1], vsz);
-        for (int j = 0; j < 4; j++) e[j] = ld_rx(&tab[sl[j]].x);
+        for (int j = 1; j < P; j++) sl[j] = next_slot(sl[j - 1], vsz);
+        for (int j = 0; j < P; j++) e[j] = FRESH ? ld_rx(&tab[sl[j]].x) : tab[sl[j]].x;
         bool stop = false;
-        for (int j = 0; j < 4 && !stop; j++) {
+        for (int j = 0; j < P && !stop; j++) {
             if (q + j >= vsz) {
                 stop = true;
             } else if (e[j] == best) {
                 success = true;
                 po = sl[j];
                 stop = true;
-            } else if (e[j] == NULL_PART) {
-                stop = true;
+            } else if (e[j] <= NULL_PART) {
+                if (free_at < 0) free_at = sl[j];
+                stop = e[j] == NULL_PART;
             }
         }
         if (stop) break;
-        s0 = next_slot(sl[3], vsz);
+        s0 = next_slot(sl[P - 1], vsz);
     }
     int32_t count = 0;
+    if (free_at < 0) count = vsz;  // every slot is another part's
+    else if (!success) po = free_at;
     while (!success && count < vsz) {
         int32_t px = ld_rx(&tab[po].x);
         while (px != best && px > NULL_PART && count++ < vsz) {

@@ -84,6 +84,7 @@ class Refiner {
     LevelRecord refine_wg(const Level& L, part_t* best_part, const std::vector<double>& temps);
     void init_conn(const Level& L, const part_t* part, const int32_t* mark);
     void build_tiers(const Level& L);
+    void build_slices(const Level& L);
     void jet_lp(const Level& L, const part_t* part, double filter_ratio);
     void rebalance(const Level& L, const part_t* part, const int64_t* sizes, bool strong);
     // Bucket layout of one rebalancing step (jet_refiner.hpp:417-428, 551-560).
@@ -159,6 +160,9 @@ class Refiner {
     vid_t* pull_mid_;  // mid-tier rows of degree > BIG_DEG
     int32_t ntier_mid_ = 0, ntier_big_ = 0, npull_mid_ = 0;
     bool has_big_ = false;
+    // rows of more than long_deg_ edges in slices (vertex, slice)
+    int32_t long_deg_ = 0, nslices_ = 0;
+    int2* slices_ = nullptr;
     // small device state; counter set layout: [0] small candidates, [1] big
     // candidates, [2] small moves, [3] big moves, [4] re-draws, [5] ranked
     // bucket members, [6] update_large chosen

@@ -33,6 +33,7 @@ namespace jet {
 
 constexpr int32_t SMALL_DEG = 16;       // rows built by one lane
 constexpr int32_t WAVE_TABLE_MAX = 1024; // rows with capacity <= this built by one wave
+constexpr int64_t SLICE_EDGES = 1024;  // edges of a long moved row that one wave updates
 constexpr int32_t BIG_DEG = 64;         // candidates/moves above this degree use one wave
 constexpr int32_t MAX_K = 8192;
 constexpr int32_t LDS_K = 2048;         // part-size deltas aggregated in LDS up to this k
@@ -147,7 +148,8 @@ __global__ void k_conn_caps(DGraph g, int32_t k, int32_t* caps) {
 // the rows whose update_small changes are pulled (degree > BIG_DEG): big-tier
 // rows and pull_mid rows; hub[] flags both kinds.
 __global__ void __launch_bounds__(256) k_conn_tiers(DGraph g, int32_t k, vid_t* mid, vid_t* big, vid_t* pull_mid,
-                                                    int32_t* cnt, uint8_t* hub, int32_t small_max) {
+                                                    int32_t* cnt, uint8_t* hub, int32_t small_max,
+                                                    int32_t long_deg) {
     __shared__ int32_t sh[256 / WAVE + 1];
     FOR_BLOCK_UNIFORM(i, g.n) {
         const bool in = i < g.n;
@@ -157,12 +159,25 @@ __global__ void __launch_bounds__(256) k_conn_tiers(DGraph g, int32_t k, vid_t* 
         bool is_big = d > SMALL_DEG && !is_mid;
         bool is_pmid = is_mid && d > BIG_DEG;
         if (in) hub[i] = (is_big || is_pmid) ? 1 : 0;
+        if (d > long_deg) atomicAdd(&cnt[4], (int32_t)((d + SLICE_EDGES - 1) / SLICE_EDGES));
         int32_t a = block_append<256>(&cnt[0], is_mid, sh);
         int32_t b = block_append<256>(&cnt[1], is_big, sh);
         int32_t c = block_append<256>(&cnt[3], is_pmid, sh);
         if (a >= 0) mid[a] = (vid_t)i;
         if (b >= 0) big[b] = (vid_t)i;
         if (c >= 0) pull_mid[c] = (vid_t)i;
+    }
+}
+
+// The rows of more than long_deg edges, SLICE_EDGES edges of one row per entry:
+// (vertex, slice). The update passes give each slice of a moved row to a wave.
+__global__ void __launch_bounds__(256) k_row_slices(DGraph g, int32_t long_deg, int2* slices, int32_t* cnt) {
+    FOR_THREAD(i, g.n) {
+        const int64_t d = g.rowptr[i + 1] - g.rowptr[i];
+        if (d <= long_deg) continue;
+        const int32_t c = (int32_t)((d + SLICE_EDGES - 1) / SLICE_EDGES);
+        const int32_t at = atomicAdd(cnt, c);
+        for (int32_t q = 0; q < c; q++) slices[at + q] = make_int2((int32_t)i, q);
     }
 }
 
@@ -822,7 +837,7 @@ __device__ inline void update_edge(vid_t v, int32_t w, part_t pold, part_t pnew,
     } else {
         const eoff_t co = conn_off[v], ce = conn_off[v + 1];
         dest_cache[v] = NULL_PART;
-        conn_add(conn + co, &conn_size[v], (int32_t)(ce - co), pnew, w, err);
+        conn_add<false>(conn + co, &conn_size[v], (int32_t)(ce - co), pnew, w, err);
     }
 }
 
@@ -958,23 +973,23 @@ __global__ void __launch_bounds__(256)
 }
 
 // The same for the moves of degree > BIG_DEG (the back of the list): a wave
-// per move, UB_UNROLL edges per lane in flight; moves of degree > long_deg are
-// queued in LDS and taken by the whole workgroup afterwards, so that one long
-// row does not serialise a wave. (Every move spread over 16 waves, whatever
-// its degree, loaded most moves' records to find no edge left: 525 us a first
-// pass and 508 us a second one on R-MAT 22, bound by those loads.)
+// per move, UB_UNROLL edges per lane in flight. The rows of more than long_deg
+// edges are left to a second loop over the level's row slices (k_row_slices),
+// a wave per slice whose row moves, so that no chain of updates is longer than
+// SLICE_EDGES / 64 edges.
+// A workgroup per long row left chains of hundreds of table updates per lane
+// for the longest ones: on R-MAT 22's level of 756,505 vertices a second pass
+// that moves them took 4.7 ms, with the slices and an insertion that starts at
+// the first free slot seen 2.1 (the level 166 ms, now 130).
 constexpr int UB_BLOCK = 1024;
 constexpr int UB_UNROLL = 4;
-constexpr int UB_QUEUE = 1024;
 template <bool ADD>
 __global__ void __launch_bounds__(UB_BLOCK)
     k_update_big(DGraph g, const vid_t* moves, MoveRec* rec, const int32_t* mc, vid_t nmax, part_t* part,
                  const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
                  int32_t k, int32_t* err, int32_t* mark, const uint8_t* hub, uint8_t* hub_dirty,
                  const int32_t* deferred, const int32_t* stamp, int32_t gen, unsigned long long* sizes,
-                 int64_t* partials, uint32_t* bits, int32_t long_deg) {
-    __shared__ int64_t queue[UB_QUEUE];
-    __shared__ int32_t nqueue;
+                 int64_t* partials, uint32_t* bits, int32_t long_deg, const int2* slices, int32_t nslices) {
     const int lane = threadIdx.x & (WAVE - 1);
     const int wv = threadIdx.x / WAVE;
     constexpr int WAVES = UB_BLOCK / WAVE;
@@ -983,18 +998,16 @@ __global__ void __launch_bounds__(UB_BLOCK)
     if (dfr || nb == 0) return;
     const bool rebuild = ns + nb > g.n / 10;  // jet_refiner.hpp:933
     const bool pull_all = ns + nb > g.n / PULL_ALL_DIV;
-    if (threadIdx.x == 0) nqueue = 0;
-    __syncthreads();
     int64_t cc = 0;
-    auto edges = [&](vid_t v, part_t pold, part_t pnew, eoff_t rs, eoff_t re, int sub, int stride) {
+    auto edges = [&](part_t pold, part_t pnew, eoff_t rs, eoff_t re) {
         // the hub flags of UB_UNROLL edges are loaded together; only the
         // neighbours that are no hubs go on to the table updates
-        for (eoff_t b0 = rs; b0 < re; b0 += (eoff_t)UB_UNROLL * stride) {
+        for (eoff_t b0 = rs; b0 < re; b0 += (eoff_t)UB_UNROLL * WAVE) {
             vid_t u[UB_UNROLL];
             uint8_t h[UB_UNROLL];
 #pragma unroll
             for (int q = 0; q < UB_UNROLL; q++) {
-                const eoff_t j = b0 + (eoff_t)q * stride + sub;
+                const eoff_t j = b0 + (eoff_t)q * WAVE + lane;
                 u[q] = j < re ? g.col[j] : -1;
             }
 #pragma unroll
@@ -1006,64 +1019,45 @@ __global__ void __launch_bounds__(UB_BLOCK)
                     if (!ADD && !pull_all) hub_dirty[u[q]] = 1;
                     continue;
                 }
-                update_edge<ADD>(u[q], g.ew[b0 + (eoff_t)q * stride + sub], pold, pnew, rebuild, part, dest, conn_off,
+                update_edge<ADD>(u[q], g.ew[b0 + (eoff_t)q * WAVE + lane], pold, pnew, rebuild, part, dest, conn_off,
                                  conn, conn_size, dest_cache, k, err, mark, stamp, gen, cc);
             }
         }
     };
-    auto one = [&](int64_t x, bool longs) {
+    // consecutive moves, and consecutive slices of a row, go to different workgroups
+    const int64_t first = (int64_t)wv * gridDim.x + blockIdx.x, stride = (int64_t)gridDim.x * WAVES;
+    for (int64_t x = first; x < nb; x += stride) {
         const int64_t at = nmax - 1 - x;
-        const int sub = longs ? threadIdx.x : lane, stride = longs ? UB_BLOCK : WAVE;
         if (ADD) {
             const MoveRec r = rec[at];
-            if (!longs) {
-                if (lane == 0) {
-                    part[r.v] = r.pnew;
-                    if (bits) bits[r.v >> 5] = 0;
-                }
-                if (rebuild) return;
-                if (r.deg > long_deg) {
-                    int32_t slot = 0;
-                    if (lane == 0) slot = atomicAdd(&nqueue, 1);
-                    slot = __shfl(slot, 0, WAVE);
-                    if (slot < UB_QUEUE) {
-                        if (lane == 0) queue[slot] = x;
-                        return;
-                    }
-                }
+            if (lane == 0) {
+                part[r.v] = r.pnew;
+                if (bits) bits[r.v >> 5] = 0;
             }
-            edges(r.v, 0, r.pnew, r.rs, r.rs + r.deg, sub, stride);
+            if (!rebuild && r.deg <= long_deg) edges(0, r.pnew, r.rs, r.rs + r.deg);
         } else {
             const vid_t i = moves[at];
             const part_t pold = part[i], pnew = dest[i];
             const eoff_t rs = g.rowptr[i], re = g.rowptr[i + 1];
-            if (!longs) {
-                if (lane == 0) {
-                    dest_cache[i] = NULL_PART;
-                    if (bits) atomicOr(&bits[i >> 5], 1u << (i & 31));
-                    rec[at] = MoveRec{rs, (int32_t)(re - rs), i, pnew, 0};
-                    const unsigned long long w = (unsigned long long)g.vw[i];
-                    atomicAdd(&sizes[pold], (unsigned long long)(-(long long)w));
-                    atomicAdd(&sizes[pnew], w);
-                }
-                if (re - rs > long_deg) {
-                    int32_t slot = 0;
-                    if (lane == 0) slot = atomicAdd(&nqueue, 1);
-                    slot = __shfl(slot, 0, WAVE);
-                    if (slot < UB_QUEUE) {
-                        if (lane == 0) queue[slot] = x;
-                        return;
-                    }
-                }
+            if (lane == 0) {
+                dest_cache[i] = NULL_PART;
+                if (bits) atomicOr(&bits[i >> 5], 1u << (i & 31));
+                rec[at] = MoveRec{rs, (int32_t)(re - rs), i, pnew, 0};
+                const unsigned long long w = (unsigned long long)g.vw[i];
+                atomicAdd(&sizes[pold], (unsigned long long)(-(long long)w));
+                atomicAdd(&sizes[pnew], w);
             }
-            edges(i, pold, pnew, rs, re, sub, stride);
+            if (re - rs <= long_deg) edges(pold, pnew, rs, re);
         }
-    };
-    // consecutive moves go to different workgroups, and with them the long ones
-    for (int64_t x = (int64_t)wv * gridDim.x + blockIdx.x; x < nb; x += (int64_t)gridDim.x * WAVES) one(x, false);
-    __syncthreads();
-    const int32_t nq = min(nqueue, UB_QUEUE);
-    for (int32_t q = 0; q < nq; q++) one(queue[q], true);
+    }
+    if (!(ADD && rebuild))
+        for (int64_t x = first; x < nslices; x += stride) {
+            const int2 sl = slices[x];
+            if (stamp[sl.x] != gen) continue;
+            const eoff_t rs = g.rowptr[sl.x] + (eoff_t)sl.y * SLICE_EDGES;
+            const eoff_t re = min(g.rowptr[sl.x + 1], rs + (eoff_t)SLICE_EDGES);
+            edges(ADD ? 0 : part[sl.x], dest[sl.x], rs, re);
+        }
     if (!ADD) {
         cc = wave_reduce_sum(cc);
         if (lane == 0 && cc)
@@ -2259,20 +2253,32 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
 
 void Refiner::build_tiers(const Level& L) {
     DGraph g = L.view();
-    fill_i32(counters_ + 16, 0, 4, s_);
+    fill_i32(counters_ + 16, 0, 8, s_);
     // on small levels every row with edges takes the wave tier: a thread per
     // row walks its edges one after another, a wave inserts them all at once
     small_max_ = g.n <= tuning().small_level_n ? 0 : SMALL_DEG;
+    long_deg_ = (int32_t)(tuning().upd_big_slices * 2 * WAVE);
     k_conn_tiers<<<grid_for(g.n, 256, 8192), 256, 0, s_>>>(g, p_.k, tier_mid_, tier_big_, pull_mid_,
-                                                            counters_ + 16, hub_, small_max_);
+                                                            counters_ + 16, hub_, small_max_, long_deg_);
     k_max_degree<<<grid_for(g.n, 256, 512), 256, 0, s_>>>(g, counters_ + 18);
     JET_LAUNCH_CHECK();
-    int32_t c[4];
-    read_i32_words(counters_ + 16, 4, c, s_);
+    int32_t c[5];
+    read_i32_words(counters_ + 16, 5, c, s_);
     ntier_mid_ = c[0];
     ntier_big_ = c[1];
     has_big_ = c[2] > BIG_DEG;
     npull_mid_ = c[3];
+    nslices_ = c[4];
+}
+
+// The level's row slices, in the caller's scope of the arena.
+void Refiner::build_slices(const Level& L) {
+    slices_ = nullptr;
+    if (nslices_ == 0) return;
+    DGraph g = L.view();
+    slices_ = a_.alloc<int2>(nslices_);
+    k_row_slices<<<grid_for(g.n, 256, 8192), 256, 0, s_>>>(g, long_deg_, slices_, counters_ + 21);
+    JET_LAUNCH_CHECK();
 }
 
 void Refiner::init_conn(const Level& L, const part_t* part, const int32_t* mark) {
@@ -2355,7 +2361,7 @@ void Refiner::jet_lp(const Level& L, const part_t* part, double fr) {
     if (has_big_)
         family_launch(PF_AFTERBURNER, k_afterburner_big, dim3(grid_for((int64_t)g.n * WAVE, AB_WAVES * WAVE, 512)),
                       dim3(AB_WAVES * WAVE), 0, s_, g, cand_, c, part, dest_, pregain_, lock_, moves_, c, nmax_, stamp_,
-                      gen_, (int32_t)(tuning().upd_big_slices * 2 * WAVE));
+                      gen_, long_deg_);
     JET_LAUNCH_CHECK();
 }
 
@@ -2593,10 +2599,10 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
         }
 #undef JET_UPD
         if (has_big_) {
-            const int32_t long_deg = (int32_t)(tuning().upd_big_slices * 2 * WAVE);
             family_launch(PF_UPDATE, add ? k_update_big<true> : k_update_big<false>, dim3(nbb), dim3(UB_BLOCK), 0, s_, g,
                           moves_, mrec_, c, nmax_, part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k,
-                          misc_ + 1, swap_bit_, hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, long_deg);
+                          misc_ + 1, swap_bit_, hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, long_deg_,
+                          slices_, nslices_);
         }
         if (!add && hubs) {
             const int want = std::max(ntier_big_, (int)ceil_div(npull_mid_, ph_waves));
@@ -2695,7 +2701,9 @@ LevelRecord Refiner::refine(const Level& L, part_t* best_part) {
     copy_i64(curr_sizes_, best_sizes_, k, s_);
     const int64_t imb_max = (int64_t)size_max_ - opt_;
     copy_i32(cur_part_, best_part, g.n, s_);
+    ArenaScope level_scope(a_);
     build_tiers(L);
+    build_slices(L);
     init_conn(L, cur_part_, nullptr);
     if (tagged) {
         LevelRecord rec = refine_wg(L, best_part, temps);

@@ -29,9 +29,8 @@ struct Tuning {
     // lanes per move in the update passes: upd_lanes times the level's lane
     // group (from its average degree), at most a wave
     int64_t upd_lanes = 2;
-    // moves and candidates of degree above 128 times this are taken by a whole
-    // workgroup
-    // (of degree above 64 by a wave)
+    // candidates of degree above 128 times this are taken by a whole workgroup,
+    // moves in slices of 1024 edges (of degree above 64 by a wave)
     int64_t upd_big_slices = 16;
     // levels of up to this many vertices run LP select with one pass per wave
     int64_t lp_one_pass_n = 524288;
