@@ -981,6 +981,14 @@ __global__ void __launch_bounds__(256)
 // for the longest ones: on R-MAT 22's level of 756,505 vertices a second pass
 // that moves them took 4.7 ms, with the slices and an insertion that starts at
 // the first free slot seen 2.1 (the level 166 ms, now 130).
+//
+// Bound: chains of table probes. Of a moved row's neighbours a quarter are no
+// hubs, so the edges that do need an update are collected in a queue per wave
+// and taken 64 at a time: lanes without work cost as much as the others. The
+// part-size deltas meet in LDS first: two atomics per move on k addresses were
+// 1.6 ms of a first pass that moves a tenth of 4,194,304 vertices. Averages
+// per pass before and now: first 577 and 235 us there, 233 and 143 at 756,505
+// vertices; second 293 and 184, 444 and 136.
 constexpr int UB_BLOCK = 1024;
 constexpr int UB_UNROLL = 4;
 template <bool ADD>
@@ -989,7 +997,10 @@ __global__ void __launch_bounds__(UB_BLOCK)
                  const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
                  int32_t k, int32_t* err, int32_t* mark, const uint8_t* hub, uint8_t* hub_dirty,
                  const int32_t* deferred, const int32_t* stamp, int32_t gen, unsigned long long* sizes,
-                 int64_t* partials, uint32_t* bits, int32_t long_deg, const int2* slices, int32_t nslices) {
+                 int64_t* partials, uint32_t* bits, int32_t long_deg, const int2* slices, int32_t nslices,
+                 unsigned long long* copies, int32_t ncopies) {
+    __shared__ int4 queues[UB_BLOCK / WAVE][2 * WAVE];
+    __shared__ unsigned long long ls[ADD ? 1 : LDS_K];
     const int lane = threadIdx.x & (WAVE - 1);
     const int wv = threadIdx.x / WAVE;
     constexpr int WAVES = UB_BLOCK / WAVE;
@@ -998,29 +1009,47 @@ __global__ void __launch_bounds__(UB_BLOCK)
     if (dfr || nb == 0) return;
     const bool rebuild = ns + nb > g.n / 10;  // jet_refiner.hpp:933
     const bool pull_all = ns + nb > g.n / PULL_ALL_DIV;
+    const bool lds = !ADD && k <= LDS_K;
+    if (lds) {
+        for (int t = threadIdx.x; t < k; t += UB_BLOCK) ls[t] = 0;
+        __syncthreads();
+    }
     int64_t cc = 0;
+    // the wave's queue of edges to neighbours that are no hubs: (neighbour,
+    // weight, old part, new part)
+    int4* queue = queues[wv];
+    int32_t nq = 0;
+    auto drain = [&](int32_t c) {  // the last c <= WAVE entries
+        wave_sync();
+        nq -= c;
+        if (lane < c) {
+            const int4 e = queue[nq + lane];
+            update_edge<ADD>(e.x, e.y, e.z, e.w, rebuild, part, dest, conn_off, conn, conn_size, dest_cache, k, err,
+                             mark, stamp, gen, cc);
+        }
+        wave_sync();
+    };
     auto edges = [&](part_t pold, part_t pnew, eoff_t rs, eoff_t re) {
-        // the hub flags of UB_UNROLL edges are loaded together; only the
-        // neighbours that are no hubs go on to the table updates
         for (eoff_t b0 = rs; b0 < re; b0 += (eoff_t)UB_UNROLL * WAVE) {
             vid_t u[UB_UNROLL];
             uint8_t h[UB_UNROLL];
+            int32_t w[UB_UNROLL];
 #pragma unroll
             for (int q = 0; q < UB_UNROLL; q++) {
                 const eoff_t j = b0 + (eoff_t)q * WAVE + lane;
                 u[q] = j < re ? g.col[j] : -1;
+                w[q] = j < re ? g.ew[j] : 0;
             }
 #pragma unroll
             for (int q = 0; q < UB_UNROLL; q++) h[q] = u[q] >= 0 && hub ? hub[u[q]] : 0;
 #pragma unroll
             for (int q = 0; q < UB_UNROLL; q++) {
-                if (u[q] < 0) continue;
-                if (h[q]) {
-                    if (!ADD && !pull_all) hub_dirty[u[q]] = 1;
-                    continue;
-                }
-                update_edge<ADD>(u[q], g.ew[b0 + (eoff_t)q * WAVE + lane], pold, pnew, rebuild, part, dest, conn_off,
-                                 conn, conn_size, dest_cache, k, err, mark, stamp, gen, cc);
+                if (!ADD && !pull_all && h[q]) hub_dirty[u[q]] = 1;
+                const bool in = u[q] >= 0 && !h[q];
+                const uint64_t mk = __ballot(in);
+                if (in) queue[nq + (int32_t)__popcll(mk & ((1ull << lane) - 1ull))] = make_int4(u[q], w[q], pold, pnew);
+                nq += (int32_t)__popcll(mk);
+                if (nq >= WAVE) drain(WAVE);
             }
         }
     };
@@ -1044,8 +1073,13 @@ __global__ void __launch_bounds__(UB_BLOCK)
                 if (bits) atomicOr(&bits[i >> 5], 1u << (i & 31));
                 rec[at] = MoveRec{rs, (int32_t)(re - rs), i, pnew, 0};
                 const unsigned long long w = (unsigned long long)g.vw[i];
-                atomicAdd(&sizes[pold], (unsigned long long)(-(long long)w));
-                atomicAdd(&sizes[pnew], w);
+                if (lds) {
+                    atomicAdd(&ls[pold], (unsigned long long)(-(long long)w));
+                    atomicAdd(&ls[pnew], w);
+                } else {
+                    atomicAdd(&sizes[pold], (unsigned long long)(-(long long)w));
+                    atomicAdd(&sizes[pnew], w);
+                }
             }
             if (re - rs <= long_deg) edges(pold, pnew, rs, re);
         }
@@ -1058,11 +1092,18 @@ __global__ void __launch_bounds__(UB_BLOCK)
             const eoff_t re = min(g.rowptr[sl.x + 1], rs + (eoff_t)SLICE_EDGES);
             edges(ADD ? 0 : part[sl.x], dest[sl.x], rs, re);
         }
+    if (nq > 0) drain(nq);
     if (!ADD) {
         cc = wave_reduce_sum(cc);
         if (lane == 0 && cc)
             atomicAdd((unsigned long long*)&partials[(int64_t)(blockIdx.x % PUB_GROUPS) * PUB_STRIDE],
                       (unsigned long long)cc);
+        if (lds) {
+            __syncthreads();
+            unsigned long long* dst = ncopies > 0 ? copies + (int64_t)(blockIdx.x % (uint32_t)ncopies) * k : sizes;
+            for (int t = threadIdx.x; t < k; t += UB_BLOCK)
+                if (ls[t]) atomicAdd(&dst[t], ls[t]);
+        }
     }
 }
 
@@ -1095,7 +1136,9 @@ __global__ void __launch_bounds__(UB_BLOCK)
 // R-MAT 22 (k = 256), averages per step: two scans per step with global
 // tables 1.36 ms in four launches, one scan probing hashed LDS tables 2.4 ms,
 // this kernel 0.32 ms on the levels of up to 438,484 vertices and 0.67 ms
-// above (0.90 ms with the stamps gathered there).
+// above (0.90 ms with the stamps gathered there). Those were with one
+// workgroup of 80 registers a thread on a CU; with the row's state in scalar
+// registers two fit, and the averages are 0.37 and 0.50 ms.
 // Steps that move few vertices scan only the rows that the first pass
 // flagged; from n / PULL_ALL_DIV moves on, about a third of the rows of
 // average degree 190 have a moved neighbour and flagging costs a store per
@@ -1148,7 +1191,7 @@ __device__ inline int32_t ph_store(int2* conn, int32_t cap, int32_t vsz, int32_t
 }
 
 template <bool EXACT>
-__global__ void __launch_bounds__(PH_WAVES_MAX* WAVE)
+__global__ void __launch_bounds__(PH_WAVES_MAX* WAVE, 8)
     k_pull_hubs(DGraph g, const vid_t* big, int32_t nbig, const vid_t* mid, int32_t nmid, const int32_t* mc,
                 const uint32_t* bits, int32_t shift, uint8_t* hub_dirty, const part_t* part,
                 const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
@@ -1160,7 +1203,7 @@ __global__ void __launch_bounds__(PH_WAVES_MAX* WAVE)
     const bool rebuild = nm > g.n / 10;  // jet_refiner.hpp:933
     const bool all = nm > g.n / PULL_ALL_DIV;
     const int lane = threadIdx.x & (WAVE - 1);
-    const int wv = threadIdx.x / WAVE;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);  // the rows' state in scalar registers
     const int nwv = blockDim.x / WAVE;
     const int32_t tw = ph_table_words(k);
     uint32_t* lbits = reinterpret_cast<uint32_t*>(ph_lds + (size_t)nwv * tw);
@@ -1195,12 +1238,15 @@ __global__ void __launch_bounds__(PH_WAVES_MAX* WAVE)
     // lane of the wave) is added to val. Returns whether one was found.
     auto scan = [&](eoff_t rs, eoff_t re, int sub, int stride, part_t pu, part_t nu, int32_t* val, auto&& first) {
         bool any = false;
-        for (eoff_t b0 = rs; b0 < re; b0 += (eoff_t)PH_UNROLL * stride) {
+        const vid_t* col = g.col + rs;
+        const int32_t* ew = g.ew + rs;
+        const uint32_t deg = (uint32_t)(re - rs);
+        for (uint32_t b0 = 0; b0 < deg; b0 += PH_UNROLL * stride) {
             vid_t v[PH_UNROLL];
 #pragma unroll
             for (int q = 0; q < PH_UNROLL; q++) {
-                const eoff_t j = b0 + (eoff_t)q * stride + sub;
-                v[q] = j < re ? g.col[j] : -1;
+                const uint32_t j = b0 + q * stride + sub;
+                v[q] = j < deg ? col[j] : -1;
             }
             uint32_t hits = 0;
 #pragma unroll
@@ -1212,7 +1258,7 @@ __global__ void __launch_bounds__(PH_WAVES_MAX* WAVE)
 #pragma unroll
             for (int q = 0; q < PH_UNROLL; q++) {
                 const bool h = (hits >> q) & 1u;
-                w[q] = h ? g.ew[b0 + (eoff_t)q * stride + sub] : 0;
+                w[q] = h ? ew[b0 + q * stride + sub] : 0;
                 po[q] = h ? part[v[q]] : 0;
                 pn[q] = h ? dest[v[q]] : 0;
             }
@@ -2602,7 +2648,7 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
             family_launch(PF_UPDATE, add ? k_update_big<true> : k_update_big<false>, dim3(nbb), dim3(UB_BLOCK), 0, s_, g,
                           moves_, mrec_, c, nmax_, part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k,
                           misc_ + 1, swap_bit_, hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, long_deg_,
-                          slices_, nslices_);
+                          slices_, nslices_, pb.copies, pb.ncopies);
         }
         if (!add && hubs) {
             const int want = std::max(ntier_big_, (int)ceil_div(npull_mid_, ph_waves));
