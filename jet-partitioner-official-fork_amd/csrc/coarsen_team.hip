@@ -512,7 +512,7 @@ int32_t coarsen_match_team(const DGraph& g, bool uniform, uint64_t seed, int32_t
     TeamSlot slot(P.team);
     P.xcd = slot.xcd();
     k_match_prep<<<1, 256, 0, s>>>(P.ctl);
-    k_match_team<<<8 * P.team, CM_BLOCK, 0, s>>>(P);
+    k_match_team<<<P.team == 1 ? 1 : 8 * P.team, CM_BLOCK, 0, s>>>(P);
     JET_LAUNCH_CHECK();
     if (!wait_mailbox(&out[1], P.seq, s)) return -1;  // no workgroup ran on the wanted XCD
     const int64_t nc = out[0];

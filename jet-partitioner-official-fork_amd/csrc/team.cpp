@@ -20,6 +20,10 @@ TeamSlot::TeamSlot(int32_t team) : team_(team) {
     int dev = 0;
     JET_HIP(hipGetDevice(&dev));
     dev_ = dev & 63;
+    if (team_ <= 1) {  // waits for nobody
+        team_ = 0;
+        return;
+    }
     for (;;) {
         {
             std::lock_guard<std::mutex> lk(g_slot_mu);

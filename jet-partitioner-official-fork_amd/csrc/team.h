@@ -21,7 +21,8 @@ struct TeamCtl {
 // A place for `team` workgroups on an XCD of the device, held while a team
 // kernel runs there: the teams in flight on an XCD never need more CUs than
 // it has, so that every team finds room for all of its workgroups. Waits
-// until one is free.
+// until one is free. A team of one waits for no other workgroup and takes no
+// place.
 class TeamSlot {
   public:
     explicit TeamSlot(int32_t team);

@@ -16,7 +16,8 @@
 // once. The first member waits until every workgroup of the launch has
 // arrived, with a bound, and then starts the team or abandons it (the host
 // then takes the multi-kernel path): nothing waits for a workgroup that might
-// not run, and every later wait is bounded too.
+// not run, and every later wait is bounded too. A team of one is launched as
+// one workgroup, on any XCD.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -50,6 +51,11 @@ __device__ inline int32_t ceil_div_dev(int32_t a, int32_t b) { return (a + b - 1
 // the launch arrived in time).
 __device__ inline int32_t team_start(TeamCtl& C, int32_t xcd, int32_t wanted, int32_t need, int32_t& go, int32_t& size,
                                      int32_t& me) {
+    if (wanted == 1) {  // launched alone, on whichever XCD
+        go = size = 1;
+        me = 0;
+        return TEAM_GO;
+    }
     go = 0;
     const bool here = xcd_id() == xcd;
     int32_t m = wanted;
@@ -88,6 +94,7 @@ struct Team {
     __device__ bool sync() {
         asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // stores and atomics have reached the L2
         __syncthreads();
+        if (size == 1) return *ok != 0;
         if (threadIdx.x == 0) {
             target += (uint32_t)size;
             __hip_atomic_fetch_add(&c->bar, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
