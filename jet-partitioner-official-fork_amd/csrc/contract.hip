@@ -14,6 +14,8 @@
 
 #include <algorithm>
 
+#include "contract_dev.h"
+#include "contract_team.h"
 #include "tuning.h"
 #include "prims.h"
 #include "wave.h"
@@ -30,9 +32,20 @@ constexpr int32_t T2_CAP = 8192;  // workgroup LDS table slots
 // slots (2 fit). One size of 256 threads and 8192 slots left 8 waves a CU.
 constexpr int32_t T2S_MAX = 1024;
 constexpr int32_t T2S_CAP = 2048;
-constexpr int32_t EMPTY = -1;
 
-__device__ inline uint32_t slot_hash(vid_t u) { return (uint32_t)u * 0x9E3779B1u; }
+__global__ void k_contract_reset(vid_t nc, eoff_t* hsize, wgt_t* cvw, int32_t* moff, int32_t* mfill, int32_t* ucount,
+                                 int32_t* cnt) {
+    FOR_THREAD(c, (int64_t)nc + 1) {
+        hsize[c] = 0;
+        moff[c] = 0;
+        ucount[c] = 0;
+        if (c < nc) {
+            cvw[c] = 0;
+            mfill[c] = 0;
+        }
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 4) cnt[threadIdx.x] = 0;
+}
 
 __global__ void k_count(DGraph g, const vid_t* map, eoff_t* hsize, wgt_t* cvw, int32_t* mcount) {
     FOR_THREAD(i, g.n) {
@@ -68,55 +81,6 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Flattened walk over the edges of a coarse row's fine members, in chunks of
-// up to 64 members: lane-strided over edges, member found by binary search on
-// the chunk's degree prefix held in LDS.
-template <class F>
-__device__ inline void wave_row_edges(const DGraph& g, const vid_t* members, int32_t mb, int32_t me, eoff_t* s_ex,
-                                      eoff_t* s_rs, F&& f) {
-    const int lane = threadIdx.x & (WAVE - 1);
-    for (int32_t m0 = mb; m0 < me; m0 += WAVE) {
-        int32_t mi = m0 + lane;
-        bool valid = mi < me;
-        eoff_t rs = 0, d = 0;
-        if (valid) {
-            vid_t i = members[mi];
-            rs = g.rowptr[i];
-            d = g.rowptr[i + 1] - rs;
-        }
-        eoff_t inc = wave_incl_scan(d);
-        eoff_t total = __shfl(inc, WAVE - 1, WAVE);
-        s_ex[lane] = inc - d;
-        s_rs[lane] = rs;
-        int32_t nm = min(WAVE, me - m0);
-        wave_sync();
-        for (eoff_t fi = lane; fi < total; fi += WAVE) {
-            int lo = 0, hi = nm - 1;
-            while (lo < hi) {
-                int mid = (lo + hi + 1) >> 1;
-                if (s_ex[mid] <= fi) lo = mid;
-                else hi = mid - 1;
-            }
-            f(s_rs[lo] + (fi - s_ex[lo]));
-        }
-        wave_sync();
-    }
-}
-
-__device__ inline void lds_insert(int32_t* keys, int32_t* vals, uint32_t mask, vid_t u, wgt_t w) {
-    uint32_t h = slot_hash(u) & mask;
-    while (true) {
-        int32_t k = keys[h];
-        if (k == u) break;
-        if (k == EMPTY) {
-            int32_t old = atomicCAS(&keys[h], EMPTY, u);
-            if (old == EMPTY || old == u) break;
-        }
-        h = (h + 1) & mask;
-    }
-    atomicAdd(&vals[h], w);
-}
-
 constexpr int T1_WAVES = 4;
 
 __global__ void __launch_bounds__(T1_WAVES* WAVE)
@@ -144,7 +108,8 @@ __global__ void __launch_bounds__(T1_WAVES* WAVE)
         wave_sync();
         int32_t* K = keys[w];
         int32_t* V = vals[w];
-        wave_row_edges(g, members, moff[c], moff[c + 1], s_ex[w], s_rs[w], [&](eoff_t j) {
+        auto member = [&](int32_t x) { return members[x]; };
+        wave_row_edges(g, member, moff[c], moff[c + 1], s_ex[w], s_rs[w], [&](eoff_t j) {
             vid_t u = map[g.col[j]];
             if (u != c) lds_insert(K, V, cap - 1, u, g.ew[j]);
         });
@@ -385,6 +350,7 @@ __global__ void k_spill_sizes(const vid_t* list, int32_t n3, const eoff_t* hoff,
 }
 
 void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena& a, hipStream_t s, Level& out) {
+    if (team_contract_fits(g.n, g.m, nc) && contract_team(g, map, nc, persist, a, s, out)) return;
     out.n = nc;
     out.rowptr = persist.alloc<eoff_t>((int64_t)nc + 1);
     out.vw = persist.alloc<wgt_t>(nc);
@@ -396,12 +362,7 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
     vid_t* members = a.alloc<vid_t>(g.n);
     vid_t* lists = a.alloc<vid_t>(4 * (int64_t)nc);
     int32_t* cnt = a.alloc<int32_t>(4);
-    fill_i64(hoff, 0, (int64_t)nc + 1, s);
-    fill_i32(out.vw, 0, nc, s);
-    fill_i32(moff, 0, (int64_t)nc + 1, s);
-    fill_i32(mfill, 0, nc, s);
-    fill_i32(ucount, 0, (int64_t)nc + 1, s);
-    fill_i32(cnt, 0, 4, s);
+    k_contract_reset<<<grid_for((int64_t)nc + 1, 256, 8192), 256, 0, s>>>(nc, hoff, out.vw, moff, mfill, ucount, cnt);
     int nb = grid_for(g.n, 256, 8192);
     k_count<<<nb, 256, 0, s>>>(g, map, hoff, out.vw, moff);
     JET_LAUNCH_CHECK();

@@ -550,7 +550,6 @@ static AttemptResult partition_once(Context& C, const jet_config_t& cfg, const L
         auto tm = clk::now();
         vid_t* map = C.persist.alloc<vid_t>(cur.n);
         int32_t nc = coarsen_level(cur, alg, seed, (int32_t)levels.size() - 1, map, C.scratch, s);
-        JET_HIP(hipStreamSynchronize(s));
         auto tb = clk::now();
         R.t_map += secs(tm, tb);
         if (nc < min_allowed) break;
@@ -573,7 +572,6 @@ static AttemptResult partition_once(Context& C, const jet_config_t& cfg, const L
         contract(cur.view(), map, nc, C.persist, C.scratch, s, next);
         next.map = map;
         next.uniform = false;
-        JET_HIP(hipStreamSynchronize(s));
         R.t_build += secs(tb, clk::now());
         levels.push_back(next);
         if (levels.size() > 200) break;
