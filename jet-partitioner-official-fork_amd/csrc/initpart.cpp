@@ -230,21 +230,51 @@ struct GainQueue {
     void clear() { q = std::priority_queue<E>(); }
 };
 
+// The same queue for dense graphs, by one key per vertex: a neighbour's new
+// gain is a store instead of a heap push, and the best vertex is found by
+// looking at all n keys. (The lazy heap holds an entry per edge of a pass:
+// 868 vertices and 251,424 entries split 64 ways on 8 threads took 35 ms, with
+// the table 13; 512 vertices and 6968 entries 2.3 and 1.2.)
+struct KeyTable {
+    static constexpr int64_t OUT = INT64_MIN;  // not in the queue
+    std::vector<int64_t> key;
+    void reset(int32_t n) { key.assign(n, OUT); }
+    int32_t best() const { return argmax(key.data(), (int32_t)key.size()); }
+
+  private:
+    // first index of the largest key, -1 when all are OUT
+    __attribute__((target_clones("avx2", "default"))) static int32_t argmax(const int64_t* k, int32_t n) {
+        int64_t m = OUT;
+        for (int32_t v = 0; v < n; v++) m = k[v] > m ? k[v] : m;
+        if (m == OUT) return -1;
+        int32_t v = 0;
+        while (k[v] != m) v++;
+        return v;
+    }
+};
+
+// Average degree of n / DENSE_DIV or more: KeyTable, else GainQueue. An edge's
+// heap push and removal take about 50 ns, a vertex's share of a search of the
+// keys less than 1 ns.
+constexpr int64_t DENSE_DIV = 32;
+
 struct Bisector {
     const Sub& s;
     std::vector<int8_t> side;
-    std::vector<int64_t> ext, inn;  // edge weight to the other side / same side
+    std::vector<int64_t> gain, tot;  // edge weight to the other side less that to the same side; and their sum
     int64_t w[2] = {0, 0};
     int64_t cut = 0;
 
     explicit Bisector(const Sub& sub) : s(sub) {}
 
-    // ext, inn, side weights and cut from `side`, on up to par threads (each
+    bool dense() const { return (int64_t)s.adj.size() * DENSE_DIV >= (int64_t)s.n * s.n; }
+
+    // gain, tot, side weights and cut from `side`, on up to par threads (each
     // vertex's sums are its own; the totals are integer sums).
     void compute(int par = 1) {
         int32_t n = s.n;
-        ext.resize(n);
-        inn.resize(n);
+        gain.resize(n);
+        tot.resize(n);
         const int T = pass_threads(s, par);
         const std::vector<int32_t> bounds = vertex_chunks(s, T);
         std::vector<int64_t> part_w(2 * T, 0), part_cut(T, 0);
@@ -258,8 +288,8 @@ struct Bisector {
                     if (side[s.adj[j]] != sv) e += s.adjw[j];
                     else i += s.adjw[j];
                 }
-                ext[v] = e;
-                inn[v] = i;
+                gain[v] = e - i;
+                tot[v] = e + i;
                 c += e;
             }
             part_w[2 * t] = w0;
@@ -281,18 +311,11 @@ struct Bisector {
         side[v] = to;
         w[from] -= s.vw[v];
         w[to] += s.vw[v];
-        cut -= ext[v] - inn[v];
-        std::swap(ext[v], inn[v]);
+        cut -= gain[v];
+        gain[v] = -gain[v];
         for (int64_t j = s.xadj[v]; j < s.xadj[v + 1]; j++) {
             int32_t u = s.adj[j];
-            int64_t ew = s.adjw[j];
-            if (side[u] == to) {
-                ext[u] -= ew;
-                inn[u] += ew;
-            } else {
-                ext[u] += ew;
-                inn[u] -= ew;
-            }
+            gain[u] += side[u] == to ? -2 * (int64_t)s.adjw[j] : 2 * (int64_t)s.adjw[j];
         }
     }
 
@@ -303,20 +326,27 @@ struct Bisector {
         compute();
         std::vector<uint8_t> tried(n, 0);
         GainQueue pq;
+        KeyTable keys;
+        const bool table = dense();
+        if (table) keys.reset(n);
         auto push_nb = [&](int32_t v) {
             for (int64_t j = s.xadj[v]; j < s.xadj[v + 1]; j++) {
                 int32_t u = s.adj[j];
-                if (side[u] == 1 && !tried[u]) pq.push(ext[u] - inn[u], u);
+                if (side[u] != 1 || tried[u]) continue;
+                if (table) keys.key[u] = gain[u];
+                else pq.push(gain[u], u);
             }
         };
         int32_t next_free = 0;
         int32_t cur = seed;
         while (w[0] < target0) {
-            if (cur < 0) {
+            if (cur < 0 && table) {
+                cur = keys.best();
+            } else if (cur < 0) {
                 while (!pq.q.empty()) {
                     auto e = pq.q.top();
                     pq.q.pop();
-                    if (side[e.v] != 1 || tried[e.v] || e.g != ext[e.v] - inn[e.v]) continue;
+                    if (side[e.v] != 1 || tried[e.v] || e.g != gain[e.v]) continue;
                     cur = e.v;
                     break;
                 }
@@ -327,6 +357,7 @@ struct Bisector {
                 cur = next_free;
             }
             tried[cur] = 1;
+            if (table) keys.key[cur] = KeyTable::OUT;
             if ((double)(w[0] + s.vw[cur]) <= maxw0 || w[0] == 0) {
                 move(cur);
                 push_nb(cur);
@@ -341,11 +372,18 @@ struct Bisector {
         int32_t n = s.n;
         std::vector<uint8_t> locked(n);
         std::vector<int32_t> moved;
+        KeyTable keys[2];
+        const bool table = dense();
         for (int pass = 0; pass < passes; pass++) {
             std::fill(locked.begin(), locked.end(), 0);
             GainQueue pq[2];
+            for (int t = 0; table && t < 2; t++) keys[t].reset(n);
+            auto push = [&](int32_t v) {
+                if (table) keys[side[v]].key[v] = gain[v];
+                else pq[side[v]].push(gain[v], v);
+            };
             for (int32_t v = 0; v < n; v++)
-                if (ext[v] > 0 || w[side[v]] > maxw[side[v]]) pq[side[v]].push(ext[v] - inn[v], v);
+                if (gain[v] > -tot[v] || w[side[v]] > maxw[side[v]]) push(v);
             auto over = [&]() {
                 double o = 0;
                 for (int t = 0; t < 2; t++)
@@ -363,9 +401,10 @@ struct Bisector {
                 int from = -1;
                 int32_t pick[2] = {-1, -1};
                 for (int t = 0; t < 2; t++) {
+                    if (table) pick[t] = keys[t].best();
                     while (!pq[t].q.empty()) {
                         auto e = pq[t].q.top();
-                        if (locked[e.v] || side[e.v] != t || e.g != ext[e.v] - inn[e.v]) {
+                        if (locked[e.v] || side[e.v] != t || e.g != gain[e.v]) {
                             pq[t].q.pop();
                             continue;
                         }
@@ -383,20 +422,28 @@ struct Bisector {
                         ok[t] = pick[t] >= 0 && (double)(w[1 - t] + s.vw[pick[t]]) <= maxw[1 - t];
                     if (!ok[0] && !ok[1]) break;
                     if (ok[0] && ok[1]) {
-                        int64_t g0 = ext[pick[0]] - inn[pick[0]], g1 = ext[pick[1]] - inn[pick[1]];
+                        int64_t g0 = gain[pick[0]], g1 = gain[pick[1]];
                         from = (g0 > g1 || (g0 == g1 && w[0] >= w[1])) ? 0 : 1;
                     } else {
                         from = ok[0] ? 0 : 1;
                     }
                 }
                 int32_t v = pick[from];
-                pq[from].q.pop();
+                if (table) keys[from].key[v] = KeyTable::OUT;
+                else pq[from].q.pop();
                 locked[v] = 1;
                 move(v);
                 moved.push_back(v);
-                for (int64_t j = s.xadj[v]; j < s.xadj[v + 1]; j++) {
-                    int32_t u = s.adj[j];
-                    if (!locked[u]) pq[side[u]].push(ext[u] - inn[u], u);
+                if (table) {
+                    for (int64_t j = s.xadj[v]; j < s.xadj[v + 1]; j++) {
+                        int32_t u = s.adj[j];
+                        keys[side[u]].key[u] = locked[u] ? KeyTable::OUT : gain[u];
+                    }
+                } else {
+                    for (int64_t j = s.xadj[v]; j < s.xadj[v + 1]; j++) {
+                        int32_t u = s.adj[j];
+                        if (!locked[u]) push(u);
+                    }
                 }
                 double o = over();
                 if (o < best_over || (o == best_over && cut < best_cut)) {
@@ -665,12 +712,11 @@ static Sub coarsen_once(const Sub& s, uint64_t seed, int par, std::vector<int32_
             int32_t best = -1;
             int64_t bw = -1;
             for (int64_t j = s.xadj[v]; j < s.xadj[v + 1]; j++) {
+                if ((int64_t)s.adjw[j] <= bw) continue;  // the edges' own array first
                 int32_t u = s.adj[j];
                 if (u == v || mate[u] >= 0 || (int64_t)s.vw[v] + s.vw[u] > cap) continue;
-                if ((int64_t)s.adjw[j] > bw) {
-                    bw = s.adjw[j];
-                    best = u;
-                }
+                bw = s.adjw[j];
+                best = u;
             }
             if (best >= 0) {
                 mate[v] = best;
@@ -707,49 +753,49 @@ static Sub coarsen_once(const Sub& s, uint64_t seed, int par, std::vector<int32_
         }
         for (; t < T; t++) bounds[t] = nc;
     }
-    // pass 1 counts each coarse row's distinct neighbours, pass 2 writes the
-    // rows at their final offsets; a row's entries keep first-seen order
+    // each chunk's rows are built in its own arrays and then put at their
+    // final offsets; a row's entries keep first-seen order
     std::vector<int64_t> rowlen(nc, 0);
-    auto pass = [&](int t, bool write) {
+    std::vector<BigVec<int32_t>> cadj(T), cadjw(T);
+    auto build = [&](int t) {
+        int64_t most = 0;
+        for (int32_t cv = bounds[t]; cv < bounds[t + 1]; cv++)
+            for (int32_t v : {first[cv], second[cv]})
+                if (v >= 0) most += s.xadj[v + 1] - s.xadj[v];
+        BigVec<int32_t>&adj = cadj[t], &adjw = cadjw[t];
+        adj.resize(most);
+        adjw.resize(most);
         std::vector<int64_t> slot(nc, -1);  // position of cu in the current row, if added there
+        int64_t at = 0;
         for (int32_t cv = bounds[t]; cv < bounds[t + 1]; cv++) {
-            const int64_t row0 = write ? c.xadj[cv] : 0;
-            int64_t len = 0;
-            int64_t tag = write ? row0 : -2 - (int64_t)cv;  // count pass: slot holds -2 - row id
+            const int64_t row0 = at;
             for (int32_t v : {first[cv], second[cv]}) {
                 if (v < 0) continue;
                 for (int64_t j = s.xadj[v]; j < s.xadj[v + 1]; j++) {
                     int32_t cu = cmap[s.adj[j]];
                     if (cu == cv) continue;
-                    if (write) {
-                        if (slot[cu] < row0) {
-                            slot[cu] = row0 + len++;
-                            c.adj[slot[cu]] = cu;
-                            c.adjw[slot[cu]] = s.adjw[j];
-                        } else {
-                            c.adjw[slot[cu]] += s.adjw[j];
-                        }
-                    } else if (slot[cu] != tag) {
-                        slot[cu] = tag;
-                        len++;
+                    if (slot[cu] < row0) {
+                        slot[cu] = at;
+                        adj[at] = cu;
+                        adjw[at++] = s.adjw[j];
+                    } else {
+                        adjw[slot[cu]] += s.adjw[j];
                     }
                 }
             }
-            if (!write) rowlen[cv] = len;
+            rowlen[cv] = at - row0;
         }
     };
-    auto run_all = [&](bool write) {
-        std::vector<std::thread> th;
-        for (int t = 1; t < T; t++) th.emplace_back(pass, t, write);
-        pass(0, write);
-        for (auto& x : th) x.join();
-    };
-    run_all(false);
+    run_threads(T, build);
     c.xadj.assign(nc + 1, 0);
     for (int32_t cv = 0; cv < nc; cv++) c.xadj[cv + 1] = c.xadj[cv] + rowlen[cv];
     c.adj.resize(c.xadj[nc]);
     c.adjw.resize(c.xadj[nc]);
-    run_all(true);
+    run_threads(T, [&](int t) {
+        const int64_t o = c.xadj[bounds[t]], len = c.xadj[bounds[t + 1]] - o;
+        std::copy_n(cadj[t].begin(), len, c.adj.begin() + o);
+        std::copy_n(cadjw[t].begin(), len, c.adjw.begin() + o);
+    });
     return c;
 }
 
