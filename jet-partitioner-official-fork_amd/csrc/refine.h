@@ -159,7 +159,7 @@ class Refiner {
     BestCopy take_best_copy();
     vid_t* pull_mid_;  // mid-tier rows of degree > BIG_DEG
     int32_t ntier_mid_ = 0, ntier_big_ = 0, npull_mid_ = 0;
-    bool has_big_ = false;
+    bool has_big_ = false, has_long_ = false;  // rows above BIG_DEG edges, tables above SEL_LONG slots
     // rows of more than long_deg_ edges in slices (vertex, slice)
     int32_t long_deg_ = 0, nslices_ = 0;
     int2* slices_ = nullptr;

@@ -389,6 +389,62 @@ __global__ void __launch_bounds__(BB_BLOCK)
 }
 
 // ---------------------------------------------------------------- jet_lp
+// A table of more than SEL_LONG slots is read by the whole wave in the select
+// kernels, one after another of its lanes' long tables: a lane that reads 256
+// slots alone takes 64 dependent trips to memory, for which its wave waits.
+// That pays where the waves wait for memory anyway: R-MAT 22 (k = 256), LP
+// select 1.06 -> 0.86 ms on 4,194,304 vertices, 0.49 -> 0.31 on 756,505 and
+// 0.19 -> 0.15 on 438,484, but 98 -> 141 us on 370,878; strong select 0.90 ->
+// 0.37, 0.15 -> 0.10, 0.08 -> 0.06 ms and 70 -> 82 us. The weak select's four
+// vertices a lane hide the trips as they are (0.15 -> 0.20 ms on 756,505).
+constexpr int32_t SEL_LONG = 16;
+constexpr int64_t SEL_LONG_N = 400000;
+
+// Calls f(lane's row broadcast) for each lane with `mine` set, the whole wave
+// together: f(b) gets the lane's number.
+template <class F>
+__device__ inline void for_long_rows(bool mine, F&& f) {
+    uint64_t mk = __ballot(mine);
+    while (mk) {
+        const int b = __ffsll((unsigned long long)mk) - 1;
+        mk &= mk - 1;
+        f(b);
+    }
+}
+
+__device__ inline uint64_t wave_reduce_max_u64(uint64_t x) {
+    for (int d = WAVE / 2; d >= 1; d >>= 1) {
+        const uint32_t lo = __shfl_xor((uint32_t)x, d, WAVE);
+        const uint32_t hi = __shfl_xor((uint32_t)(x >> 32), d, WAVE);
+        const uint64_t y = ((uint64_t)hi << 32) | lo;
+        x = y > x ? y : x;
+    }
+    return x;
+}
+
+// The slot of largest positive connectivity among those ok() accepts (ties:
+// smaller part id) and part p's connectivity, by a wave; `none` when no slot
+// qualifies.
+template <class OK>
+__device__ inline void wave_best_slot(const int2* tab, int32_t sz, part_t p, part_t none, OK&& ok, part_t& best,
+                                      int32_t& gain, int32_t& p_gain) {
+    const int lane = threadIdx.x & (WAVE - 1);
+    uint64_t key = 0;
+    int32_t pg = 0;
+    for (int32_t s = lane; s < sz; s += WAVE) {
+        const int2 e = tab[s];
+        if (e.y > 0 && ok(e)) {
+            const uint64_t x = ((uint64_t)(uint32_t)e.y << 32) | (uint32_t)~e.x;
+            key = x > key ? x : key;
+        }
+        if (e.x == p) pg = e.y;
+    }
+    key = wave_reduce_max_u64(key);
+    gain = (int32_t)(key >> 32);
+    best = gain > 0 ? (part_t)~(uint32_t)key : none;
+    p_gain = wave_reduce_sum(pg);
+}
+
 // jet_refiner.hpp:211-268: destination selection, viable-move filter.
 // Each wave owns a contiguous chunk of CHW vertices (CHW / WAVE passes);
 // candidates are staged in LDS and published with one atomic per workgroup
@@ -404,7 +460,7 @@ constexpr int LS_WAVES = 8;
 constexpr int LS_MULTI_CHW = 128;
 constexpr int LS_MULTI_WAVES = 16;
 
-template <int CHW, int W>
+template <int CHW, int W, bool LONG>
 __global__ void __launch_bounds__(W* WAVE)
     k_lp_select(DGraph g, const part_t* part, const eoff_t* conn_off, const int2* conn, const int32_t* conn_size,
                 part_t* dest_cache, int32_t* gain_p, int32_t* lock, double fr, part_t* dest, int32_t* pregain,
@@ -454,25 +510,41 @@ __global__ void __launch_bounds__(W* WAVE)
         nm += (int32_t)__popcll(mk);
     }
     wave_sync();
-    for (int32_t m = lane; m < nm; m += WAVE) {
-        const int32_t slot = mslot[wv][m];
+    for (int32_t m0 = 0; m0 < nm; m0 += WAVE) {
+        const bool in = m0 + lane < nm;
+        const int32_t slot = in ? mslot[wv][m0 + lane] : 0;
         const int64_t i = wbase + slot;
-        const part_t p = part[i];
+        const part_t p = in ? part[i] : 0;
         part_t best = NO_MOVE;
         int32_t b_conn = 0, p_conn = 0;
-        const int32_t sz = conn_size[i];
-        n_miss++;
+        const int32_t sz = in ? conn_size[i] : 0;
+        const eoff_t off = in ? conn_off[i] : 0;
+        n_miss += in;
         n_slot += sz;
-        for_slots(conn + conn_off[i], sz, [&](int2 e) {
-            if (e.y > b_conn && e.x != p) {
-                best = e.x;
-                b_conn = e.y;
-            } else if (e.y == b_conn && b_conn > 0 && e.x != p && e.x < best) {
-                best = e.x;
-            } else if (e.y > 0 && e.x == p) {
-                p_conn = e.y;
+        if (!LONG || sz <= SEL_LONG)
+            for_slots(conn + off, sz, [&](int2 e) {
+                if (e.y > b_conn && e.x != p) {
+                    best = e.x;
+                    b_conn = e.y;
+                } else if (e.y == b_conn && b_conn > 0 && e.x != p && e.x < best) {
+                    best = e.x;
+                } else if (e.y > 0 && e.x == p) {
+                    p_conn = e.y;
+                }
+            });
+        for_long_rows(LONG && sz > SEL_LONG, [&](int b) {
+            const part_t bp = __shfl(p, b, WAVE);
+            part_t x;
+            int32_t gx, px;
+            wave_best_slot(conn + (eoff_t)__shfl((int64_t)off, b, WAVE), __shfl(sz, b, WAVE), bp, NO_MOVE,
+                           [&](int2 e) { return e.x != bp; }, x, gx, px);
+            if (lane == b) {
+                best = x;
+                b_conn = gx;
+                p_conn = px;
             }
         });
+        if (!in) continue;
         int32_t gsv = 0;
         if (best != NO_MOVE) {
             if (b_conn >= p_conn || ((double)(p_conn - b_conn) < floor(fr * (double)p_conn))) gsv = b_conn - p_conn;
@@ -1572,7 +1644,7 @@ __global__ void __launch_bounds__(SEL_BLOCK_MAX)
 }
 
 // jet_refiner.hpp:449-481.
-template <bool LDS>
+template <bool LDS, bool LONG>
 __global__ void __launch_bounds__(SEL_BLOCK_MAX)
     k_strong_select(DGraph g, const part_t* part, const int64_t* sizes, int32_t k, int64_t size_max, int32_t opt,
                     int64_t max_dest, const int64_t* acc, const eoff_t* conn_off, const int2* conn,
@@ -1590,20 +1662,52 @@ __global__ void __launch_bounds__(SEL_BLOCK_MAX)
     BucketMap bm{bk, bv};
     bm.init();
     const int64_t max_vwgt = acc[3];
-    FOR_BLOCK_RANGE(i, g.n) {
-        const part_t p = part[i];
-        if (bc.part_out) bc.part_out[i] = p;
+    // every lane of a wave takes part in each pass (long tables are shared)
+    const int lane = threadIdx.x & (WAVE - 1);
+    const int64_t per_block = ((g.n + gridDim.x - 1) / gridDim.x + blockDim.x - 1) / blockDim.x * blockDim.x;
+    const int64_t lo = (int64_t)blockIdx.x * per_block;
+    const int64_t hi = min((int64_t)g.n, lo + per_block);
+    for (int64_t b0 = lo; b0 < hi; b0 += blockDim.x) {
+        const int64_t i = b0 + threadIdx.x;
+        const bool in = i < hi;
+        const part_t p = in ? part[i] : 0;
+        if (bc.part_out && in) bc.part_out[i] = p;
         int32_t b = -1;
         const int64_t sp = ps[p];
-        const bool over = sp > size_max;
+        const bool over = in && sp > size_max;
         const int64_t w = over ? g.vw[i] : 0;
         const eoff_t off = over ? conn_off[i] : 0;
         const int32_t sz = over ? conn_size[i] : 0;
         bool vw_ok = max_vwgt > 0 && w <= 2 * max_vwgt;
-        if (over && vw_ok && w < 2 * (sp - opt)) {
-            uint64_t tk = 0, tg = 0;
-            int64_t p_gain = 0;
-            for_slots(conn + off, sz, [&](int2 e) {
+        const bool ev = over && vw_ok && w < 2 * (sp - opt);
+        const bool lng = LONG && ev && sz > SEL_LONG;
+        uint64_t tk = 0, tg = 0;
+        int64_t p_gain = 0;
+        for_long_rows(lng, [&](int q) {
+            const part_t qp = __shfl(p, q, WAVE);
+            const int2* tab = conn + (eoff_t)__shfl((int64_t)off, q, WAVE);
+            const int32_t qs = __shfl(sz, q, WAVE);
+            int64_t x = 0, c = 0, px = 0;
+            for (int32_t s = lane; s < qs; s += WAVE) {
+                const int2 e = tab[s];
+                if (e.x == qp) {
+                    px = e.y;
+                } else if (e.x > NULL_PART && ps[e.x] < max_dest) {
+                    x += e.y;
+                    c++;
+                }
+            }
+            x = wave_reduce_sum(x);
+            c = wave_reduce_sum(c);
+            px = wave_reduce_sum(px);
+            if (lane == q) {
+                tg = (uint64_t)x;
+                tk = (uint64_t)c;
+                p_gain = px;
+            }
+        });
+        if (ev) {
+            if (!lng) for_slots(conn + off, sz, [&](int2 e) {
                 if (e.x == p) {
                     p_gain = e.y;
                 } else if (e.x > NULL_PART && ps[e.x] < max_dest) {
@@ -1620,7 +1724,7 @@ __global__ void __launch_bounds__(SEL_BLOCK_MAX)
                 bm.add(b, (unsigned long long)w, buckets);
             }
         }
-        bid[i] = b;
+        if (in) bid[i] = b;
     }
     bm.flush(buckets);
 }
@@ -2313,6 +2417,7 @@ void Refiner::build_tiers(const Level& L) {
     ntier_mid_ = c[0];
     ntier_big_ = c[1];
     has_big_ = c[2] > BIG_DEG;
+    has_long_ = c[2] > SEL_LONG && p_.k > SEL_LONG && g.n > SEL_LONG_N;
     npull_mid_ = c[3];
     nslices_ = c[4];
 }
@@ -2375,13 +2480,15 @@ void Refiner::jet_lp(const Level& L, const part_t* part, double fr) {
     // passes per wave in 16-wave workgroups above that (see LS_MULTI_CHW)
     if (g.n <= tuning().lp_one_pass_n) {
         int nb = (int)std::max<int64_t>(1, ceil_div(g.n, (int64_t)LS_WAVES * WAVE));
-        family_launch(PF_LP_SELECT, k_lp_select<WAVE, LS_WAVES>, dim3(nb), dim3(LS_WAVES * WAVE), 0, s_, g, part,
+        family_launch(PF_LP_SELECT, k_lp_select<WAVE, LS_WAVES, false>, dim3(nb), dim3(LS_WAVES * WAVE), 0, s_, g, part,
                       conn_off_, conn_, conn_size_, dest_cache_, gain_p_, lock_, fr, dest_, pregain_, cand_, c, nmax_,
                       cnt_next(), prof_counters(PF_LP_SELECT), bcp);
     } else {
         int nb = (int)std::max<int64_t>(1, ceil_div(g.n, (int64_t)LS_MULTI_WAVES * LS_MULTI_CHW));
-        family_launch(PF_LP_SELECT, k_lp_select<LS_MULTI_CHW, LS_MULTI_WAVES>, dim3(nb), dim3(LS_MULTI_WAVES * WAVE),
-                      0, s_, g, part, conn_off_, conn_, conn_size_, dest_cache_, gain_p_, lock_, fr, dest_, pregain_,
+        family_launch(PF_LP_SELECT,
+                      has_long_ ? k_lp_select<LS_MULTI_CHW, LS_MULTI_WAVES, true>
+                                : k_lp_select<LS_MULTI_CHW, LS_MULTI_WAVES, false>,
+                      dim3(nb), dim3(LS_MULTI_WAVES * WAVE), 0, s_, g, part, conn_off_, conn_, conn_size_, dest_cache_, gain_p_, lock_, fr, dest_, pregain_,
                       cand_, c, nmax_, cnt_next(), prof_counters(PF_LP_SELECT), bcp);
     }
     JET_LAUNCH_CHECK();
@@ -2541,11 +2648,11 @@ void Refiner::rebalance(const Level& L, const part_t* part, const int64_t* sizes
     const int selb = g.n > tuning().small_level_n ? SEL_BLOCK_MAX : 128;
     if (strong) {
         if (lds)
-            k_strong_select<true><<<nsel, selb, 0, s_>>>(g, part, sizes, k, smax, opt_, max_dest, acc_, conn_off_,
+            (has_long_ ? k_strong_select<true, true> : k_strong_select<true, false>)<<<nsel, selb, 0, s_>>>(g, part, sizes, k, smax, opt_, max_dest, acc_, conn_off_,
                                                          conn_, conn_size_, sections, bid_, bk, bc, copies, nbuckets_,
                                                          cnt_next(), bcp);
         else
-            k_strong_select<false><<<nsel, selb, 0, s_>>>(g, part, sizes, k, smax, opt_, max_dest, acc_, conn_off_,
+            (has_long_ ? k_strong_select<false, true> : k_strong_select<false, false>)<<<nsel, selb, 0, s_>>>(g, part, sizes, k, smax, opt_, max_dest, acc_, conn_off_,
                                                           conn_, conn_size_, sections, bid_, bk, bc, copies, nbuckets_,
                                                           cnt_next(), bcp);
     } else {
