@@ -146,6 +146,7 @@ class Refiner {
     uint8_t* hub_;
     uint8_t* hub_dirty_;
     uint32_t* moved_bits_;
+    uint64_t* cand_bits_;  // levels with rows above BIG_DEG: a bit per LP candidate
     // stamp_[v] == gen_: v is in the current step's move list (the move-list
     // producers write it; every selection step takes a new generation)
     int32_t* stamp_;
@@ -160,6 +161,7 @@ class Refiner {
     vid_t* pull_mid_;  // mid-tier rows of degree > BIG_DEG
     int32_t ntier_mid_ = 0, ntier_big_ = 0, npull_mid_ = 0;
     bool has_big_ = false, has_long_ = false;  // rows above BIG_DEG edges, tables above SEL_LONG slots
+    double avg_ = 0;  // average degree (with rows above BIG_DEG edges: of the rows of 1 to BIG_DEG edges)
     // rows of more than long_deg_ edges in slices (vertex, slice)
     int32_t long_deg_ = 0, nslices_ = 0;
     int2* slices_ = nullptr;

@@ -273,6 +273,29 @@ __device__ inline void lds_table_add(int2* T, int32_t cap, int32_t k, part_t p, 
     atomicAdd(&T[po].y, w);
 }
 
+// The edges rs + sub + q * stride of a row by this thread, CB_UNROLL of their
+// parts in flight.
+constexpr int CB_UNROLL = 4;
+__device__ inline void table_add_row(int2* T, int32_t cap, int32_t k, const DGraph& g, eoff_t rs, eoff_t re, int sub,
+                                     int stride, const part_t* part, int32_t* used) {
+    for (eoff_t b0 = rs + sub; b0 < re; b0 += (eoff_t)CB_UNROLL * stride) {
+        vid_t v[CB_UNROLL];
+        int32_t w[CB_UNROLL];
+        part_t p[CB_UNROLL];
+#pragma unroll
+        for (int q = 0; q < CB_UNROLL; q++) {
+            const eoff_t j = b0 + (eoff_t)q * stride;
+            v[q] = j < re ? g.col[j] : -1;
+            w[q] = j < re ? g.ew[j] : 0;
+        }
+#pragma unroll
+        for (int q = 0; q < CB_UNROLL; q++) p[q] = v[q] >= 0 ? part[v[q]] : 0;
+#pragma unroll
+        for (int q = 0; q < CB_UNROLL; q++)
+            if (v[q] >= 0) lds_table_add(T, cap, k, p[q], w[q], used);
+    }
+}
+
 // Re-inserts the entries of T (cap slots) into T2 (size slots, linear probing).
 __device__ inline void lds_table_shrink(const int2* T, int32_t cap, int2* T2, int32_t size, int start, int stride) {
     for (int32_t s = start; s < cap; s += stride) {
@@ -300,7 +323,7 @@ __global__ void __launch_bounds__(WB_WAVES* WAVE)
     extern __shared__ int2 tabs[];
     __shared__ int32_t used[WB_WAVES];
     const int lane = threadIdx.x & (WAVE - 1);
-    const int w = threadIdx.x / WAVE;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);
     const int32_t tcap = k < WAVE_TABLE_MAX ? k : WAVE_TABLE_MAX;
     int2* Tw = tabs + (size_t)(2 * w) * tcap;
     int2* T2w = Tw + tcap;
@@ -318,7 +341,7 @@ __global__ void __launch_bounds__(WB_WAVES* WAVE)
         }
         if (lane == 0) used[w] = 0;
         wave_sync();
-        for (eoff_t j = rs + lane; j < re; j += WAVE) lds_table_add(Tw, cap, k, part[g.col[j]], g.ew[j], &used[w]);
+        table_add_row(Tw, cap, k, g, rs, re, lane, WAVE, part, &used[w]);
         wave_sync();
         int32_t size = shrink_size(used[w], cap);
         int2* out = conn + conn_off[i];
@@ -365,8 +388,7 @@ __global__ void __launch_bounds__(BB_BLOCK)
         }
         if (threadIdx.x == 0) used = 0;
         __syncthreads();
-        for (eoff_t j = rs + threadIdx.x; j < re; j += BB_BLOCK)
-            lds_table_add(T, cap, k, part[g.col[j]], g.ew[j], &used);
+        table_add_row(T, cap, k, g, rs, re, threadIdx.x, BB_BLOCK, part, &used);
         __syncthreads();
         int32_t size = shrink_size(used, cap);
         int2* out = conn + conn_off[i];
@@ -464,8 +486,8 @@ template <int CHW, int W, bool LONG>
 __global__ void __launch_bounds__(W* WAVE)
     k_lp_select(DGraph g, const part_t* part, const eoff_t* conn_off, const int2* conn, const int32_t* conn_size,
                 part_t* dest_cache, int32_t* gain_p, int32_t* lock, double fr, part_t* dest, int32_t* pregain,
-                vid_t* cand, int32_t* counters, vid_t nmax, int32_t* next_counters, unsigned long long* pc,
-                BestCopy bc) {
+                vid_t* cand, int32_t* counters, vid_t nmax, int32_t* next_counters, uint64_t* cbits, int4* crec,
+                unsigned long long* pc, BestCopy bc) {
     constexpr int NPASS = CHW / WAVE;
     __shared__ vid_t sbuf[W * CHW];
     __shared__ int32_t sh[2 * W + 2];
@@ -561,6 +583,7 @@ __global__ void __launch_bounds__(W* WAVE)
     // pre-gain, which is then only written for candidates. The candidates'
     // gains and row offsets of all passes are loaded together.
     bool is_cand[NPASS];
+    part_t dst[NPASS];
     int32_t gain[NPASS];
     eoff_t r0[NPASS], r1[NPASS];
 #pragma unroll
@@ -569,6 +592,7 @@ __global__ void __launch_bounds__(W* WAVE)
         const bool miss = cached[u] == NULL_PART;
         const part_t best = miss ? mbest[wv][u * WAVE + lane] : cached[u];
         is_cand[u] = i < g.n && best != NO_MOVE && locks[u] == 0;
+        dst[u] = best;
         if (i < g.n) {
             dest[i] = is_cand[u] ? best : NO_MOVE;
             if (!is_cand[u] && locks[u]) lock[i] = 0;
@@ -586,6 +610,11 @@ __global__ void __launch_bounds__(W* WAVE)
         const int64_t i = wbase + u * WAVE + lane;
         const eoff_t deg = r1[u] - r0[u];
         if (is_cand[u]) pregain[i] = gain[u];
+        if (cbits) {
+            const uint64_t mk = __ballot(is_cand[u]);
+            if (lane == 0 && i < g.n) cbits[i / WAVE] = mk;
+            if (is_cand[u]) crec[i] = make_int4(dst[u], gain[u], part[i], 0);
+        }
         st.push(is_cand[u] && deg <= BIG_DEG, is_cand[u] && deg > BIG_DEG, (vid_t)i);
     }
     st.flush(cand, &counters[0], &counters[1], nmax, sh);
@@ -604,11 +633,29 @@ __global__ void __launch_bounds__(W* WAVE)
 constexpr int AB_WAVES = 16;
 constexpr int AB_CHW = 256;
 
-template <int G>
+// A neighbour's term from its record (destination, pre-gain, part), and the
+// same behind its candidate bit (a vertex without it contributes nothing).
+__device__ inline int64_t burn_term(vid_t v, vid_t i, int32_t ig, int32_t w, part_t p, part_t best, int4 r) {
+    int64_t ch = 0;
+    if (r.y > ig || (r.y == ig && v < i)) {  // afterburn_edge
+        if (r.x == p) ch -= w;
+        else if (r.x == best) ch += w;
+        if (r.z == p) ch += w;
+        else if (r.z == best) ch -= w;
+    }
+    return ch;
+}
+__device__ inline int64_t afterburn_rec(vid_t v, vid_t i, int32_t ig, int32_t w, part_t p, part_t best,
+                                        const uint32_t* cbits, const int4* crec) {
+    if (((cbits[v >> 5] >> (v & 31)) & 1u) == 0) return 0;
+    return burn_term(v, i, ig, w, p, best, crec[v]);
+}
+
+template <int G, bool REC>
 __global__ void __launch_bounds__(AB_WAVES* WAVE)
     k_afterburner_small(DGraph g, const vid_t* cand, const int32_t* counters, const part_t* part, const part_t* dest,
                         const int32_t* pregain, int32_t* lock, vid_t* moves, int32_t* mcounters, vid_t nmax,
-                        int32_t* stamp, int32_t gen) {
+                        int32_t* stamp, int32_t gen, const uint32_t* cbits, const int4* crec) {
     __shared__ vid_t sbuf[AB_WAVES * AB_CHW];
     __shared__ int32_t sh[2 * AB_WAVES + 2];
     StagedLists<AB_WAVES, AB_CHW> st(sbuf);
@@ -635,7 +682,8 @@ __global__ void __launch_bounds__(AB_WAVES* WAVE)
             int32_t ig = pregain[i];
             int64_t change = 0;
             for (eoff_t j = g.rowptr[i] + sub; j < g.rowptr[i + 1]; j += G)
-                change += afterburn_edge(g.col[j], i, ig, g.ew[j], p, best, part, dest, pregain);
+                change += REC ? afterburn_rec(g.col[j], i, ig, g.ew[j], p, best, cbits, crec)
+                              : afterburn_edge(g.col[j], i, ig, g.ew[j], p, best, part, dest, pregain);
 #pragma unroll
             for (int d = G / 2; d >= 1; d >>= 1) change += __shfl_xor(change, d, G);
             keep = (int64_t)ig + change >= 0;
@@ -647,21 +695,26 @@ __global__ void __launch_bounds__(AB_WAVES* WAVE)
 }
 
 // A wave per candidate of degree > BIG_DEG, AB_UNROLL edges per lane in
-// flight. The neighbours' destinations are gathered first: a neighbour that is
-// no candidate (NO_MOVE) contributes nothing, so its pre-gain and part are not
-// read. Candidates of degree > long_deg are queued in LDS and taken by the
+// flight. A bit per vertex says which neighbours are candidates (n / 8 bytes,
+// resident in L2; the others contribute nothing), and a candidate's
+// destination, pre-gain and part come in one 16-byte record. A wave appends
+// its moves 64 at a time: one atomic per move on the list's counter was the
+// bound where a tenth of the vertices move (R-MAT 22, 4,194,304 vertices: 1.55
+// ms on average, now 0.38; 756,505: 1.08, now 0.59, bound by the gathers).
+// Candidates of degree > long_deg are queued in LDS and taken by the
 // whole workgroup afterwards.
 constexpr int AB_UNROLL = 4;
 constexpr int AB_QUEUE = 1024;
 __global__ void __launch_bounds__(AB_WAVES* WAVE)
     k_afterburner_big(DGraph g, const vid_t* cand, const int32_t* counters, const part_t* part, const part_t* dest,
                       const int32_t* pregain, int32_t* lock, vid_t* moves, int32_t* mcounters, vid_t nmax,
-                      int32_t* stamp, int32_t gen, int32_t long_deg) {
+                      int32_t* stamp, int32_t gen, int32_t long_deg, const uint32_t* cbits, const int4* crec) {
     __shared__ vid_t queue[AB_QUEUE];
+    __shared__ vid_t keeps[AB_WAVES][WAVE];
     __shared__ int32_t nqueue;
     __shared__ int64_t red[AB_WAVES];
     const int lane = threadIdx.x & (WAVE - 1);
-    const int wv = threadIdx.x / WAVE;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE);  // the candidates' state in scalar registers
     const int32_t nb = counters[1];
     if (nb == 0) return;
     if (threadIdx.x == 0) nqueue = 0;
@@ -672,35 +725,47 @@ __global__ void __launch_bounds__(AB_WAVES* WAVE)
         int64_t change = 0;
         for (eoff_t b0 = rs; b0 < re; b0 += (eoff_t)AB_UNROLL * stride) {
             vid_t v[AB_UNROLL];
-            part_t vd[AB_UNROLL];
+            bool c[AB_UNROLL];
+            int32_t w[AB_UNROLL];
+            int4 r[AB_UNROLL];
 #pragma unroll
             for (int q = 0; q < AB_UNROLL; q++) {
                 const eoff_t j = b0 + (eoff_t)q * stride + sub;
                 v[q] = j < re ? g.col[j] : -1;
             }
 #pragma unroll
-            for (int q = 0; q < AB_UNROLL; q++) vd[q] = v[q] >= 0 ? dest[v[q]] : NO_MOVE;
+            for (int q = 0; q < AB_UNROLL; q++) c[q] = v[q] >= 0 && ((cbits[v[q] >> 5] >> (v[q] & 31)) & 1u);
 #pragma unroll
             for (int q = 0; q < AB_UNROLL; q++) {
-                if (vd[q] == NO_MOVE) continue;
-                const int32_t vg = pregain[v[q]];
-                const part_t vq = part[v[q]];
-                const int32_t w = g.ew[b0 + (eoff_t)q * stride + sub];
-                if (vg > ig || (vg == ig && v[q] < i)) {  // afterburn_edge
-                    if (vd[q] == p) change -= w;
-                    else if (vd[q] == best) change += w;
-                    if (vq == p) change += w;
-                    else if (vq == best) change -= w;
-                }
+                r[q] = c[q] ? crec[v[q]] : make_int4(0, 0, 0, 0);
+                w[q] = c[q] ? g.ew[b0 + (eoff_t)q * stride + sub] : 0;
             }
+#pragma unroll
+            for (int q = 0; q < AB_UNROLL; q++)
+                if (c[q]) change += burn_term(v[q], i, ig, w[q], p, best, r[q]);
         }
         return change;
     };
-    auto keep = [&](vid_t i, int64_t change) {  // one thread
+    // the wave's moves, appended to the list WAVE at a time
+    vid_t* kept = keeps[wv];
+    int32_t nkept = 0;
+    auto flush = [&]() {
+        wave_sync();
+        int32_t at = 0;
+        if (lane == 0) at = atomicAdd(&mcounters[3], nkept);
+        at = __shfl(at, 0, WAVE);
+        if (lane < nkept) moves[nmax - 1 - (at + lane)] = kept[lane];
+        nkept = 0;
+        wave_sync();
+    };
+    auto keep = [&](vid_t i, int64_t change) {  // a wave
         if ((int64_t)pregain[i] + change < 0) return;
-        lock[i] = 1;
-        stamp[i] = gen;
-        moves[nmax - 1 - atomicAdd(&mcounters[3], 1)] = i;
+        if (lane == 0) {
+            lock[i] = 1;
+            stamp[i] = gen;
+            kept[nkept] = i;
+        }
+        if (++nkept == WAVE) flush();
     };
     // consecutive candidates go to different workgroups
     for (int64_t x = (int64_t)wv * gridDim.x + blockIdx.x; x < nb; x += (int64_t)gridDim.x * AB_WAVES) {
@@ -715,8 +780,7 @@ __global__ void __launch_bounds__(AB_WAVES* WAVE)
                 continue;
             }
         }
-        const int64_t change = wave_reduce_sum(burn(i, rs, re, lane, WAVE));
-        if (lane == 0) keep(i, change);
+        keep(i, wave_reduce_sum(burn(i, rs, re, lane, WAVE)));
     }
     __syncthreads();
     const int32_t nq = min(nqueue, AB_QUEUE);
@@ -724,8 +788,9 @@ __global__ void __launch_bounds__(AB_WAVES* WAVE)
         const vid_t i = queue[q];
         const int64_t change = block_reduce_sum<int64_t, AB_WAVES * WAVE>(
             burn(i, g.rowptr[i], g.rowptr[i + 1], threadIdx.x, AB_WAVES * WAVE), red);
-        if (threadIdx.x == 0) keep(i, change);
+        if (wv == 0) keep(i, change);
     }
+    if (nkept > 0) flush();
 }
 
 // ---------------------------------------------------------------- perform_moves
@@ -957,7 +1022,7 @@ __global__ void __launch_bounds__(256)
                    const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
                    int32_t k, int32_t* err, int32_t* mark, const uint8_t* hub, uint8_t* hub_dirty,
                    const int32_t* deferred, const int32_t* stamp, int32_t gen, unsigned long long* sizes,
-                   int64_t* partials, uint32_t* bits, Publish pb, RebalPrep prep) {
+                   int64_t* partials, uint32_t* bits, int2* moved, Publish pb, RebalPrep prep) {
     __shared__ int64_t red[256 / WAVE];
     __shared__ int32_t ws[ADD ? 256 / WAVE + 1 : 1];
     __shared__ unsigned long long ls[ADD ? 1 : LDS_K];
@@ -1017,7 +1082,10 @@ __global__ void __launch_bounds__(256)
             const eoff_t rs = g.rowptr[i], re = g.rowptr[i + 1];
             if (sub == 0) {
                 dest_cache[i] = NULL_PART;
-                if (bits) atomicOr(&bits[i >> 5], 1u << (i & 31));
+                if (bits) {
+                    atomicOr(&bits[i >> 5], 1u << (i & 31));
+                    moved[i] = make_int2(pold, pnew);
+                }
                 rec[x] = MoveRec{rs, (int32_t)(re - rs), i, pnew, 0};
                 const unsigned long long w = (unsigned long long)g.vw[i];
                 if (lds) {
@@ -1069,7 +1137,7 @@ __global__ void __launch_bounds__(UB_BLOCK)
                  const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
                  int32_t k, int32_t* err, int32_t* mark, const uint8_t* hub, uint8_t* hub_dirty,
                  const int32_t* deferred, const int32_t* stamp, int32_t gen, unsigned long long* sizes,
-                 int64_t* partials, uint32_t* bits, int32_t long_deg, const int2* slices, int32_t nslices,
+                 int64_t* partials, uint32_t* bits, int2* moved, int32_t long_deg, const int2* slices, int32_t nslices,
                  unsigned long long* copies, int32_t ncopies) {
     __shared__ int4 queues[UB_BLOCK / WAVE][2 * WAVE];
     __shared__ unsigned long long ls[ADD ? 1 : LDS_K];
@@ -1142,7 +1210,10 @@ __global__ void __launch_bounds__(UB_BLOCK)
             const eoff_t rs = g.rowptr[i], re = g.rowptr[i + 1];
             if (lane == 0) {
                 dest_cache[i] = NULL_PART;
-                if (bits) atomicOr(&bits[i >> 5], 1u << (i & 31));
+                if (bits) {
+                    atomicOr(&bits[i >> 5], 1u << (i & 31));
+                    moved[i] = make_int2(pold, pnew);
+                }
                 rec[at] = MoveRec{rs, (int32_t)(re - rs), i, pnew, 0};
                 const unsigned long long w = (unsigned long long)g.vw[i];
                 if (lds) {
@@ -1210,7 +1281,8 @@ __global__ void __launch_bounds__(UB_BLOCK)
 // this kernel 0.32 ms on the levels of up to 438,484 vertices and 0.67 ms
 // above (0.90 ms with the stamps gathered there). Those were with one
 // workgroup of 80 registers a thread on a CU; with the row's state in scalar
-// registers two fit, and the averages are 0.37 and 0.50 ms.
+// registers two fit (0.37 and 0.50 ms), and with a moved neighbour's two parts
+// in one 8-byte word, written by the first pass, 0.30 and 0.43 ms.
 // Steps that move few vertices scan only the rows that the first pass
 // flagged; from n / PULL_ALL_DIV moves on, about a third of the rows of
 // average degree 190 have a moved neighbour and flagging costs a store per
@@ -1265,7 +1337,7 @@ __device__ inline int32_t ph_store(int2* conn, int32_t cap, int32_t vsz, int32_t
 template <bool EXACT>
 __global__ void __launch_bounds__(PH_WAVES_MAX* WAVE, 8)
     k_pull_hubs(DGraph g, const vid_t* big, int32_t nbig, const vid_t* mid, int32_t nmid, const int32_t* mc,
-                const uint32_t* bits, int32_t shift, uint8_t* hub_dirty, const part_t* part,
+                const uint32_t* bits, int32_t shift, const int2* parts, uint8_t* hub_dirty, const part_t* part,
                 const part_t* dest, const eoff_t* conn_off, int2* conn, int32_t* conn_size, part_t* dest_cache,
                 int32_t k, int32_t* err, int32_t* mark, const int32_t* deferred, int64_t* partials) {
     extern __shared__ int32_t ph_lds[];  // a dense table per wave, then the bits
@@ -1331,8 +1403,9 @@ __global__ void __launch_bounds__(PH_WAVES_MAX* WAVE, 8)
             for (int q = 0; q < PH_UNROLL; q++) {
                 const bool h = (hits >> q) & 1u;
                 w[q] = h ? ew[b0 + q * stride + sub] : 0;
-                po[q] = h ? part[v[q]] : 0;
-                pn[q] = h ? dest[v[q]] : 0;
+                const int2 p = h ? parts[v[q]] : make_int2(0, 0);
+                po[q] = p.x;
+                pn[q] = p.y;
             }
             if (!any) first();
             any = true;
@@ -2294,32 +2367,47 @@ static inline int32_t sections_for(vid_t n, int32_t k) {
 
 // Lanes per vertex of a list: the average degree rounded up to a power of
 // two.
-static int group_for_avg(const DGraph& g) {
-    double avg = g.n > 0 ? (double)g.m / g.n : 0.0;
+static int lanes_for(double avg) {
     return avg <= 4 ? 4 : avg <= 8 ? 8 : avg <= 16 ? 16 : avg <= 32 ? 32 : 64;
 }
 
 // Lanes per candidate in the afterburner: doubled on levels of up to
 // SMALL_LEVEL_N vertices, whose few candidates leave the GPU idle otherwise.
+// On levels with rows above BIG_DEG edges the average is that of the short
+// rows, which these kernels take (R-MAT 22, 4,194,304 vertices: first update
+// pass 0.18 -> 0.14 ms, second 0.13 -> 0.09).
 // Lanes per move in the update passes: doubled on every level, so that a
 // lane's chain of table updates is shorter (each measured 0.5 ms less per
 // 128^3 stencil partition; doubling the afterburner's on large levels was
 // slower).
-static int group_for_afterburner(const DGraph& g) {
+static int group_for_avg(const DGraph& g) { return lanes_for(g.n > 0 ? (double)g.m / g.n : 0.0); }
+static int group_for_afterburner(const DGraph& g, double avg) {
     const int m = g.n <= tuning().small_level_n ? (int)tuning().ab_lanes_small : 1;
-    return std::min(64, m * group_for_avg(g));
+    return std::min(64, m * lanes_for(avg));
 }
-static int group_for_update(const DGraph& g) { return std::min(64, (int)tuning().upd_lanes * group_for_avg(g)); }
+static int group_for_update(double avg) { return std::min(64, (int)tuning().upd_lanes * lanes_for(avg)); }
 
-__global__ void __launch_bounds__(256) k_max_degree(DGraph g, int32_t* out) {
+// out: the largest degree; small[0], small[1]: the rows of 1 to BIG_DEG edges,
+// and a sixteenth of their edges.
+__global__ void __launch_bounds__(256) k_max_degree(DGraph g, int32_t* out, int32_t* small) {
     __shared__ int32_t red[256 / WAVE];
-    int32_t mx = 0;
+    int32_t mx = 0, rows = 0, edges = 0;
     FOR_THREAD(i, g.n) {
         int64_t d = g.rowptr[i + 1] - g.rowptr[i];
         if (d > mx) mx = (int32_t)(d > ORD_MAX ? ORD_MAX : d);
+        if (d > 0 && d <= BIG_DEG) {
+            rows++;
+            edges += (int32_t)d;
+        }
     }
     mx = block_reduce_max<int32_t, 256>(mx, red);
     if (threadIdx.x == 0 && mx) atomicMax(out, mx);
+    rows = block_reduce_sum<int32_t, 256>(rows, red);
+    edges = block_reduce_sum<int32_t, 256>(edges, red);
+    if (threadIdx.x == 0) {
+        atomicAdd(&small[0], rows);
+        atomicAdd(&small[1], (edges + 8) / 16);
+    }
 }
 
 Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefineParams& p) : a_(a), s_(s), p_(p), nmax_(n) {
@@ -2376,6 +2464,7 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     JET_HIP(hipMemsetAsync(hub_dirty_, 0, (size_t)N, s));
     fill_i32(stamp_, -1, N, s);
     moved_bits_ = a.alloc<uint32_t>((N + 31) / 32);
+    cand_bits_ = a.alloc<uint64_t>((N + WAVE - 1) / WAVE);
     fill_i32(reinterpret_cast<int32_t*>(moved_bits_), 0, (N + 31) / 32, s);
     for (const void* f : {reinterpret_cast<const void*>(&k_pull_hubs<true>),
                           reinterpret_cast<const void*>(&k_pull_hubs<false>)})
@@ -2410,16 +2499,19 @@ void Refiner::build_tiers(const Level& L) {
     long_deg_ = (int32_t)(tuning().upd_big_slices * 2 * WAVE);
     k_conn_tiers<<<grid_for(g.n, 256, 8192), 256, 0, s_>>>(g, p_.k, tier_mid_, tier_big_, pull_mid_,
                                                             counters_ + 16, hub_, small_max_, long_deg_);
-    k_max_degree<<<grid_for(g.n, 256, 512), 256, 0, s_>>>(g, counters_ + 18);
+    k_max_degree<<<grid_for(g.n, 256, 512), 256, 0, s_>>>(g, counters_ + 18, counters_ + 22);
     JET_LAUNCH_CHECK();
-    int32_t c[5];
-    read_i32_words(counters_ + 16, 5, c, s_);
+    int32_t c[8];
+    read_i32_words(counters_ + 16, 8, c, s_);
     ntier_mid_ = c[0];
     ntier_big_ = c[1];
     has_big_ = c[2] > BIG_DEG;
     has_long_ = c[2] > SEL_LONG && p_.k > SEL_LONG && g.n > SEL_LONG_N;
     npull_mid_ = c[3];
     nslices_ = c[4];
+    // with long rows apart, the short ones' average says how many lanes they
+    // keep busy
+    avg_ = has_big_ ? 16.0 * (uint32_t)c[7] / std::max(1, c[6]) : (double)g.m / std::max<vid_t>(1, g.n);
 }
 
 // The level's row slices, in the caller's scope of the arena.
@@ -2476,20 +2568,25 @@ void Refiner::jet_lp(const Level& L, const part_t* part, double fr) {
     int32_t* c = cnt();
     gen_++;  // this step's moves are stamped with a new generation
     const BestCopy bcp = take_best_copy();
+    // on levels with long rows the candidates' records, in the moves' array,
+    // which the update passes fill later
+    uint64_t* cbits = has_big_ ? cand_bits_ : nullptr;
+    const uint32_t* cb = reinterpret_cast<const uint32_t*>(cbits);
+    int4* crec = has_big_ ? reinterpret_cast<int4*>(mrec_) : nullptr;
     // a pass per wave on levels that fill the GPU with single-pass waves, two
     // passes per wave in 16-wave workgroups above that (see LS_MULTI_CHW)
     if (g.n <= tuning().lp_one_pass_n) {
         int nb = (int)std::max<int64_t>(1, ceil_div(g.n, (int64_t)LS_WAVES * WAVE));
         family_launch(PF_LP_SELECT, k_lp_select<WAVE, LS_WAVES, false>, dim3(nb), dim3(LS_WAVES * WAVE), 0, s_, g, part,
                       conn_off_, conn_, conn_size_, dest_cache_, gain_p_, lock_, fr, dest_, pregain_, cand_, c, nmax_,
-                      cnt_next(), prof_counters(PF_LP_SELECT), bcp);
+                      cnt_next(), cbits, crec, prof_counters(PF_LP_SELECT), bcp);
     } else {
         int nb = (int)std::max<int64_t>(1, ceil_div(g.n, (int64_t)LS_MULTI_WAVES * LS_MULTI_CHW));
         family_launch(PF_LP_SELECT,
                       has_long_ ? k_lp_select<LS_MULTI_CHW, LS_MULTI_WAVES, true>
                                 : k_lp_select<LS_MULTI_CHW, LS_MULTI_WAVES, false>,
                       dim3(nb), dim3(LS_MULTI_WAVES * WAVE), 0, s_, g, part, conn_off_, conn_, conn_size_, dest_cache_, gain_p_, lock_, fr, dest_, pregain_,
-                      cand_, c, nmax_, cnt_next(), prof_counters(PF_LP_SELECT), bcp);
+                      cand_, c, nmax_, cnt_next(), cbits, crec, prof_counters(PF_LP_SELECT), bcp);
     }
     JET_LAUNCH_CHECK();
     // per vertex: cached destination 4, lock 4 (and part 4, best copy 4 when
@@ -2501,9 +2598,10 @@ void Refiner::jet_lp(const Level& L, const part_t* part, double fr) {
     }
     unsigned ab = (unsigned)std::max<int64_t>(256, ceil_div((int64_t)g.n, (int64_t)AB_WAVES * AB_CHW));
 #define JET_AB(GG)                                                                                                    \
-    family_launch(PF_AFTERBURNER, k_afterburner_small<GG>, dim3(ab), dim3(AB_WAVES * WAVE), 0, s_, g, cand_, c, part, \
-                  dest_, pregain_, lock_, moves_, c, nmax_, stamp_, gen_)
-    switch (group_for_afterburner(g)) {
+    family_launch(PF_AFTERBURNER, has_big_ ? k_afterburner_small<GG, true> : k_afterburner_small<GG, false>, dim3(ab),  \
+                  dim3(AB_WAVES * WAVE), 0, s_, g, cand_, c, part, dest_, pregain_, lock_, moves_, c, nmax_, stamp_, gen_, \
+                  cb, crec)
+    switch (group_for_afterburner(g, avg_)) {
         case 4: JET_AB(4); break;
         case 8: JET_AB(8); break;
         case 16: JET_AB(16); break;
@@ -2514,7 +2612,7 @@ void Refiner::jet_lp(const Level& L, const part_t* part, double fr) {
     if (has_big_)
         family_launch(PF_AFTERBURNER, k_afterburner_big, dim3(grid_for((int64_t)g.n * WAVE, AB_WAVES * WAVE, 512)),
                       dim3(AB_WAVES * WAVE), 0, s_, g, cand_, c, part, dest_, pregain_, lock_, moves_, c, nmax_, stamp_,
-                      gen_, long_deg_);
+                      gen_, long_deg_, cb, crec);
     JET_LAUNCH_CHECK();
 }
 
@@ -2703,7 +2801,7 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
     const int32_t k = p_.k;
     int32_t* c = cnt();
     unsigned long long* usz = reinterpret_cast<unsigned long long*>(sizes);
-    int G = group_for_update(g);
+    int G = group_for_update(avg_);
     int nbs = grid_for((int64_t)g.n * G, 256, 1024);
     const int64_t seq = ++mailbox_->seq;
     // size-delta copies for the LDS-aggregated deltas (k <= LDS_K): about
@@ -2729,6 +2827,7 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
     auto bits_bytes = [&] { return 4 * (size_t)(((int64_t)g.n + (32ll << ph_shift) - 1) >> (5 + ph_shift)); };
     while (bits_bytes() > PH_BITS_MAX) ph_shift++;
     uint32_t* bits = hubs ? moved_bits_ : nullptr;
+    int2* mv = reinterpret_cast<int2*>(score_);  // the scores of a strong step are done with
     const uint8_t* hub = hubs ? hub_ : nullptr;
     for (int add = 0; add < 2; add++) {
         if (unsigned long long* pc = prof_counters(PF_UPDATE)) {
@@ -2739,10 +2838,10 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
 #define JET_UPD(GG)                                                                                                   \
     if (add) family_launch(PF_UPDATE, k_update_small<true, GG>, dim3(nbs + 1), dim3(256), 0, s_, g, moves_, mrec_, c, \
                            nmax_, part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k, misc_ + 1, swap_bit_,    \
-                           hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, pb, prep);                      \
+                           hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, mv, pb, prep);                  \
     else family_launch(PF_UPDATE, k_update_small<false, GG>, dim3(nbs), dim3(256), 0, s_, g, moves_, mrec_, c, nmax_, \
                        part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k, misc_ + 1, swap_bit_, hub,          \
-                       hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, pb, no_prep);
+                       hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, mv, pb, no_prep);
         switch (G) {
             case 4: JET_UPD(4) break;
             case 8: JET_UPD(8) break;
@@ -2754,7 +2853,7 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
         if (has_big_) {
             family_launch(PF_UPDATE, add ? k_update_big<true> : k_update_big<false>, dim3(nbb), dim3(UB_BLOCK), 0, s_, g,
                           moves_, mrec_, c, nmax_, part, dest_, conn_off_, conn_, conn_size_, dest_cache_, k,
-                          misc_ + 1, swap_bit_, hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, long_deg_,
+                          misc_ + 1, swap_bit_, hub, hub_dirty_, misc_ + 2, stamp_, gen_, usz, pub_, bits, mv, long_deg_,
                           slices_, nslices_, pb.copies, pb.ncopies);
         }
         if (!add && hubs) {
@@ -2762,7 +2861,7 @@ bool Refiner::perform_moves(const Level& L, part_t* part, int64_t* sizes, int64_
             const int pb = std::max(1, std::min(want, 512));
             family_launch(PF_UPDATE, ph_shift == 0 ? k_pull_hubs<true> : k_pull_hubs<false>, dim3(pb),
                           dim3(ph_waves * WAVE), (uint32_t)(ph_tables + bits_bytes()), s_, g, tier_big_, ntier_big_,
-                          pull_mid_, npull_mid_, c, moved_bits_, ph_shift, hub_dirty_, part, dest_, conn_off_, conn_,
+                          pull_mid_, npull_mid_, c, moved_bits_, ph_shift, mv, hub_dirty_, part, dest_, conn_off_, conn_,
                           conn_size_, dest_cache_, k, misc_ + 1, swap_bit_, misc_ + 2, pub_);
         }
         JET_LAUNCH_CHECK();
