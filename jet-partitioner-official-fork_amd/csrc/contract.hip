@@ -63,6 +63,13 @@ __global__ void k_members(vid_t n, const vid_t* map, const int32_t* moff, int32_
     }
 }
 
+__global__ void k_member_degrees(DGraph g, const vid_t* members, int32_t* deg) {
+    FOR_THREAD(x, g.n) {
+        const vid_t i = members[x];
+        deg[x] = (int32_t)(g.rowptr[i + 1] - g.rowptr[i]);
+    }
+}
+
 __global__ void __launch_bounds__(256)
     k_tiers(vid_t nc, const eoff_t* hoff, vid_t* l1, vid_t* l2, vid_t* l3, vid_t* l4, int32_t* cnt, int32_t t1max,
             int32_t t2max) {
@@ -144,14 +151,19 @@ __global__ void __launch_bounds__(T1_WAVES* WAVE)
 
 // One workgroup per row: hash into LDS, compact the unique entries (they fill
 // at most half of the table), then bitonic-sort only those. Sorting the whole
-// table took four times the exchanges: 7.5 ms a call on R-MAT 22's levels.
+// table took four times the exchanges: 7.5 ms a call on R-MAT 22's levels,
+// 4.7 with the entries packed and rows in two sizes, 2.6 with the row's edges
+// shared equally by the waves. Bound by the insertions' and the sort's LDS
+// round trips.
 template <int BLOCK, int CAP>
 __global__ void __launch_bounds__(BLOCK)
-    k_dedupe_block(DGraph g, const vid_t* map, const vid_t* members, const int32_t* moff, const eoff_t* hoff,
-                   const vid_t* list, int32_t nrows, vid_t* tkey, wgt_t* tval, int32_t* ucount) {
+    k_dedupe_block(DGraph g, const vid_t* map, const vid_t* members, const eoff_t* medge, const int32_t* moff,
+                   const eoff_t* hoff, const vid_t* list, int32_t nrows, vid_t* tkey, wgt_t* tval, int32_t* ucount) {
     __shared__ int32_t keys[CAP];
     __shared__ int32_t vals[CAP];
     __shared__ int32_t ws[BLOCK / WAVE + 1];
+    __shared__ int32_t s_e[BLOCK / WAVE][WAVE];
+    __shared__ eoff_t s_rs[BLOCK / WAVE][WAVE];
     constexpr int PER = CAP / BLOCK;
     for (int32_t r = blockIdx.x; r < nrows; r += gridDim.x) {
         vid_t c = list[r];
@@ -164,17 +176,15 @@ __global__ void __launch_bounds__(BLOCK)
             vals[t] = 0;
         }
         __syncthreads();
-        int32_t mb = moff[c], me = moff[c + 1];
-        const int lane = threadIdx.x & (WAVE - 1);
+        // an equal share of the row's edges to each wave, whatever members they
+        // are of: a member per wave left most waves waiting for the longest
         const int wid = threadIdx.x / WAVE;
-        // members round-robin over waves; each wave walks its member's row
-        for (int32_t mi = mb + wid; mi < me; mi += BLOCK / WAVE) {
-            vid_t i = members[mi];
-            for (eoff_t j = g.rowptr[i] + lane; j < g.rowptr[i + 1]; j += WAVE) {
-                vid_t u = map[g.col[j]];
-                if (u != c) lds_insert(keys, vals, cap - 1, u, g.ew[j]);
-            }
-        }
+        const int32_t share = (hsz + BLOCK / WAVE * WAVE - 1) / (BLOCK / WAVE * WAVE) * WAVE;
+        const eoff_t ea = hs + min(hsz, wid * share), eb = hs + min(hsz, (wid + 1) * share);
+        wave_edge_range(g, members, medge, moff[c], moff[c + 1], ea, eb, s_e[wid], s_rs[wid], [&](eoff_t j, eoff_t) {
+            const vid_t u = map[g.col[j]];
+            if (u != c) lds_insert(keys, vals, cap - 1, u, g.ew[j]);
+        });
         __syncthreads();
         // the unique entries, packed to the front through registers
         int32_t rk[PER], rv[PER];
@@ -227,41 +237,40 @@ __global__ void __launch_bounds__(BLOCK)
     }
 }
 
-// ---- spill path: (row rank << 32 | neighbour) keys, radix sort, reduce by key
+// ---- spill path: (row rank << nbits | neighbour) keys, all ones for the
+// diagonal; radix sort, reduce by key
+// A wave takes SPILL_CHUNK consecutive places of the concatenated spilled rows,
+// whatever rows and members they are of. (A workgroup per row and a wave per
+// member left one wave with the longest member: 2.4 ms a call on R-MAT 22's
+// levels and 7.5 on the first; now 0.44 and 0.65.)
+constexpr int64_t SPILL_CHUNK = 1024;
 __global__ void __launch_bounds__(256)
-    k_spill_gather(DGraph g, const vid_t* map, const vid_t* members, const int32_t* moff, const vid_t* list,
-                   int32_t n3, const eoff_t* soff, uint64_t* skey, uint32_t* sval) {
-    const int lane = threadIdx.x & (WAVE - 1);
+    k_spill_gather(DGraph g, const vid_t* map, const vid_t* members, const eoff_t* medge, const int32_t* moff,
+                   const eoff_t* hoff, const vid_t* list, int32_t n3, const eoff_t* soff, eoff_t len, int nbits,
+                   uint64_t* skey, uint32_t* sval) {
+    __shared__ int32_t s_e[256 / WAVE][WAVE];
+    __shared__ eoff_t s_rs[256 / WAVE][WAVE];
     const int wid = threadIdx.x / WAVE;
-    __shared__ eoff_t wpos[256 / WAVE];
-    for (int32_t r = blockIdx.x; r < n3; r += gridDim.x) {
-        vid_t c = list[r];
-        eoff_t base = soff[r];
-        int32_t mb = moff[c], me = moff[c + 1];
-        // members round-robin over waves; wave-private output cursors derived
-        // from the member's position in the row's member prefix
-        for (int32_t mi0 = mb; mi0 < me; mi0 += 256 / WAVE) {
-            int32_t mi = mi0 + wid;
-            eoff_t d = 0, rs = 0;
-            if (mi < me) {
-                vid_t i = members[mi];
-                rs = g.rowptr[i];
-                d = g.rowptr[i + 1] - rs;
-            }
-            if (lane == 0) wpos[wid] = d;
-            __syncthreads();
-            eoff_t before = 0;
-            for (int q = 0; q < wid; q++) before += wpos[q];
-            eoff_t chunk = 0;
-            for (int q = 0; q < 256 / WAVE; q++) chunk += wpos[q];
-            for (eoff_t t = lane; t < d; t += WAVE) {
-                vid_t u = map[g.col[rs + t]];
-                uint64_t key = u == c ? ~0ull : (((uint64_t)r << 32) | (uint32_t)u);
-                skey[base + before + t] = key;
-                sval[base + before + t] = (uint32_t)g.ew[rs + t];
-            }
-            __syncthreads();
-            base += chunk;
+    const int64_t stride = (int64_t)gridDim.x * (256 / WAVE) * SPILL_CHUNK;
+    for (int64_t t0 = ((int64_t)blockIdx.x * (256 / WAVE) + wid) * SPILL_CHUNK; t0 < len; t0 += stride) {
+        const int64_t t1 = min((int64_t)len, t0 + SPILL_CHUNK);
+        int32_t r = 0, hi = n3 - 1;  // the row that holds place t0
+        while (r < hi) {
+            const int32_t mid = (r + hi + 1) >> 1;
+            if (soff[mid] <= t0) r = mid;
+            else hi = mid - 1;
+        }
+        for (int64_t t = t0; t < t1; r++) {
+            const vid_t c = list[r];
+            const eoff_t base = soff[r], end = min((eoff_t)t1, soff[r + 1]), h = hoff[c];
+            wave_edge_range(g, members, medge, moff[c], moff[c + 1], h + (t - base), h + (end - base), s_e[wid],
+                            s_rs[wid], [&](eoff_t j, eoff_t e) {
+                                const vid_t u = map[g.col[j]];
+                                const eoff_t at = base + (e - h);
+                                skey[at] = u == c ? ~0ull : (((uint64_t)r << nbits) | (uint32_t)u);
+                                sval[at] = (uint32_t)g.ew[j];
+                            });
+            t = end;
         }
     }
 }
@@ -279,9 +288,9 @@ __global__ void k_spill_heads(const uint64_t* skey, int64_t len, int32_t* head) 
 // unique entry is found by its neighbour's key instead of a minimum over the
 // row. With an atomic per entry, the entries of the few hub rows met on a few
 // addresses: 11.1 ms per call on R-MAT 22's levels (spill_write, which
-// counted a row's uniques with an atomic each, 10.5 ms).
+// counted a row's uniques with an atomic each, 10.5 ms); now 0.34 and 0.29.
 __global__ void __launch_bounds__(256)
-    k_spill_reduce(const uint64_t* skey, const uint32_t* sval, int64_t len, const int32_t* uid_ex, int32_t* ukey,
+    k_spill_reduce(const uint64_t* skey, const uint32_t* sval, int64_t len, int nbits, const int32_t* uid_ex, int32_t* ukey,
                    wgt_t* uval, int32_t* urow, int32_t* rowfirst) {
     const int lane = threadIdx.x & (WAVE - 1);
     for (int64_t t0 = blockIdx.x * (int64_t)256 + (threadIdx.x - lane); t0 < len; t0 += (int64_t)gridDim.x * 256) {
@@ -305,10 +314,10 @@ __global__ void __launch_bounds__(256)
         const bool last = lane == WAVE - 1 || kn != k;  // of the wave's stretch of the run
         if (valid && last) atomicAdd(&uval[uid], v);
         if (valid && head) {
-            const int32_t r = (int32_t)(k >> 32);
-            ukey[uid] = (int32_t)(k & 0xffffffffull);
+            const int32_t r = (int32_t)(k >> nbits);
+            ukey[uid] = (int32_t)(k & ((1ull << nbits) - 1ull));
             urow[uid] = r;
-            if (t == 0 || (int32_t)(kp >> 32) != r) rowfirst[r] = uid;
+            if (t == 0 || (int32_t)(kp >> nbits) != r) rowfirst[r] = uid;
         }
     }
 }
@@ -327,19 +336,17 @@ __global__ void k_spill_write(int32_t U, const int32_t* ukey, const wgt_t* uval,
     }
 }
 
-__global__ void k_consolidate(vid_t nc, int64_t mc, const eoff_t* crow, const eoff_t* hoff, const vid_t* tkey,
-                              const wgt_t* tval, vid_t* col, wgt_t* ew) {
-    FOR_THREAD(e, mc) {
-        int32_t lo = 0, hi = nc - 1;
-        while (lo < hi) {
-            int32_t mid = (lo + hi + 1) >> 1;
-            if (crow[mid] <= e) lo = mid;
-            else hi = mid - 1;
-        }
-        eoff_t src = hoff[lo] + (e - crow[lo]);
+// A search of all rows per entry was 1.43 ms a call on R-MAT 22's levels, of
+// a tile's rows in LDS 0.54 (16 bytes per entry at the copy rate: 0.22).
+__global__ void __launch_bounds__(256)
+    k_consolidate(vid_t nc, int64_t mc, const eoff_t* crow, const eoff_t* hoff, const vid_t* tkey, const wgt_t* tval,
+                  vid_t* col, wgt_t* ew) {
+    __shared__ EdgeWalkLds walk;
+    block_edges<256>(crow, nc, mc, walk, [&](vid_t r, eoff_t e) {
+        const eoff_t src = hoff[r] + (e - crow[r]);
         col[e] = tkey[src];
         ew[e] = tval[src];
-    }
+    });
 }
 
 __global__ void k_spill_sizes(const vid_t* list, int32_t n3, const eoff_t* hoff, eoff_t* ssz) {
@@ -388,14 +395,23 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
                                                                                    cnt, tkey, tval, ucount);
         JET_LAUNCH_CHECK();
     }
+    eoff_t* medge = nullptr;  // the first fine edge of each member, in the rows' concatenated edges
+    if (hcnt[1] > 0 || hcnt[2] > 0 || hcnt[3] > 0) {
+        medge = a.alloc<eoff_t>((int64_t)g.n + 1);
+        ArenaScope scd(a);
+        int32_t* deg = a.alloc<int32_t>((int64_t)g.n + 1);
+        k_member_degrees<<<nb, 256, 0, s>>>(g, members, deg);
+        JET_LAUNCH_CHECK();
+        excl_scan_i32_i64(deg, medge, g.n, a, s);
+    }
     if (hcnt[1] > 0) {
-        k_dedupe_block<256, T2S_CAP><<<std::min(hcnt[1], 8192), 256, 0, s>>>(g, map, members, moff, hoff, l2, hcnt[1],
-                                                                            tkey, tval, ucount);
+        k_dedupe_block<256, T2S_CAP><<<std::min(hcnt[1], 8192), 256, 0, s>>>(g, map, members, medge, moff, hoff, l2,
+                                                                            hcnt[1], tkey, tval, ucount);
         JET_LAUNCH_CHECK();
     }
     if (hcnt[3] > 0) {
-        k_dedupe_block<1024, T2_CAP><<<std::min(hcnt[3], 2048), 1024, 0, s>>>(g, map, members, moff, hoff, l4, hcnt[3],
-                                                                             tkey, tval, ucount);
+        k_dedupe_block<1024, T2_CAP><<<std::min(hcnt[3], 2048), 1024, 0, s>>>(g, map, members, medge, moff, hoff, l4,
+                                                                             hcnt[3], tkey, tval, ucount);
         JET_LAUNCH_CHECK();
     }
     if (hcnt[2] > 0) {
@@ -410,11 +426,15 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
         uint32_t* sval = a.alloc<uint32_t>(H3);
         uint64_t* ktmp = a.alloc<uint64_t>(H3);
         uint32_t* vtmp = a.alloc<uint32_t>(H3);
-        k_spill_gather<<<std::min(n3, 4096), 256, 0, s>>>(g, map, members, moff, l3, n3, soff, skey, sval);
-        JET_LAUNCH_CHECK();
-        int rbits = 1;
+        // keys of as few bits as the rows and neighbours need: four or five radix
+        // passes instead of six on R-MAT 22's levels
+        int rbits = 1, nbits = 1;
         while ((int64_t(1) << rbits) < n3 + 1) rbits++;
-        radix_sort_u64(skey, sval, H3, 32 + rbits + 1, ktmp, vtmp, a, s);
+        while ((int64_t(1) << nbits) < nc) nbits++;
+        k_spill_gather<<<grid_for(ceil_div(H3, SPILL_CHUNK) * WAVE, 256, 8192), 256, 0, s>>>(
+            g, map, members, medge, moff, hoff, l3, n3, soff, H3, nbits, skey, sval);
+        JET_LAUNCH_CHECK();
+        radix_sort_u64(skey, sval, H3, nbits + rbits, ktmp, vtmp, a, s);
         int32_t* uid = a.alloc<int32_t>(H3 + 1);
         int hb = grid_for(H3, 256, 8192);
         k_spill_heads<<<hb, 256, 0, s>>>(skey, H3, uid);
@@ -426,7 +446,7 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
         int32_t* urow = a.alloc<int32_t>(U);
         int32_t* rowfirst = a.alloc<int32_t>(n3);
         fill_i32(uval, 0, U, s);
-        k_spill_reduce<<<hb, 256, 0, s>>>(skey, sval, H3, uid, ukey, uval, urow, rowfirst);
+        k_spill_reduce<<<hb, 256, 0, s>>>(skey, sval, H3, nbits, uid, ukey, uval, urow, rowfirst);
         JET_LAUNCH_CHECK();
         if (U > 0) {
             k_spill_write<<<grid_for(U, 256, 8192), 256, 0, s>>>(U, ukey, uval, urow, rowfirst, l3, hoff, tkey, tval,
@@ -439,7 +459,7 @@ void contract(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, Arena
     out.col = persist.alloc<vid_t>(out.m);
     out.ew = persist.alloc<wgt_t>(out.m);
     if (out.m > 0) {
-        k_consolidate<<<grid_for(out.m, 256, 16384), 256, 0, s>>>(nc, out.m, out.rowptr, hoff, tkey, tval, out.col,
+        k_consolidate<<<grid_for(ceil_div(out.m, EB_TILE) * 256, 256, 4096), 256, 0, s>>>(nc, out.m, out.rowptr, hoff, tkey, tval, out.col,
                                                                    out.ew);
         JET_LAUNCH_CHECK();
     }
