@@ -20,6 +20,7 @@
 // rebalancer's destination re-draws run in increasing vertex id.
 #include <algorithm>
 #include <chrono>
+#include <mutex>
 #include <cmath>
 
 #include "prims.h"
@@ -2410,6 +2411,37 @@ __global__ void __launch_bounds__(256) k_max_degree(DGraph g, int32_t* out, int3
     }
 }
 
+// The refiner's state that starts at a fixed value, filled in one launch (ten
+// launches of some 3 us each were a tenth of a small quality call).
+struct InitWords {
+    struct Seg {
+        int32_t* p;
+        int32_t v;
+        int64_t words;
+    } seg[10];
+    int count;
+};
+__global__ void __launch_bounds__(256) k_init_words(InitWords w) {
+    for (int q = 0; q < w.count; q++) FOR_THREAD(i, w.seg[q].words) w.seg[q].p[i] = w.seg[q].v;
+}
+
+// Dynamic LDS above 64 KB is allowed per kernel and device, once.
+static void allow_pull_lds() {
+    static std::once_flag once[64];
+    static hipError_t rc[64];
+    int dev = 0;
+    JET_HIP(hipGetDevice(&dev));
+    if (dev < 0 || dev >= 64) throw DeviceError("device index beyond 64");
+    std::call_once(once[dev], [&] {
+        for (const void* f : {reinterpret_cast<const void*>(&k_pull_hubs<true>),
+                              reinterpret_cast<const void*>(&k_pull_hubs<false>)}) {
+            rc[dev] = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PH_LDS_MAX);
+            if (rc[dev] != hipSuccess) return;
+        }
+    });
+    JET_HIP(rc[dev]);
+}
+
 Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefineParams& p) : a_(a), s_(s), p_(p), nmax_(n) {
     if (p.k < 1 || p.k > MAX_K) throw std::invalid_argument("k out of range");
     if (2 * sizeof(int2) * (size_t)p.k > 65536) {
@@ -2417,6 +2449,7 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
         JET_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conn_build_block),
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)(2 * sizeof(int2) * MAX_K)));
     }
+    allow_pull_lds();
     int64_t N = std::max<int64_t>(n, 1);
     conn_off_ = a.alloc<eoff_t>(N + 1);
     conn_ = a.alloc<int2>(std::max<int64_t>(cap, 1));
@@ -2458,19 +2491,8 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     ncopies_ = (int32_t)std::max<int64_t>(
         1, std::min<int64_t>(BUCKET_COPIES_MAX, BUCKET_COPIES_BYTES / ((int64_t)sizeof(int64_t) * nbuckets_)));
     bcopies_ = a.alloc<int64_t>(std::max<int64_t>(1, nbuckets_ * (ncopies_ - 1)));
-    if (ncopies_ > 1) fill_i64(bcopies_, 0, nbuckets_ * (ncopies_ - 1), s);
-    fill_i32(swap_bit_, 0, N, s);
-    fill_i32(rd_mark_, 0, N, s);
-    JET_HIP(hipMemsetAsync(hub_dirty_, 0, (size_t)N, s));
-    fill_i32(stamp_, -1, N, s);
     moved_bits_ = a.alloc<uint32_t>((N + 31) / 32);
     cand_bits_ = a.alloc<uint64_t>((N + WAVE - 1) / WAVE);
-    fill_i32(reinterpret_cast<int32_t*>(moved_bits_), 0, (N + 31) / 32, s);
-    for (const void* f : {reinterpret_cast<const void*>(&k_pull_hubs<true>),
-                          reinterpret_cast<const void*>(&k_pull_hubs<false>)})
-        JET_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)PH_LDS_MAX));
-    fill_i32(counters_, 0, 32, s);
-    fill_i64(acc_, 0, 8, s);
     wg_state_ = a.alloc<WgState>(1);
     wg_list_ = a.alloc<vid_t>(N);
     wg_runb_ = a.alloc<int32_t>(WG_MAX_NBK + 1);
@@ -2480,9 +2502,23 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     team_rkey_ = a.alloc<uint64_t>(std::min<int64_t>(N, TEAM_MAX_N));
     team_rweight_ = a.alloc<int32_t>(std::min<int64_t>(N, TEAM_MAX_N));
     pub_ = a.alloc<int64_t>((int64_t)PUB_GROUPS * PUB_STRIDE);
-    fill_i64(pub_, 0, (int64_t)PUB_GROUPS * PUB_STRIDE, s);
     szc_ = a.alloc<int64_t>((int64_t)SIZE_COPIES_MAX * p.k);
-    fill_i64(szc_, 0, (int64_t)SIZE_COPIES_MAX * p.k, s);
+    InitWords iw{};
+    auto set = [&](void* p, int32_t v, int64_t bytes) { iw.seg[iw.count++] = {static_cast<int32_t*>(p), v, (bytes + 3) / 4}; };
+    set(bcopies_, 0, 8 * nbuckets_ * (ncopies_ - 1));
+    set(swap_bit_, 0, 4 * N);
+    set(rd_mark_, 0, 4 * N);
+    set(hub_dirty_, 0, N);
+    set(stamp_, -1, 4 * N);
+    set(moved_bits_, 0, 4 * ((N + 31) / 32));
+    set(counters_, 0, 4 * 32);
+    set(acc_, 0, 8 * 8);
+    set(pub_, 0, 8 * (int64_t)PUB_GROUPS * PUB_STRIDE);
+    set(szc_, 0, 8 * (int64_t)SIZE_COPIES_MAX * p.k);
+    int64_t words = 0;
+    for (int q = 0; q < iw.count; q++) words = std::max(words, iw.seg[q].words);
+    k_init_words<<<grid_for(words, 256, 8192), 256, 0, s>>>(iw);
+    JET_LAUNCH_CHECK();
     // (cut change, largest part) of each iteration land in mailbox slots 8, 9
     Mailbox& mb = thread_mailbox();
     mailbox_ = &mb;
