@@ -63,10 +63,10 @@ __global__ void k_hec_uniform(DGraph g, uint64_t seed, uint32_t level, vid_t* hn
 }
 
 __global__ void k_vw_sum(DGraph g, unsigned long long* out) {
-    __shared__ int64_t red[256 / WAVE];
+    __shared__ int64_t red[1024 / WAVE];
     int64_t s = 0;
     FOR_THREAD(i, g.n) s += g.vw[i];
-    s = block_reduce_sum<int64_t, 256>(s, red);
+    s = block_reduce_sum<int64_t, 1024>(s, red);
     if (threadIdx.x == 0) atomicAdd(out, (unsigned long long)s);
 }
 
@@ -146,7 +146,7 @@ void hec_heavy_neighbours(const DGraph& g, bool uniform, uint64_t seed, int32_t 
     ArenaScope sc(a);
     unsigned long long* sum = a.alloc<unsigned long long>(1);
     fill_i64(reinterpret_cast<int64_t*>(sum), 0, 1, s);
-    k_vw_sum<<<grid_for(g.n, 256, 1024), 256, 0, s>>>(g, sum);
+    k_vw_sum<<<grid_for(g.n, 1024, 256), 1024, 0, s>>>(g, sum);
     JET_LAUNCH_CHECK();
     int G = group_for(g);
     int blocks = grid_for((int64_t)g.n * G, 256, 16384);

@@ -19,9 +19,13 @@ __global__ void k_validate_offsets(vid_t n, const eoff_t* rowptr, eoff_t m, int3
 // err bits: 2 column out of range, 4 non-positive edge weight, 8 non-positive
 // vertex weight, 16 weight total overflows int32 (set on the host). Flat
 // passes over vertices and over edges, so hubs do not serialise a thread.
-__global__ void k_validate(vid_t n, eoff_t m, const vid_t* col, const wgt_t* ew, const wgt_t* vw, int32_t* err,
-                           unsigned long long* sums) {
-    __shared__ int64_t red[256 / WAVE];
+// Few large workgroups: each adds to the two sums once, and atomics on one
+// address take some 12 ns each (4096 workgroups: 103 us whatever the size).
+constexpr int VA_BLOCK = 1024;
+__global__ void __launch_bounds__(VA_BLOCK)
+    k_validate(vid_t n, eoff_t m, const vid_t* col, const wgt_t* ew, const wgt_t* vw, int32_t* err,
+               unsigned long long* sums) {
+    __shared__ int64_t red[VA_BLOCK / WAVE];
     int64_t se = 0, sv = 0;
     int32_t e = 0;
     FOR_THREAD(i, n) {
@@ -43,8 +47,8 @@ __global__ void k_validate(vid_t n, eoff_t m, const vid_t* col, const wgt_t* ew,
         }
     }
     if (e) atomicOr(err, e);
-    se = block_reduce_sum<int64_t, 256>(se, red);
-    sv = block_reduce_sum<int64_t, 256>(sv, red);
+    se = block_reduce_sum<int64_t, VA_BLOCK>(se, red);
+    sv = block_reduce_sum<int64_t, VA_BLOCK>(sv, red);
     if (threadIdx.x == 0) {
         atomicAdd(&sums[0], (unsigned long long)se);
         atomicAdd(&sums[1], (unsigned long long)sv);
@@ -58,7 +62,7 @@ void launch_validate_offsets(vid_t n, const eoff_t* rowptr, eoff_t m, int32_t* e
 
 void launch_validate(vid_t n, eoff_t m, const vid_t* col, const wgt_t* ew, const wgt_t* vw, int32_t* err,
                      unsigned long long* sums, hipStream_t s) {
-    k_validate<<<grid_for(std::max<int64_t>(n, m), 256, 4096), 256, 0, s>>>(n, m, col, ew, vw, err, sums);
+    k_validate<<<grid_for(std::max<int64_t>(n, m), VA_BLOCK, 512), VA_BLOCK, 0, s>>>(n, m, col, ew, vw, err, sums);
     JET_LAUNCH_CHECK();
 }
 
@@ -146,14 +150,15 @@ bool parts_in_range(int64_t n, const int32_t* part, int32_t k, Arena& a, hipStre
     return read_scalar(err, s) == 0;
 }
 
-__global__ void k_conn_capacity(vid_t n, const eoff_t* rowptr, int32_t k, unsigned long long* out) {
-    __shared__ int64_t red[256 / WAVE];
+__global__ void __launch_bounds__(VA_BLOCK)
+    k_conn_capacity(vid_t n, const eoff_t* rowptr, int32_t k, unsigned long long* out) {
+    __shared__ int64_t red[VA_BLOCK / WAVE];
     int64_t c = 0;
     FOR_THREAD(i, n) {
         int64_t d = rowptr[i + 1] - rowptr[i];
         c += d > k ? k : d;
     }
-    c = block_reduce_sum<int64_t, 256>(c, red);
+    c = block_reduce_sum<int64_t, VA_BLOCK>(c, red);
     if (threadIdx.x == 0 && c) atomicAdd(out, (unsigned long long)c);
 }
 
@@ -162,7 +167,7 @@ int64_t conn_capacity(vid_t n, const eoff_t* rowptr, int32_t k, Arena& a, hipStr
     unsigned long long* out = a.alloc<unsigned long long>(1);
     fill_i64(reinterpret_cast<int64_t*>(out), 0, 1, s);
     if (n > 0) {
-        k_conn_capacity<<<grid_for(n, 256, 4096), 256, 0, s>>>(n, rowptr, k, out);
+        k_conn_capacity<<<grid_for(n, VA_BLOCK, 512), VA_BLOCK, 0, s>>>(n, rowptr, k, out);
         JET_LAUNCH_CHECK();
     }
     return (int64_t)read_scalar(out, s);

@@ -59,7 +59,8 @@ __global__ void k_cut2(DGraph g, const part_t* part, unsigned long long* out) {
 
 void launch_cut2(const DGraph& g, const part_t* part, unsigned long long* out, hipStream_t s) {
     if (g.n > 0 && g.m > 0) {
-        k_cut2<<<grid_for(g.m, EB_TILE, 8192), 256, 0, s>>>(g, part, out);
+        // 1024 workgroups fill the device; each adds to the one sum (12 ns)
+        k_cut2<<<grid_for(g.m, EB_TILE, 1024), 256, 0, s>>>(g, part, out);
         JET_LAUNCH_CHECK();
     }
 }
@@ -93,7 +94,7 @@ __global__ void k_part_sizes(DGraph g, const part_t* part, int32_t k, unsigned l
 void part_sizes(const DGraph& g, const part_t* part, int32_t k, int64_t* sizes, hipStream_t s) {
     fill_i64(sizes, 0, k, s);
     if (g.n > 0) {
-        k_part_sizes<<<grid_for(g.n, 256, 2048), 256, 0, s>>>(g, part, k, reinterpret_cast<unsigned long long*>(sizes));
+        k_part_sizes<<<grid_for(g.n, 1024, 256), 1024, 0, s>>>(g, part, k, reinterpret_cast<unsigned long long*>(sizes));
         JET_LAUNCH_CHECK();
     }
 }
@@ -2389,9 +2390,11 @@ static int group_for_afterburner(const DGraph& g, double avg) {
 static int group_for_update(double avg) { return std::min(64, (int)tuning().upd_lanes * lanes_for(avg)); }
 
 // out: the largest degree; small[0], small[1]: the rows of 1 to BIG_DEG edges,
-// and a sixteenth of their edges.
-__global__ void __launch_bounds__(256) k_max_degree(DGraph g, int32_t* out, int32_t* small) {
-    __shared__ int32_t red[256 / WAVE];
+// and a sixteenth of their edges. Few workgroups: atomics on one address take
+// some 12 ns each.
+constexpr int MD_BLOCK = 1024;
+__global__ void __launch_bounds__(MD_BLOCK) k_max_degree(DGraph g, int32_t* out, int32_t* small) {
+    __shared__ int32_t red[MD_BLOCK / WAVE];
     int32_t mx = 0, rows = 0, edges = 0;
     FOR_THREAD(i, g.n) {
         int64_t d = g.rowptr[i + 1] - g.rowptr[i];
@@ -2401,10 +2404,10 @@ __global__ void __launch_bounds__(256) k_max_degree(DGraph g, int32_t* out, int3
             edges += (int32_t)d;
         }
     }
-    mx = block_reduce_max<int32_t, 256>(mx, red);
+    mx = block_reduce_max<int32_t, MD_BLOCK>(mx, red);
     if (threadIdx.x == 0 && mx) atomicMax(out, mx);
-    rows = block_reduce_sum<int32_t, 256>(rows, red);
-    edges = block_reduce_sum<int32_t, 256>(edges, red);
+    rows = block_reduce_sum<int32_t, MD_BLOCK>(rows, red);
+    edges = block_reduce_sum<int32_t, MD_BLOCK>(edges, red);
     if (threadIdx.x == 0) {
         atomicAdd(&small[0], rows);
         atomicAdd(&small[1], (edges + 8) / 16);
@@ -2535,7 +2538,7 @@ void Refiner::build_tiers(const Level& L) {
     long_deg_ = (int32_t)(tuning().upd_big_slices * 2 * WAVE);
     k_conn_tiers<<<grid_for(g.n, 256, 8192), 256, 0, s_>>>(g, p_.k, tier_mid_, tier_big_, pull_mid_,
                                                             counters_ + 16, hub_, small_max_, long_deg_);
-    k_max_degree<<<grid_for(g.n, 256, 512), 256, 0, s_>>>(g, counters_ + 18, counters_ + 22);
+    k_max_degree<<<grid_for(g.n, MD_BLOCK, 256), MD_BLOCK, 0, s_>>>(g, counters_ + 18, counters_ + 22);
     JET_LAUNCH_CHECK();
     int32_t c[8];
     read_i32_words(counters_ + 16, 8, c, s_);
@@ -3260,26 +3263,38 @@ void Refiner::single_step(const Level& L, const part_t* part, int kind, double f
 // part_stat.hpp:131-144, 186-239 from the connectivity tables: the
 // communication volume (per vertex, the parts other than its own that its
 // neighbours are in) and the cut weight incident to each part.
-__global__ void k_quality(DGraph g, const part_t* part, const eoff_t* conn_off, const int2* conn,
-                          const int32_t* conn_size, unsigned long long* comm, unsigned long long* cut_per_part) {
-    __shared__ int64_t red[256 / WAVE];
+// Each workgroup sums the parts' cut weights in LDS (k <= LDS_K): an atomic per
+// vertex on k addresses took 296 us on a 64^3 stencil with k = 256.
+constexpr int QU_BLOCK = 1024;
+__global__ void __launch_bounds__(QU_BLOCK)
+    k_quality(DGraph g, const part_t* part, int32_t k, const eoff_t* conn_off, const int2* conn,
+              const int32_t* conn_size, unsigned long long* comm, unsigned long long* cut_per_part) {
+    __shared__ int64_t red[QU_BLOCK / WAVE];
+    __shared__ unsigned long long ls[LDS_K];
+    const bool lds = k <= LDS_K;
+    if (lds) {
+        for (int t = threadIdx.x; t < k; t += QU_BLOCK) ls[t] = 0;
+        __syncthreads();
+    }
     int64_t c = 0;
     FOR_THREAD(i, g.n) {
         const part_t p = part[i];
-        const int2* tab = conn + conn_off[i];
-        const int32_t sz = conn_size[i];
         int64_t ext = 0;
-        for (int32_t s = 0; s < sz; s++) {
-            int2 e = tab[s];
+        for_slots(conn + conn_off[i], conn_size[i], [&](int2 e) {
             if (e.x > NULL_PART && e.x != p && e.y > 0) {
                 c++;
                 ext += e.y;
             }
-        }
-        if (ext) atomicAdd(&cut_per_part[p], (unsigned long long)ext);
+        });
+        if (ext) atomicAdd(lds ? &ls[p] : &cut_per_part[p], (unsigned long long)ext);
     }
-    c = block_reduce_sum<int64_t, 256>(c, red);
+    c = block_reduce_sum<int64_t, QU_BLOCK>(c, red);
     if (threadIdx.x == 0 && c) atomicAdd(comm, (unsigned long long)c);
+    if (lds) {
+        __syncthreads();
+        for (int t = threadIdx.x; t < k; t += QU_BLOCK)
+            if (ls[t]) atomicAdd(&cut_per_part[t], ls[t]);
+    }
 }
 
 void Refiner::quality(const Level& L, const part_t* part, int64_t& comm_size, std::vector<int64_t>& cut_per_part) {
@@ -3290,7 +3305,8 @@ void Refiner::quality(const Level& L, const part_t* part, int64_t& comm_size, st
     ArenaScope sc(a_);
     unsigned long long* d = a_.alloc<unsigned long long>(1 + p_.k);
     fill_i64(reinterpret_cast<int64_t*>(d), 0, 1 + p_.k, s_);
-    k_quality<<<grid_for(g.n, 256, 4096), 256, 0, s_>>>(g, cur_part_, conn_off_, conn_, conn_size_, d, d + 1);
+    k_quality<<<grid_for(g.n, QU_BLOCK, 512), QU_BLOCK, 0, s_>>>(g, cur_part_, p_.k, conn_off_, conn_, conn_size_, d,
+                                                                 d + 1);
     JET_LAUNCH_CHECK();
     std::vector<int64_t> h(1 + p_.k);
     JET_HIP(hipMemcpyAsync(h.data(), d, sizeof(int64_t) * h.size(), hipMemcpyDeviceToHost, s_));
