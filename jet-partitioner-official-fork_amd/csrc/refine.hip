@@ -2777,7 +2777,12 @@ void Refiner::rebalance(const Level& L, const part_t* part, const int64_t* sizes
     unsigned long long* bc = reinterpret_cast<unsigned long long*>(bcopies_);
     // one copy per sel_copy_wgs workgroups (256 by default): fewer
     // workgroups meet on a line, and a copy costs a pass of the fold
-    const int32_t copies = std::max(1, std::min<int32_t>(ncopies_, (int32_t)(nsel / tuning().sel_copy_wgs)));
+    // With few parts every workgroup adds to every bucket, and the atomics of
+    // all workgroups meet on each line (10 ns each): a copy per 16 k workgroups.
+    // Stencil levels of 136,971 and 254,104 vertices: k = 2 42 -> 34 and 36 ->
+    // 34 us an iteration, k = 4 47 -> 40 and 67 -> 45, k = 8 43 -> 40 and 49 -> 45.
+    const int64_t copy_wgs = std::min<int64_t>(tuning().sel_copy_wgs, std::max<int64_t>(32, 16 * (int64_t)k));
+    const int32_t copies = std::max(1, std::min<int32_t>(ncopies_, (int32_t)(nsel / copy_wgs)));
     const bool lds = k <= SEL_LDS_K;
     // 512 threads on large levels (half the serial vertices per thread), 128
     // on small ones (more workgroups over few vertices; 0.3 ms less per 128^3
