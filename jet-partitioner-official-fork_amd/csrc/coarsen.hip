@@ -361,10 +361,6 @@ int32_t map_construct(vid_t n, const vid_t* hn, vid_t* map, Arena& a, hipStream_
 
 int32_t coarsen_hec(const DGraph& g, bool uniform, uint64_t seed, int32_t level, vid_t* map, Arena& a,
                     hipStream_t s) {
-    if (team_match_fits(g.n, g.m)) {
-        const int32_t nc = coarsen_hec_team(g, uniform, seed, level, map, a, s);
-        if (nc >= 0) return nc;
-    }
     ArenaScope sc(a);
     vid_t* hn = a.alloc<vid_t>(g.n);
     hec_heavy_neighbours(g, uniform, seed, level, hn, a, s);

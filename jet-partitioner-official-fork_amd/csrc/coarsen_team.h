@@ -19,8 +19,4 @@ bool team_match_fits(int64_t n, int64_t m);
 int32_t coarsen_match_team(const DGraph& g, bool uniform, uint64_t seed, int32_t level, bool two_hop, vid_t* map,
                            Arena& a, hipStream_t s);
 
-// coarsen_hec in one launch, for the same levels; likewise.
-int32_t coarsen_hec_team(const DGraph& g, bool uniform, uint64_t seed, int32_t level, vid_t* map, Arena& a,
-                         hipStream_t s);
-
 }  // namespace jet

@@ -40,7 +40,6 @@ struct MatchCtl {
     TeamCtl team;
     int32_t left[2], pad1[30];  // work-list lengths of alternate passes
     int32_t unmatched[3], total[3], nbig[3], pad2[23];
-    unsigned long long vwsum;  // HEC: the level's vertex weight
 };
 
 struct MatchParams {
@@ -82,50 +81,6 @@ __device__ inline void cm_publish(const MatchParams& P, int64_t nc) {
     __threadfence_system();
     P.host_out[1] = P.seq;  // the host waits for this word
     __threadfence_system();
-}
-
-// The coarse ids: roots (vcmap[i] == i) in increasing id, everyone its root's
-// (heuristics.hpp:147-165). singles: a vertex still without a match is a root.
-template <class OWN>
-__device__ inline bool cm_number(const MatchParams& P, MatchShared& L, Team& team, OWN&& for_own, bool singles,
-                                 int32_t& nc) {
-    const int t = threadIdx.x;
-    const int lane = t & (WAVE - 1);
-    const int32_t nchunks = (P.g.n + WAVE - 1) / WAVE;
-    for_own([&](int32_t, vid_t i, bool in) {
-        vid_t c = in ? ld_rx(&P.vcmap[i]) : -1;
-        if (singles && c == ORD_MAX) {
-            c = i;
-            P.vcmap[i] = i;
-        }
-        const uint64_t m = __ballot(in && c == i);
-        if (lane == 0) P.csum[i / WAVE] = (int32_t)__popcll(m);
-    });
-    if (!team.sync()) return false;
-    const int32_t v = t < nchunks ? ld_rx(&P.csum[t]) : 0;
-    const int32_t pre = block_excl_scan<int32_t, CM_BLOCK>(v, nc, L.red);
-    if (t < nchunks) L.pre[t] = pre;
-    __syncthreads();
-    // claim[] takes the roots' ids
-    for_own([&](int32_t, vid_t i, bool in) {
-        const bool root = in && ld_rx(&P.vcmap[i]) == i;
-        const uint64_t m = __ballot(root);
-        if (root) P.claim[i] = L.pre[i / WAVE] + (int32_t)__popcll(m & ((1ull << lane) - 1ull));
-    });
-    if (!team.sync()) return false;
-    for_own([&](int32_t, vid_t i, bool in) {
-        if (in) P.map[i] = ld_rx(&P.claim[ld_rx(&P.vcmap[i])]);
-    });
-    return true;
-}
-
-// Heavy-neighbour choice: max weight, then the last edge among equal ones
-// (hec_better in coarsen.hip).
-__device__ inline void cm_hec_better(int64_t& bw, int64_t& bj, int64_t w, int64_t j) {
-    if (w > bw || (w == bw && j > bj)) {
-        bw = w;
-        bj = j;
-    }
 }
 
 }  // namespace
@@ -482,164 +437,35 @@ __global__ void __launch_bounds__(CM_BLOCK) k_match_team(MatchParams P) {
     // ------------------------------------------------------------ ids (:147-165, :650-665)
     // roots get dense ids in increasing order; unmatched vertices are roots
     int32_t nc = 0;
-    if (alive) alive = cm_number(P, L, team, for_own, true, nc);
-    if (me == 0 && t == 0) cm_publish(P, alive && !ld_rx(&C->team.fail) ? nc : -2);
-}
-
-// Heavy edge coarsening of a level (hec_heavy_neighbours and map_construct in
-// coarsen.hip) in one launch: the same rounds (mark, claim, resolve, next) over
-// each workgroup's own part of the work list, where the kernels take about
-// eighteen launches and four host reads.
-// Measured on a stencil of 871,933 vertices (22 levels, 17 of them here):
-// mapping 4.7 ms with the kernels, 4.25 with the teams.
-__global__ void __launch_bounds__(CM_BLOCK) k_hec_team(MatchParams P) {
-    __shared__ MatchShared L;
-    __shared__ vid_t list[2][TEAM_OWN];  // the work list's own vertices, this round's and the next's
-    const DGraph g = P.g;
-    const vid_t n = g.n;
-    const int t = threadIdx.x;
-    const int lane = t & (WAVE - 1);
-    const int wv = t / WAVE;
-    MatchCtl* C = P.ctl;
-    int32_t* stamp = P.count;  // n of its entries
-    if (t == 0) {
-        const int32_t st = team_start(C->team, P.xcd, P.team, ceil_div_dev(n, TEAM_OWN), L.go, L.size, L.me);
-        if (st == TEAM_ABANDON) cm_publish(P, -1);
-        L.n0 = L.n1 = 0;
-    }
-    __syncthreads();
-    if (!L.go) return;
-    const int32_t T = L.size, me = L.me;
-    Team team{&C->team, T, me, 0, &L.go};
-    auto for_own = [&](auto&& f) {
-        for (int32_t x0 = WAVE * wv;; x0 += WAVE * CM_WAVES) {
-            if (own_vertex(x0, WAVE, T, me) >= n) break;
-            const int64_t i = own_vertex(x0 + lane, WAVE, T, me);
-            f(x0 + lane, (vid_t)i, i < n);
-        }
-    };
-    // ------------------------------------------------------------ heavy neighbours
-    int64_t vs = 0;
-    for_own([&](int32_t x, vid_t i, bool in) {
-        if (in) {
-            list[0][x] = i;
-            P.vcmap[i] = ORD_MAX;
-            stamp[i] = 0;
-            P.claim[i] = ORD_MAX;
-            vs += g.vw[i];
-            if (P.uniform) {
-                const uint64_t r = rng(P.seed, (uint32_t)P.level, SITE_HEC, 0, (uint32_t)i);
-                const eoff_t s0 = g.rowptr[i];
-                const int64_t deg = g.rowptr[i + 1] - s0;
-                P.hn[i] = deg > 0 ? g.col[s0 + (int64_t)(r % (uint64_t)deg)] : (vid_t)(r % (uint64_t)n);
+    if (alive) {
+        for_own([&](int32_t, vid_t i, bool in) {
+            vid_t c = in ? ld_rx(&P.vcmap[i]) : -1;
+            if (c == ORD_MAX) {
+                c = i;
+                P.vcmap[i] = i;
             }
-        }
-        const uint64_t m = __ballot(in);
-        if (lane == 0 && m) atomicAdd(&L.n0, (int32_t)__popcll(m));
-    });
-    bool alive = true;
-    if (!P.uniform) {
-        vs = wave_reduce_sum(vs);
-        if (lane == 0 && vs) atomicAdd(&C->vwsum, (unsigned long long)vs);
+            const uint64_t m = __ballot(in && c == i);
+            if (lane == 0) P.csum[i / WAVE] = (int32_t)__popcll(m);
+        });
         alive = team.sync();
     }
-    __syncthreads();
-    int32_t len = L.n0;
-    if (alive && !P.uniform) {
-        const int64_t max_allowed = 6 * (int64_t)ldr64(reinterpret_cast<const uint64_t*>(&C->vwsum)) / n;
-        auto best = [&](vid_t u, int sub, int lanes, int64_t& bw, int64_t& bj) {
-            const eoff_t re = g.rowptr[u + 1];
-            for (eoff_t j = g.rowptr[u] + sub; j < re; j += lanes)
-                if (g.vw[g.col[j]] < max_allowed) cm_hec_better(bw, bj, g.ew[j], j);
-        };
-        auto reduce = [&](int lanes, int64_t& bw, int64_t& bj) {
-            for (int d = 1; d < lanes; d <<= 1) {
-                const int64_t ow = __shfl_xor(bw, d, WAVE), oj = __shfl_xor(bj, d, WAVE);
-                cm_hec_better(bw, bj, ow, oj);
-            }
-        };
-        const int G = P.lanes, sub = t & (G - 1);
-        for (int32_t x0 = 0; x0 < len; x0 += CM_BLOCK / G) {
-            const int32_t x = x0 + t / G;
-            const vid_t u = x < len ? list[0][x] : 0;
-            const bool go = x < len && g.rowptr[u + 1] - g.rowptr[u] <= P.big_deg;
-            int64_t bw = INT64_MIN, bj = -1;
-            if (go && g.vw[u] < max_allowed) best(u, sub, G, bw, bj);
-            reduce(G, bw, bj);
-            if (go && sub == 0) P.hn[u] = bj >= 0 ? g.col[bj] : u;
-        }
-        for (int32_t x = wv; x < len; x += CM_WAVES) {
-            const vid_t u = list[0][x];
-            if (g.rowptr[u + 1] - g.rowptr[u] <= P.big_deg) continue;
-            int64_t bw = INT64_MIN, bj = -1;
-            if (g.vw[u] < max_allowed) best(u, lane, WAVE, bw, bj);
-            reduce(WAVE, bw, bj);
-            if (lane == 0) P.hn[u] = bj >= 0 ? g.col[bj] : u;
-        }
-    }
-    if (alive) alive = team.sync();
-
-    // ------------------------------------------------------------ map construction
-    int cur = 0, swap = 1;
-    auto acting = [&](vid_t u, vid_t h) { return (((u < h) ? 1 : 0) ^ swap) != 0; };
-    for (int32_t round = 0; alive; round++) {
-        if (round > 2 * n + 8) {  // each round resolves at least one vertex
-            alive = false;
-            break;
-        }
-        const vid_t* wl = list[cur];
-        if (swap == 0) {
-            for (int32_t x = t; x < len; x += CM_BLOCK) {
-                const vid_t u = wl[x], v = ld_rx(&P.hn[u]);
-                if (u < v && ld_rx(&stamp[v]) == round && !(v < ld_rx(&P.hn[v]))) atomicMin(&P.claim[v], u);
-            }
-            if (!(alive = team.sync())) break;
-        }
-        for (int32_t x = t; x < len; x += CM_BLOCK) {
-            const vid_t u = wl[x], v = ld_rx(&P.hn[u]);
-            if (!acting(u, v)) continue;
-            if (v == u) {
-                P.vcmap[u] = u;
-            } else if (ld_rx(&stamp[v]) == round) {
-                if (acting(v, ld_rx(&P.hn[v]))) {
-                    P.vcmap[u] = ORD_MAX;
-                } else {
-                    const vid_t cv = swap ? v : ld_rx(&P.claim[v]);
-                    P.vcmap[u] = cv;
-                    P.vcmap[v] = cv;
-                }
-            } else {
-                P.vcmap[u] = ld_rx(&P.vcmap[v]);
-            }
-        }
-        if (t == 0) L.n1 = 0;
-        if (!(alive = team.sync())) break;
-        // the next round's list and marks
-        vid_t* next = list[cur ^ 1];
-        for (int32_t x0 = 0; x0 < len; x0 += CM_BLOCK) {
-            const int32_t x = x0 + t;
-            const vid_t u = x < len ? wl[x] : 0;
-            const bool keep = x < len && ld_rx(&P.vcmap[u]) >= n;
-            const int32_t at = wave_append(&L.n1, keep);
-            if (at >= 0) {
-                next[at] = u;
-                stamp[u] = round + 1;
-                P.claim[u] = ORD_MAX;
-            }
-        }
+    if (alive) {
+        const int32_t v = t < nchunks ? ld_rx(&P.csum[t]) : 0;
+        const int32_t pre = block_excl_scan<int32_t, CM_BLOCK>(v, nc, L.red);
+        if (t < nchunks) L.pre[t] = pre;
         __syncthreads();
-        len = L.n1;
-        if (t == 0) {
-            if (len) atomicAdd(&C->total[round % 3], len);
-            if (me == 0) __hip_atomic_store(&C->total[(round + 1) % 3], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        if (!(alive = team.sync())) break;
-        if (ld_rx(&C->total[round % 3]) == 0) break;
-        cur ^= 1;
-        swap ^= 1;
+        // claim[] takes the roots' ids
+        for_own([&](int32_t, vid_t i, bool in) {
+            const bool root = in && ld_rx(&P.vcmap[i]) == i;
+            const uint64_t m = __ballot(root);
+            if (root) P.claim[i] = L.pre[i / WAVE] + (int32_t)__popcll(m & ((1ull << lane) - 1ull));
+        });
+        alive = team.sync();
     }
-    int32_t nc = 0;
-    if (alive) alive = cm_number(P, L, team, for_own, false, nc);
+    if (alive)
+        for_own([&](int32_t, vid_t i, bool in) {
+            if (in) P.map[i] = ld_rx(&P.claim[ld_rx(&P.vcmap[i])]);
+        });
     if (me == 0 && t == 0) cm_publish(P, alive && !ld_rx(&C->team.fail) ? nc : -2);
 }
 
@@ -649,8 +475,8 @@ bool team_match_fits(int64_t n, int64_t m) {
     return n >= 1 && n <= std::min<int64_t>(max_n, TEAM_MAX_N) && m <= TEAM_MATCH_M;
 }
 
-static int32_t launch_team(bool hec, const DGraph& g, bool uniform, uint64_t seed, int32_t level, bool two_hop,
-                           vid_t* map, Arena& a, hipStream_t s) {
+int32_t coarsen_match_team(const DGraph& g, bool uniform, uint64_t seed, int32_t level, bool two_hop, vid_t* map,
+                           Arena& a, hipStream_t s) {
     ArenaScope sc(a);
     const int64_t n = g.n, nchunks = ceil_div(n, (int64_t)WAVE);
     MatchParams P{};
@@ -686,22 +512,12 @@ static int32_t launch_team(bool hec, const DGraph& g, bool uniform, uint64_t see
     TeamSlot slot(P.team);
     P.xcd = slot.xcd();
     k_match_prep<<<1, 256, 0, s>>>(P.ctl);
-    (hec ? k_hec_team : k_match_team)<<<P.team == 1 ? 1 : 8 * P.team, CM_BLOCK, 0, s>>>(P);
+    k_match_team<<<P.team == 1 ? 1 : 8 * P.team, CM_BLOCK, 0, s>>>(P);
     JET_LAUNCH_CHECK();
     if (!wait_mailbox(&out[1], P.seq, s)) return -1;  // no workgroup ran on the wanted XCD
     const int64_t nc = out[0];
-    if (nc == -2) throw DeviceError(hec ? "map construction made no progress" : "matching made no progress");
+    if (nc == -2) throw DeviceError("matching made no progress");
     return (int32_t)nc;
-}
-
-int32_t coarsen_match_team(const DGraph& g, bool uniform, uint64_t seed, int32_t level, bool two_hop, vid_t* map,
-                           Arena& a, hipStream_t s) {
-    return launch_team(false, g, uniform, seed, level, two_hop, map, a, s);
-}
-
-int32_t coarsen_hec_team(const DGraph& g, bool uniform, uint64_t seed, int32_t level, vid_t* map, Arena& a,
-                         hipStream_t s) {
-    return launch_team(true, g, uniform, seed, level, false, map, a, s);
 }
 
 }  // namespace jet
