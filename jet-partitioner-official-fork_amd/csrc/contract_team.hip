@@ -433,7 +433,9 @@ bool contract_team(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, 
     P.g = g;
     P.map = map;
     P.nc = nc;
-    P.team = (int32_t)std::max<int64_t>(1, std::min<int64_t>(TEAM_MAX, ceil_div((int64_t)nc, CT_ROWS_WG)));
+    // at most CT_ROWS fine vertices each, too
+    P.team = (int32_t)std::max<int64_t>(ceil_div((int64_t)g.n, (int64_t)CT_ROWS),
+                                        std::min<int64_t>(TEAM_MAX, ceil_div((int64_t)nc, CT_ROWS_WG)));
     P.rows = (int32_t)ceil_div((int64_t)nc, (int64_t)P.team);
     if (P.rows > CT_ROWS || ceil_div((int64_t)g.n, (int64_t)P.team * WAVE) * WAVE > CT_ROWS)
         throw DeviceError("team contraction: level outside the kernel's limits");

@@ -58,3 +58,15 @@ def test_coarse_rows_without_members():
     n = 2000
     g = graphs.from_edges(n, np.arange(n - 1), np.arange(1, n), np.ones(n - 1, dtype=np.int64))
     check(g, (3 * (np.arange(n) // 3)).astype(np.int32), n)
+
+
+@pytest.mark.parametrize("n,nc", [(2048, 1), (2049, 1), (5000, 3), (30000, 64), (65536, 65), (65536, 1)])
+def test_few_coarse_rows_of_many_vertices(n, nc):
+    # hardly an edge: the fine vertices, not the rows, ask for workgroups
+    rs = np.random.default_rng(n + nc)
+    e = min(32 * nc, n // 2)
+    u = rs.permutation(n)
+    g = graphs.from_edges(n, u[:e], u[e : 2 * e], rs.integers(1, 9, e))
+    mp = rs.integers(0, nc, n).astype(np.int32)
+    print("few rows", n, nc, flush=True)
+    check(g, mp, nc)
