@@ -19,7 +19,7 @@ from collections import defaultdict
 FAMILY_OF = [
     (re.compile(r"\bk_lp_select\b"), "lp_select"),
     (re.compile(r"\bk_afterburner_"), "afterburner"),
-    (re.compile(r"\bk_update_(small|big|hubs)\b"), "update"),
+    (re.compile(r"\bk_(update_(small|big)|pull_hubs)\b"), "update"),
     (re.compile(r"\bk_weak_select\b"), "weak_select"),
 ]
 
