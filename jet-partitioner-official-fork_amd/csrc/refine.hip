@@ -2778,10 +2778,13 @@ void Refiner::rebalance(const Level& L, const part_t* part, const int64_t* sizes
     // one copy per sel_copy_wgs workgroups (256 by default): fewer
     // workgroups meet on a line, and a copy costs a pass of the fold
     // With few parts every workgroup adds to every bucket, and the atomics of
-    // all workgroups meet on each line (10 ns each): a copy per 16 k workgroups.
-    // Stencil levels of 136,971 and 254,104 vertices: k = 2 42 -> 34 and 36 ->
-    // 34 us an iteration, k = 4 47 -> 40 and 67 -> 45, k = 8 43 -> 40 and 49 -> 45.
-    const int64_t copy_wgs = std::min<int64_t>(tuning().sel_copy_wgs, std::max<int64_t>(32, 16 * (int64_t)k));
+    // all workgroups meet on each line (10 ns each): up to 64 parts a copy per
+    // 32 to 64 workgroups. Stencil levels of 136,971 and 254,104 vertices with a
+    // copy per 256 and now: k = 2 42 and 34, 36 and 34 us an iteration, k = 4
+    // 47 and 40, 67 and 45, k = 30 43 and 42, 52 and 49; 2,097,152 vertices with
+    // k = 32 77 and 75, k = 64 79 and 76, but k = 256 94 and 97.
+    const int64_t copy_wgs =
+        std::min<int64_t>(tuning().sel_copy_wgs, k > 64 ? INT64_MAX : std::min<int64_t>(64, std::max<int64_t>(32, 16 * (int64_t)k)));
     const int32_t copies = std::max(1, std::min<int32_t>(ncopies_, (int32_t)(nsel / copy_wgs)));
     const bool lds = k <= SEL_LDS_K;
     // 512 threads on large levels (half the serial vertices per thread), 128
