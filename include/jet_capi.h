@@ -381,11 +381,10 @@ int jet_partition_batch(jet_ctx_t* ctx, int32_t count, const jet_config_t* cfgs,
  * defaults stay. Names:
  * "wg_max_n": levels of up to this many vertices (and at most 65536) are
  *   refined in one launch, by a team of workgroups on one XCD (0 = never);
- * "batch_wg_max_n": for jobs of jet_partition_batch and jet_submit on contexts
- *   of at least 8 workers, levels of up to this many vertices are refined by
- *   one workgroup each, those of concurrent jobs launched together (0 =
- *   never, the default);
- * "wg_big_deg": in both kernels, items above this degree take a whole wave;
+ * "batch_wg_max_n": accepted and without effect (the path it selected, levels
+ *   of concurrent jobs refined by one workgroup each, is closed);
+ * "wg_big_deg": in that team's kernel, items above this degree take a whole
+ *   wave;
  * "small_level_n": levels treated as small (wave-built connectivity rows,
  *   wider afterburner lane groups, 128-thread rebalancer select workgroups);
  * "ab_lanes_small", "upd_lanes": lane-group multipliers (1-4) of the

@@ -21,9 +21,7 @@
 
 #include "coarsen_rules.h"
 #include "prims.h"
-#include "refine_team.h"
 #include "team_dev.h"
-#include "tuning.h"
 #include "wave.h"
 
 namespace jet {
@@ -471,8 +469,7 @@ __global__ void __launch_bounds__(CM_BLOCK) k_match_team(MatchParams P) {
 
 // ---------------------------------------------------------------- host side
 bool team_match_fits(int64_t n, int64_t m) {
-    const int64_t max_n = wg_collector() ? std::min<int64_t>(tuning().wg_max_n, TEAM_BATCH_N) : tuning().wg_max_n;
-    return n >= 1 && n <= std::min<int64_t>(max_n, TEAM_MAX_N) && m <= TEAM_MATCH_M;
+    return n >= 1 && n <= team_max_n() && m <= TEAM_MATCH_M;
 }
 
 int32_t coarsen_match_team(const DGraph& g, bool uniform, uint64_t seed, int32_t level, bool two_hop, vid_t* map,

@@ -24,9 +24,7 @@
 
 #include "contract_dev.h"
 #include "prims.h"
-#include "refine_team.h"
 #include "team_dev.h"
-#include "tuning.h"
 #include "wave.h"
 
 namespace jet {
@@ -410,8 +408,7 @@ __global__ void __launch_bounds__(CT_BLOCK) k_contract_team(ContractParams P) {
 
 // ---------------------------------------------------------------- host side
 bool team_contract_fits(int64_t n, int64_t m, int64_t nc) {
-    const int64_t max_n = wg_collector() ? std::min<int64_t>(tuning().wg_max_n, TEAM_BATCH_N) : tuning().wg_max_n;
-    return n >= 1 && nc >= 1 && m >= 1 && n <= std::min<int64_t>(max_n, TEAM_MAX_N) && nc <= n && m <= CT_TEAM_M &&
+    return n >= 1 && nc >= 1 && m >= 1 && n <= team_max_n() && nc <= n && m <= CT_TEAM_M &&
            m <= CT_TEAM_AVG * nc;
 }
 

@@ -7,7 +7,6 @@
 #include "contract.h"
 #include "jet_types.h"
 #include "refine_team.h"
-#include "refine_wg.h"
 
 namespace jet {
 
@@ -79,9 +78,6 @@ class Refiner {
     // jet_refine on one level by a team of workgroups of one XCD (small
     // levels); false when no team could start (nothing was changed)
     bool refine_team(const Level& L, part_t* best_part, const std::vector<double>& temps, LevelRecord& rec);
-    // jet_refine on one level by the graph-tagged one-workgroup kernel (the
-    // batched and served layer's collector)
-    LevelRecord refine_wg(const Level& L, part_t* best_part, const std::vector<double>& temps);
     void init_conn(const Level& L, const part_t* part, const int32_t* mark);
     void build_tiers(const Level& L);
     void build_slices(const Level& L);
@@ -190,9 +186,6 @@ class Refiner {
     int64_t* bcopies_ = nullptr;  // ncopies_ - 1 more bucket arrays, kept zero between uses
     int32_t ncopies_ = 1;
     int64_t nbuckets_ = 0;
-    WgState* wg_state_ = nullptr;  // the one-workgroup kernel's controller state
-    vid_t* wg_list_ = nullptr;     // its ranked-member list (n)
-    int32_t* wg_runb_ = nullptr;   // its per-bucket running weights (WG_MAX_NBK)
     // the team kernel's tables (rows at their adjacency's offset), control
     // words and scratch
     int2* team_conn_ = nullptr;

@@ -2496,9 +2496,6 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     bcopies_ = a.alloc<int64_t>(std::max<int64_t>(1, nbuckets_ * (ncopies_ - 1)));
     moved_bits_ = a.alloc<uint32_t>((N + 31) / 32);
     cand_bits_ = a.alloc<uint64_t>((N + WAVE - 1) / WAVE);
-    wg_state_ = a.alloc<WgState>(1);
-    wg_list_ = a.alloc<vid_t>(N);
-    wg_runb_ = a.alloc<int32_t>(WG_MAX_NBK + 1);
     team_conn_ = a.alloc<int2>(TEAM_MAX_M);
     team_ctl_ = a.alloc<RefineCtl>(1);
     team_buckets_ = a.alloc<int32_t>(TEAM_MAX_NBK + 1);
@@ -2981,13 +2978,10 @@ LevelRecord Refiner::refine(const Level& L, part_t* best_part) {
         temps.push_back(0.75);
     }
     const RebalanceShape wr = rebalance_shape(g.n, false);
-    const bool tagged = !trace && wg_collector() && wg_fits(g.n, k, wr.nbk, tuning().batch_wg_max_n) &&
-                        (int)temps.size() <= WG_MAX_TEMPS;
     // the kernel families are measured, and iterations traced, on the
     // multi-kernel path
-    const int64_t team_n = wg_collector() ? std::min<int64_t>(tuning().wg_max_n, TEAM_BATCH_N) : tuning().wg_max_n;
-    if (!tagged && !trace && !prof_active() && team_fits(g.n, g.m, k, wr.nbk, team_n) &&
-        (int)temps.size() <= WG_MAX_TEMPS && !(team_irregular_ && g.m > TEAM_REGULAR_M)) {
+    if (!trace && !prof_active() && team_fits(g.n, g.m, k, wr.nbk, team_max_n()) &&
+        (int)temps.size() <= TEAM_MAX_TEMPS && !(team_irregular_ && g.m > TEAM_REGULAR_M)) {
         LevelRecord rec;
         if (refine_team(L, best_part, temps, rec)) {
             rec.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
@@ -3004,11 +2998,6 @@ LevelRecord Refiner::refine(const Level& L, part_t* best_part) {
     build_tiers(L);
     build_slices(L);
     init_conn(L, cur_part_, nullptr);
-    if (tagged) {
-        LevelRecord rec = refine_wg(L, best_part, temps);
-        rec.seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-        return rec;
-    }
     LevelRecord rec;
     int balance_counter = 0;
     for (double fr : temps) {
@@ -3130,10 +3119,10 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
     launch_refine_team(P, s_);
     if (!wait_mailbox(&out[TEAM_OUT_WORDS], P.seq, s_)) return false;  // no workgroup ran on the wanted XCD
     const int64_t status = out[5], err = out[6];
-    if (status == WG_IRREGULAR) team_irregular_ = true;
-    if (status == WG_ABANDONED || status == WG_IRREGULAR) return false;
+    if (status == LEVEL_IRREGULAR) team_irregular_ = true;
+    if (status == LEVEL_ABANDONED || status == LEVEL_IRREGULAR) return false;
     if (err) throw DeviceError(refine_error_text((int32_t)err));
-    if (status != WG_DONE) throw DeviceError("team refinement made no progress");
+    if (status != LEVEL_DONE) throw DeviceError("team refinement made no progress");
     cut_ = out[0];
     total_imb_ = out[1];
     rec.iterations = (int32_t)out[2];
@@ -3145,73 +3134,6 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
     rec.n = g.n;
     rec.m = g.m;
     return true;
-}
-
-// The level's iterations in the graph-tagged one-workgroup kernel
-// (csrc/refine_wg.hip), from the tables init_conn built. The kernel stops
-// early only when a step chose update_large: the marked rows are then rebuilt
-// here, by the same multi-workgroup build as flush_rebuild, and the kernel
-// continues.
-LevelRecord Refiner::refine_wg(const Level& L, part_t* best_part, const std::vector<double>& temps) {
-    DGraph g = L.view();
-    const int32_t k = p_.k;
-    const RebalanceShape weak = rebalance_shape(g.n, false), strong = rebalance_shape(g.n, true);
-    WgParams P{};
-    P.g = g;
-    P.k = k;
-    P.big_deg = (int32_t)tuning().wg_big_deg;
-    P.lanes = group_for_avg(g);  // the average degree rounded up to a power of two (4-64)
-    P.sections = weak.sections;
-    P.nbk = (int32_t)weak.nbk;
-    P.opt = opt_;
-    P.size_max = size_max_;
-    P.imb_max = (int64_t)size_max_ - opt_;
-    P.max_dest_weak = weak.max_dest;
-    P.max_dest_strong = strong.max_dest;
-    P.tol = p_.tol;
-    P.ntemps = (int32_t)temps.size();
-    for (size_t i = 0; i < temps.size(); i++) P.temps[i] = temps[i];
-    P.part = cur_part_;
-    P.best_part = best_part;
-    P.conn_off = conn_off_;
-    P.conn = conn_;
-    P.conn_size = conn_size_;
-    P.dest_cache = dest_cache_;
-    P.lock = lock_;
-    P.gain_p = gain_p_;
-    P.pregain = pregain_;
-    P.dest = dest_;
-    P.bid = bid_;
-    P.cand = cand_;
-    P.moves = moves_;
-    P.rlist = wg_list_;
-    P.score = score_;
-    P.mark = swap_bit_;
-    P.runb = wg_runb_;
-    P.curr_sizes = curr_sizes_;
-    P.best_sizes = best_sizes_;
-    P.st = wg_state_;
-    wg_init_state(wg_state_, cut_, total_imb_, s_);
-    WgState h{};
-    for (int launches = 0;; launches++) {
-        if (launches > 100000) throw DeviceError("one-workgroup refinement made no progress");
-        wg_collector()->run(P, s_, h);  // graph-tagged with the levels of other jobs
-        if (h.err) throw DeviceError(refine_error_text(h.err));
-        if (h.status == WG_STALLED) throw DeviceError("one-workgroup refinement exceeded its iteration bound");
-        if (h.status != WG_REBUILD) break;
-        init_conn(L, cur_part_, swap_bit_);  // update_large's rebuild of the marked rows
-    }
-    if (h.changed) changed_ = true;
-    cut_ = h.best_cut;
-    total_imb_ = h.best_imb;
-    LevelRecord rec;
-    rec.iterations = h.iterations;
-    rec.lp_iterations = h.lp_iterations;
-    rec.cut2 = cut_;
-    rec.total_imb = total_imb_;
-    rec.n = g.n;
-    rec.m = g.m;
-    return rec;
 }
 
 void Refiner::single_step(const Level& L, const part_t* part, int kind, double fr, std::vector<int32_t>& moves,

@@ -3,21 +3,21 @@
 #include <hip/hip_runtime.h>
 
 #include "jet_types.h"
-#include "refine_wg.h"
 #include "team.h"
 
 namespace jet {
 
-// Jobs of contexts of many workers use teams on levels of up to this many
-// vertices: a team kernel holds one of the process's four hardware queues for
-// the whole level, and the workgroups of its launch that fall on an XCD where
-// another team runs wait for a free CU. 60 mixed graphs on 16 workers: 298-312
-// ms without teams, 284 up to 512 vertices, 275 up to 2048, 268-273 up to
-// 4096, 287 up to 8192, 342 up to 65,536.
-constexpr int32_t TEAM_BATCH_N = 4096;
 constexpr int64_t TEAM_MAX_M = 600000;
 constexpr int32_t TEAM_MAX_K = 256;
 constexpr int32_t TEAM_MAX_NBK = 16384;
+constexpr int TEAM_MAX_TEMPS = 20;
+
+// Controller state of jet_refine (jet_refiner.hpp:1079-1134).
+struct LevelState {
+    int64_t curr_cut, curr_imb, best_cut, best_imb;
+    int32_t temp_idx, count, balance_counter, iterations, lp_iterations;
+    int32_t changed, status;
+};
 
 // Device words the level's team shares: the team's own, and the step's sums.
 struct RefineCtl {
@@ -37,7 +37,7 @@ struct TeamParams {
     int64_t opt, size_max, imb_max, max_dest_weak, max_dest_strong;
     double tol;
     int32_t ntemps;
-    double temps[WG_MAX_TEMPS];
+    double temps[TEAM_MAX_TEMPS];
     int64_t cut, imb;  // of the partition the level starts from
     part_t* part;
     part_t* best_part;  // in: the level's partition; out: the best one
@@ -76,11 +76,11 @@ bool team_fits(int64_t n, int64_t m, int32_t k, int64_t nbk, int64_t max_n);
 int32_t team_size(int64_t n, int64_t m);
 // Clears the control words and the bucket sums and copies the best part sizes
 // to the current ones, then runs the level, on stream s. The result words are
-// published to p.host_out; status WG_ABANDONED (or a finished stream without a
-// result) means that no team could start: the level's arrays are untouched.
-// WG_IRREGULAR: the level has rows of more than TEAM_MAX_DEG edges, and too
+// published to p.host_out; status LEVEL_ABANDONED (or a finished stream without
+// a result) means that no team could start: the level's arrays are untouched.
+// LEVEL_IRREGULAR: the level has rows of more than TEAM_MAX_DEG edges, and too
 // many edges (likewise nothing has changed).
-enum : int32_t { WG_ABANDONED = 3, WG_IRREGULAR = 4 };
+enum : int32_t { LEVEL_DONE = 0, LEVEL_STALLED = 2, LEVEL_ABANDONED = 3, LEVEL_IRREGULAR = 4 };
 void launch_refine_team(TeamParams p, hipStream_t s);
 
 }  // namespace jet

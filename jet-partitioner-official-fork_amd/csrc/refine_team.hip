@@ -69,7 +69,7 @@ struct TeamShared {
     int32_t done;
     int64_t counter;
     int64_t cc;
-    WgState S;
+    LevelState S;
 };
 
 __device__ inline int2 ldr_slot(const int2* p) {
@@ -237,21 +237,21 @@ __device__ inline int32_t tm_walk(const int64_t* es, int32_t lo, int32_t hi, int
 // The next step of the temperature loop of :1095-1134: `for (fr : temps) {
 // count = 0; while (count++ <= 11) ... }` as the state (temp_idx, count).
 __device__ inline void tm_next_step(TeamShared& L, int32_t ntemps) {
-    WgState& S = L.S;
+    LevelState& S = L.S;
     if (S.count > 11) {
         S.temp_idx++;
         S.count = 0;
     }
     L.done = S.temp_idx >= ntemps ? 1 : 0;
     if (!L.done && S.iterations >= TM_ITER_CAP) {
-        S.status = WG_STALLED;
+        S.status = LEVEL_STALLED;
         L.done = 1;
     }
     S.count++;
     if (!L.done) S.iterations++;
 }
 
-__device__ inline void tm_publish(const TeamParams& P, const WgState& S, int32_t err) {
+__device__ inline void tm_publish(const TeamParams& P, const LevelState& S, int32_t err) {
     P.host_out[0] = S.best_cut;
     P.host_out[1] = S.best_imb;
     P.host_out[2] = S.iterations;
@@ -292,14 +292,14 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
     // ------------------------------------------------------------ start-up
     if (t == 0) {
         const int32_t st = team_start(C->team, P.xcd, P.team, ceil_div_dev(n, TEAM_OWN), L.go, L.size, L.me);
-        WgState S{};
+        LevelState S{};
         if (st == TEAM_ABANDON) {
-            S.status = WG_ABANDONED;
+            S.status = LEVEL_ABANDONED;
             tm_publish(P, S, 0);
         }
         S.curr_cut = S.best_cut = P.cut;
         S.curr_imb = S.best_imb = P.imb;
-        S.status = WG_DONE;
+        S.status = LEVEL_DONE;
         L.S = S;
     }
     __syncthreads();
@@ -330,7 +330,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
             const bool ok = team.sync();
             if (!ok || ld_rx(&C->max_deg) > TEAM_MAX_DEG) {
                 if (me == 0 && t == 0) {
-                    L.S.status = ok ? WG_IRREGULAR : WG_STALLED;
+                    L.S.status = ok ? LEVEL_IRREGULAR : LEVEL_STALLED;
                     tm_publish(P, L.S, 0);
                 }
                 return;
@@ -935,7 +935,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
                     C->redraws = 0;
                 }
                 L.cc = 0;
-                WgState& S = L.S;
+                LevelState& S = L.S;
                 S.curr_cut -= change;
                 S.curr_imb = mx > P.opt ? mx - P.opt : 0;
                 if (kind == 0) {
@@ -970,7 +970,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
     }
     __syncthreads();
     if (me == 0 && t == 0) {
-        if (!alive || ld_rx(&C->team.fail)) L.S.status = WG_STALLED;
+        if (!alive || ld_rx(&C->team.fail)) L.S.status = LEVEL_STALLED;
         tm_publish(P, L.S, ld_rx(err));
     }
 }
@@ -1023,7 +1023,7 @@ void launch_refine_team(TeamParams p, hipStream_t s) {
                                       hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);
     });
     JET_HIP(rc[dev]);
-    if (!team_fits(p.g.n, p.g.m, p.k, p.nbk, TEAM_MAX_N) || p.ntemps > WG_MAX_TEMPS || p.team < 1 ||
+    if (!team_fits(p.g.n, p.g.m, p.k, p.nbk, TEAM_MAX_N) || p.ntemps > TEAM_MAX_TEMPS || p.team < 1 ||
         p.team > TEAM_MAX || (int64_t)p.team * TEAM_OWN < p.g.n)
         throw DeviceError("team refinement: level outside the kernel's limits");
     // chunks of 64 vertices keep a wave's loads together; shorter ones when a

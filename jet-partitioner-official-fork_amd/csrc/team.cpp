@@ -4,9 +4,11 @@
 #include <hip/hip_runtime.h>
 #include <sched.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "jet_types.h"
+#include "tuning.h"
 
 namespace jet {
 
@@ -14,7 +16,14 @@ namespace {
 constexpr int XCDS = 8;
 std::mutex g_slot_mu;
 int32_t g_slot_load[64][XCDS];
+thread_local bool t_batch_thread = false;
 }  // namespace
+
+void set_batch_thread(bool on) { t_batch_thread = on; }
+
+int64_t team_max_n() {
+    return std::min<int64_t>(tuning().wg_max_n, t_batch_thread ? TEAM_BATCH_N : TEAM_MAX_N);
+}
 
 TeamSlot::TeamSlot(int32_t team) : team_(team) {
     int dev = 0;

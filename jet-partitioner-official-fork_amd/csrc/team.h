@@ -18,6 +18,18 @@ struct TeamCtl {
     int32_t fail, pad4[31];
 };
 
+// Jobs of contexts of many workers use teams on levels of up to this many
+// vertices: a team kernel holds one of the process's four hardware queues for
+// the whole level, and the workgroups of its launch that fall on an XCD where
+// another team runs wait for a free CU. 60 mixed graphs on 16 workers: 298-312
+// ms without teams, 284 up to 512 vertices, 275 up to 2048, 268-273 up to
+// 4096, 287 up to 8192, 342 up to 65,536.
+constexpr int32_t TEAM_BATCH_N = 4096;
+// Marks the calling thread as a worker of such a context.
+void set_batch_thread(bool on);
+// Levels of up to this many vertices may take a team on the calling thread.
+int64_t team_max_n();
+
 // A place for `team` workgroups on an XCD of the device, held while a team
 // kernel runs there: the teams in flight on an XCD never need more CUs than
 // it has, so that every team finds room for all of its workgroups. Waits

@@ -13,13 +13,13 @@ struct Tuning {
     // too many edges: team_fits) are refined in one launch by a team of
     // workgroups on one XCD (0: never)
     int64_t wg_max_n = 65536;
-    // jobs of the batched and served layer on contexts of at least
-    // BATCH_WG_MIN_WORKERS workers: levels of up to this many vertices are
-    // refined by one workgroup each, the levels of concurrent jobs in one
-    // launch (0: never)
+    // once the levels that jobs of the batched and served layer refined by one
+    // workgroup each; that path is closed (a case with levels of up to 16384
+    // vertices ended in a GPU fault of unknown cause), and the value is kept so
+    // that tables and callers that set it still work, but read by nothing
     int64_t batch_wg_max_n = 0;
-    // in both kernels, candidates and moves of higher degree are taken by a
-    // whole wave instead of a group of lanes
+    // in that kernel, candidates and moves of higher degree are taken by a whole
+    // wave instead of a group of lanes
     int64_t wg_big_deg = 32;
     // "small" levels: every connectivity row is built by a wave, the
     // afterburner takes ab_lanes_small times its lanes per candidate, and the
@@ -51,9 +51,9 @@ struct Tuning {
 };
 
 Tuning& tuning();
-// Contexts with fewer workers gather too few levels per launch for the
-// one-workgroup kernel to pay: their jobs refine as single calls do.
-constexpr int BATCH_WG_MIN_WORKERS = 8;
+// Contexts of at least this many workers hold their jobs' teams to
+// TEAM_BATCH_N vertices (team.h); jobs of smaller ones run as single calls do.
+constexpr int BATCH_MANY_WORKERS = 8;
 // Applies a tuning table (lines "name value"; '#' starts a comment). Returns
 // the number of settings applied, or -1 when the file cannot be read or holds
 // an unknown name or a value out of range (nothing is applied then).
