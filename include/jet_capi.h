@@ -383,6 +383,9 @@ int jet_partition_batch(jet_ctx_t* ctx, int32_t count, const jet_config_t* cfgs,
  *   refined in one launch, by a team of workgroups on one XCD (0 = never);
  * "batch_wg_max_n": accepted and without effect (the path it selected, levels
  *   of concurrent jobs refined by one workgroup each, is closed);
+ * "team_start_spins": polls of a team's first workgroup before it gives up
+ *   waiting for the others (0-4194304; 0: no team of more than one workgroup);
+ *   the call then takes the paths of larger levels;
  * "wg_big_deg": in that team's kernel, items above this degree take a whole
  *   wave;
  * "small_level_n": levels treated as small (wave-built connectivity rows,

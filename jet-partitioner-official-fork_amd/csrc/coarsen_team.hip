@@ -22,6 +22,7 @@
 #include "coarsen_rules.h"
 #include "prims.h"
 #include "team_dev.h"
+#include "tuning.h"
 #include "wave.h"
 
 namespace jet {
@@ -46,7 +47,7 @@ struct MatchParams {
     uint64_t seed;
     int32_t lanes;    // lanes per vertex of a neighbourhood walk: a power of two up to a wave
     int32_t big_deg;  // longer rows take a whole wave
-    int32_t team, xcd;
+    int32_t team, xcd, start_spins;
     int32_t hmask;    // hash slots - 1 (a power of two above 2 n)
     vid_t* hn;
     vid_t* vcmap;
@@ -100,7 +101,7 @@ __global__ void __launch_bounds__(CM_BLOCK) k_match_team(MatchParams P) {
     const int wv = t / WAVE;
     MatchCtl* C = P.ctl;
     if (t == 0) {
-        const int32_t st = team_start(C->team, P.xcd, P.team, ceil_div_dev(n, TEAM_OWN), L.go, L.size, L.me);
+        const int32_t st = team_start(C->team, P.xcd, P.team, ceil_div_dev(n, TEAM_OWN), P.start_spins, L.go, L.size, L.me);
         if (st == TEAM_ABANDON) cm_publish(P, -1);
         L.n0 = L.n1 = 0;
     }
@@ -508,12 +509,14 @@ int32_t coarsen_match_team(const DGraph& g, bool uniform, uint64_t seed, int32_t
     P.seq = ++mb.seq;
     TeamSlot slot(P.team);
     P.xcd = slot.xcd();
+    P.start_spins = (int32_t)tuning().team_start_spins;
     k_match_prep<<<1, 256, 0, s>>>(P.ctl);
     k_match_team<<<P.team == 1 ? 1 : 8 * P.team, CM_BLOCK, 0, s>>>(P);
     JET_LAUNCH_CHECK();
-    if (!wait_mailbox(&out[1], P.seq, s)) return -1;  // no workgroup ran on the wanted XCD
-    const int64_t nc = out[0];
+    // without a result: no workgroup ran on the wanted XCD
+    const int64_t nc = wait_mailbox(&out[1], P.seq, s) ? out[0] : -1;
     if (nc == -2) throw DeviceError("matching made no progress");
+    if (nc < 0) team_abandoned();
     return (int32_t)nc;
 }
 

@@ -25,6 +25,7 @@
 #include "contract_dev.h"
 #include "prims.h"
 #include "team_dev.h"
+#include "tuning.h"
 #include "wave.h"
 
 namespace jet {
@@ -64,7 +65,7 @@ struct ContractParams {
     DGraph g;
     const vid_t* map;
     int32_t nc, rows;  // rows of a workgroup
-    int32_t team, xcd;
+    int32_t team, xcd, start_spins;
     uint64_t* count;  // nc: fine edges (high word) and members (low word), zero at the launch
     int32_t* moff;    // nc
     vid_t* members;   // n
@@ -74,7 +75,7 @@ struct ContractParams {
     wgt_t* vw;  // zero at the launch
     char* out;  // columns, then at a multiple of 256 bytes the weights
     ContractCtl* ctl;
-    int64_t* host_out;  // coarse edges (-1 not built, -2 failed), then the sequence word
+    int64_t* host_out;  // coarse edges (-1 not built, -2 failed, -3 abandoned), then the sequence word
     int64_t seq;
 };
 
@@ -172,8 +173,8 @@ __global__ void __launch_bounds__(CT_BLOCK) k_contract_team(ContractParams P) {
     const int wv = t / WAVE;
     ContractCtl* C = P.ctl;
     if (t == 0) {
-        const int32_t st = team_start(C->team, P.xcd, P.team, P.team, L.go, L.size, L.me);
-        if (st == TEAM_ABANDON) ct_publish(P, -1);
+        const int32_t st = team_start(C->team, P.xcd, P.team, P.team, P.start_spins, L.go, L.size, L.me);
+        if (st == TEAM_ABANDON) ct_publish(P, -3);
         L.nbig = 0;
     }
     __syncthreads();
@@ -455,13 +456,15 @@ bool contract_team(const DGraph& g, const vid_t* map, vid_t nc, Arena& persist, 
     P.seq = ++mb.seq;
     TeamSlot slot(P.team);
     P.xcd = slot.xcd();
+    P.start_spins = (int32_t)tuning().team_start_spins;
     k_contract_prep<<<grid_for(nc, 256, 256), 256, 0, s>>>(P.ctl, P.count, P.vw, nc);
     k_contract_team<<<P.team == 1 ? 1 : 8 * P.team, CT_BLOCK, lds, s>>>(P);
     JET_LAUNCH_CHECK();
     const bool ran = wait_mailbox(&res[1], P.seq, s);
-    const int64_t mc = ran ? res[0] : -1;
-    if (mc < -1) throw DeviceError("team contraction made no progress");
+    const int64_t mc = ran ? res[0] : -3;
+    if (mc == -2) throw DeviceError("team contraction made no progress");
     if (mc < 0) {
+        if (mc == -3) team_abandoned();
         JET_HIP(hipStreamSynchronize(s));  // the kernel's last stores to what is released here
         persist.release(start);
         return false;

@@ -89,6 +89,7 @@ struct CallScope {
     Context& c;
     std::lock_guard<std::mutex> lk;
     explicit CallScope(Context& ctx) : c(ctx), lk(ctx.mu) {
+        team_call_begins();
         c.persist.reset();
         c.scratch.reset();
     }

@@ -3116,9 +3116,12 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
     P.team = team_size(g.n, g.m);
     TeamSlot slot(P.team);
     P.xcd = slot.xcd();
+    P.start_spins = (int32_t)tuning().team_start_spins;
     launch_refine_team(P, s_);
-    if (!wait_mailbox(&out[TEAM_OUT_WORDS], P.seq, s_)) return false;  // no workgroup ran on the wanted XCD
-    const int64_t status = out[5], err = out[6];
+    // without a result: no workgroup ran on the wanted XCD
+    const bool ran = wait_mailbox(&out[TEAM_OUT_WORDS], P.seq, s_);
+    const int64_t status = ran ? out[5] : LEVEL_ABANDONED, err = ran ? out[6] : 0;
+    if (status == LEVEL_ABANDONED) team_abandoned();
     if (status == LEVEL_IRREGULAR) team_irregular_ = true;
     if (status == LEVEL_ABANDONED || status == LEVEL_IRREGULAR) return false;
     if (err) throw DeviceError(refine_error_text((int32_t)err));

@@ -33,6 +33,7 @@ struct TeamParams {
     int32_t lanes;    // lanes per smaller item: a power of two up to a wave
     int32_t team;     // workgroups wanted
     int32_t xcd;      // the XCD they run on
+    int32_t start_spins;
     int32_t own;      // consecutive vertices of a workgroup's chunks (launch_refine_team sets it)
     int64_t opt, size_max, imb_max, max_dest_weak, max_dest_strong;
     double tol;

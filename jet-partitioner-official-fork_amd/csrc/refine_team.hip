@@ -291,7 +291,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
 
     // ------------------------------------------------------------ start-up
     if (t == 0) {
-        const int32_t st = team_start(C->team, P.xcd, P.team, ceil_div_dev(n, TEAM_OWN), L.go, L.size, L.me);
+        const int32_t st = team_start(C->team, P.xcd, P.team, ceil_div_dev(n, TEAM_OWN), P.start_spins, L.go, L.size, L.me);
         LevelState S{};
         if (st == TEAM_ABANDON) {
             S.status = LEVEL_ABANDONED;

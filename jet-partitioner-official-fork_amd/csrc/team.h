@@ -13,7 +13,7 @@ constexpr int32_t TEAM_MAX_N = TEAM_MAX * TEAM_OWN;
 struct TeamCtl {
     int32_t arrived, pad0[31];
     int32_t members, pad1[31];
-    int32_t state, pad2[31];  // 0 undecided, 1 go, 2 abandoned
+    int32_t state, pad2[31];  // 0 undecided, the team's size, or -1 (abandoned)
     uint32_t bar, pad3[31];
     int32_t fail, pad4[31];
 };
@@ -27,14 +27,23 @@ struct TeamCtl {
 constexpr int32_t TEAM_BATCH_N = 4096;
 // Marks the calling thread as a worker of such a context.
 void set_batch_thread(bool on);
-// Levels of up to this many vertices may take a team on the calling thread.
+// Levels of up to this many vertices may take a team on the calling thread (0
+// after an abandoned start).
 int64_t team_max_n();
+// An abandoned start costs the bound of its wait: something else holds the
+// XCD's CUs, and is likely to hold them for the next level too. The calling
+// thread therefore starts no further team until its entry point returns
+// (team_call_begins: the next one begins).
+void team_abandoned();
+void team_call_begins();
 
-// A place for `team` workgroups on an XCD of the device, held while a team
-// kernel runs there: the teams in flight on an XCD never need more CUs than
-// it has, so that every team finds room for all of its workgroups. Waits
-// until one is free. A team of one waits for no other workgroup and takes no
-// place.
+// A place for `team` workgroups on an XCD of the device, held from the launch
+// of a team kernel until its result is read: the teams that this process has
+// running on an XCD ask for no more CUs than it has. A team that has published
+// its result may still be storing for some microseconds, and other kernels and
+// other processes are not counted: a team then waits for a CU within the bound
+// of its start. Waits until a place is free. A team of one waits for no other
+// workgroup and takes no place.
 class TeamSlot {
   public:
     explicit TeamSlot(int32_t team);

@@ -12,12 +12,15 @@
 // kernel boundary takes 0.5 us.
 //
 // A launch starts eight workgroups (one per XCD in dispatch order) for each
-// one wanted; each reads the number of its XCD, and those elsewhere end at
-// once. The first member waits until every workgroup of the launch has
-// arrived, with a bound, and then starts the team or abandons it (the host
-// then takes the multi-kernel path): nothing waits for a workgroup that might
-// not run, and every later wait is bounded too. A team of one is launched as
-// one workgroup, on any XCD.
+// one wanted; each reads the number of its XCD, and those elsewhere end
+// whenever they run. The first member starts the team as soon as the members
+// wanted are there: it waits for nothing on the other XCDs, so two teams never
+// wait for each other's CUs. It stops waiting when every workgroup of the
+// launch has arrived (no member is to come) or the bound is reached, and then
+// starts with the members there are, or abandons the team when they are too
+// few (the host then takes the multi-kernel path). Members that come after the
+// decision end at once. Every later wait is for members of a team that runs,
+// and bounded too. A team of one is launched as one workgroup, on any XCD.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -27,8 +30,7 @@
 
 namespace jet {
 
-constexpr int32_t TEAM_START_SPINS = 1 << 19;  // some 0.1 s for every workgroup to arrive
-constexpr int32_t TEAM_SPINS = 1 << 24;        // seconds: the members are resident
+constexpr int32_t TEAM_SPINS = 1 << 24;  // seconds: the members are resident
 
 __device__ inline int64_t ldr64(const int64_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -45,12 +47,12 @@ enum : int32_t { TEAM_OUT = 0, TEAM_GO = 1, TEAM_ABANDON = 2 };
 __device__ inline int32_t ceil_div_dev(int32_t a, int32_t b) { return (a + b - 1) / b; }
 
 // Registers the calling workgroup (its thread 0) and decides: `go` becomes 1
-// for the members of a team that runs, with its size and the member's number.
-// Returns TEAM_ABANDON to the one workgroup that has to report that the team
-// was given up (it had fewer than `need` members, or not every workgroup of
-// the launch arrived in time).
-__device__ inline int32_t team_start(TeamCtl& C, int32_t xcd, int32_t wanted, int32_t need, int32_t& go, int32_t& size,
-                                     int32_t& me) {
+// for the members of a team that runs, with its size (`need` to `wanted`) and
+// the member's number. Returns TEAM_ABANDON to the one workgroup that has to
+// report that the team was given up. max_spins: polls of the first member
+// before it decides with the members there are (0: never a team).
+__device__ inline int32_t team_start(TeamCtl& C, int32_t xcd, int32_t wanted, int32_t need, int32_t max_spins,
+                                     int32_t& go, int32_t& size, int32_t& me) {
     if (wanted == 1) {  // launched alone, on whichever XCD
         go = size = 1;
         me = 0;
@@ -66,18 +68,18 @@ __device__ inline int32_t team_start(TeamCtl& C, int32_t xcd, int32_t wanted, in
     if (!here || m >= wanted) return TEAM_OUT;
     int32_t st = 0, spins = 0;
     if (m == 0) {
-        while (ld_rx(&C.arrived) < (int32_t)gridDim.x && ++spins <= TEAM_START_SPINS) {
+        while (ld_rx(&C.members) < wanted && ld_rx(&C.arrived) < (int32_t)gridDim.x && ++spins <= max_spins) {
         }
-        const bool all = ld_rx(&C.arrived) >= (int32_t)gridDim.x;
-        st = all && min(ld_rx(&C.members), wanted) >= need ? TEAM_GO : TEAM_ABANDON;
+        const int32_t there = min(ld_rx(&C.members), wanted);
+        st = there >= need && max_spins > 0 ? there : -1;
         __hip_atomic_store(&C.state, st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     } else {
         while ((st = ld_rx(&C.state)) == 0 && ++spins <= TEAM_SPINS) {
         }
     }
-    if (st == TEAM_GO) {
+    if (st > m) {
         go = 1;
-        size = min(ld_rx(&C.members), wanted);
+        size = st;
         me = m;
         return TEAM_GO;
     }

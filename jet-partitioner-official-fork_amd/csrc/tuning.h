@@ -18,9 +18,12 @@ struct Tuning {
     // vertices ended in a GPU fault of unknown cause), and the value is kept so
     // that tables and callers that set it still work, but read by nothing
     int64_t batch_wg_max_n = 0;
-    // in that kernel, candidates and moves of higher degree are taken by a whole
-    // wave instead of a group of lanes
+    // in the team's kernel, candidates and moves of higher degree are taken by a
+    // whole wave instead of a group of lanes
     int64_t wg_big_deg = 32;
+    // polls of a team's first workgroup before it gives up waiting for the
+    // others (some 0.1 s; 0: every team of more than one workgroup is given up)
+    int64_t team_start_spins = 1 << 18;
     // "small" levels: every connectivity row is built by a wave, the
     // afterburner takes ab_lanes_small times its lanes per candidate, and the
     // rebalancers' select kernels run 128-thread workgroups
