@@ -386,6 +386,8 @@ int jet_partition_batch(jet_ctx_t* ctx, int32_t count, const jet_config_t* cfgs,
  * "team_start_spins": polls of a team's first workgroup before it gives up
  *   waiting for the others (0-4194304; 0: no team of more than one workgroup);
  *   the call then takes the paths of larger levels;
+ * "team_launch_iters": refinement iterations of a level that one launch of a
+ *   team runs (1-65536); longer levels go on in another launch;
  * "wg_big_deg": in that team's kernel, items above this degree take a whole
  *   wave;
  * "small_level_n": levels treated as small (wave-built connectivity rows,

@@ -3086,8 +3086,8 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
     P.tol = p_.tol;
     P.ntemps = (int32_t)temps.size();
     for (size_t i = 0; i < temps.size(); i++) P.temps[i] = temps[i];
-    P.cut = cut_;
-    P.imb = total_imb_;
+    P.start.curr_cut = P.start.best_cut = cut_;
+    P.start.curr_imb = P.start.best_imb = total_imb_;
     P.part = cur_part_;
     P.best_part = best_part;
     P.conn = team_conn_;
@@ -3112,20 +3112,36 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
     P.ctl = team_ctl_;
     P.host_out = mailbox_->dev + 16;
     volatile int64_t* out = mailbox_->host + 16;
-    P.seq = ++mailbox_->seq;
     P.team = team_size(g.n, g.m);
-    TeamSlot slot(P.team);
-    P.xcd = slot.xcd();
     P.start_spins = (int32_t)tuning().team_start_spins;
-    launch_refine_team(P, s_);
-    // without a result: no workgroup ran on the wanted XCD
-    const bool ran = wait_mailbox(&out[TEAM_OUT_WORDS], P.seq, s_);
-    const int64_t status = ran ? out[5] : LEVEL_ABANDONED, err = ran ? out[6] : 0;
-    if (status == LEVEL_ABANDONED) team_abandoned();
-    if (status == LEVEL_IRREGULAR) team_irregular_ = true;
-    if (status == LEVEL_ABANDONED || status == LEVEL_IRREGULAR) return false;
-    if (err) throw DeviceError(refine_error_text((int32_t)err));
-    if (status != LEVEL_DONE) throw DeviceError("team refinement made no progress");
+    // A launch ends after team_launch_iters iterations (about a second by
+    // default, which no level measured here reaches); the next one goes on from
+    // the state it left.
+    for (int tries = 0;;) {
+        P.seq = ++mailbox_->seq;
+        P.iter_cap = P.start.iterations + (int32_t)tuning().team_launch_iters;
+        TeamSlot slot(P.team);
+        P.xcd = slot.xcd();
+        launch_refine_team(P, s_);
+        // without a result: no workgroup ran on the wanted XCD
+        const bool ran = wait_mailbox(&out[TEAM_OUT_WORDS], P.seq, s_);
+        const int64_t status = ran ? out[5] : LEVEL_ABANDONED, err = ran ? out[6] : 0;
+        if (err) throw DeviceError(refine_error_text((int32_t)err));
+        if (status == LEVEL_DONE) break;
+        if (status == LEVEL_MORE) {
+            P.start = LevelState{out[7],           out[8],           out[0],          out[1],          (int32_t)out[9],
+                                 (int32_t)out[10], (int32_t)out[11], (int32_t)out[2], (int32_t)out[3], (int32_t)out[4]};
+            P.resume = 1;
+            tries = 0;
+            continue;
+        }
+        if (status == LEVEL_IRREGULAR) team_irregular_ = true;
+        if (status == LEVEL_ABANDONED) team_abandoned();
+        // a level that has begun can only go on where it was
+        if (P.resume && status == LEVEL_ABANDONED && ++tries < 100) continue;
+        if (!P.resume && (status == LEVEL_ABANDONED || status == LEVEL_IRREGULAR)) return false;
+        throw DeviceError("team refinement made no progress");
+    }
     cut_ = out[0];
     total_imb_ = out[1];
     rec.iterations = (int32_t)out[2];

@@ -39,7 +39,9 @@ struct TeamParams {
     double tol;
     int32_t ntemps;
     double temps[TEAM_MAX_TEMPS];
-    int64_t cut, imb;  // of the partition the level starts from
+    LevelState start;
+    int32_t resume;     // the level goes on from `start` (LEVEL_MORE); else from best_part
+    int32_t iter_cap;   // iterations of the level after which the launch ends
     part_t* part;
     part_t* best_part;  // in: the level's partition; out: the best one
     int2* conn;         // m slots: the table of row i starts at slot rowptr[i]
@@ -66,7 +68,10 @@ struct TeamParams {
     int64_t seq;
 };
 
-constexpr int TEAM_OUT_WORDS = 7;  // best cut, best imbalance, iterations, LP iterations, changed, status, error bits
+// best cut, best imbalance, iterations, LP iterations, changed, status, error
+// bits; then what a continued level starts from: current cut and imbalance,
+// temperature, count, balance counter
+constexpr int TEAM_OUT_WORDS = 12;
 // Levels of more edges are refined by a team only when no row is longer.
 constexpr int64_t TEAM_REGULAR_M = 100000;
 constexpr int32_t TEAM_MAX_DEG = 128;
@@ -80,8 +85,9 @@ int32_t team_size(int64_t n, int64_t m);
 // published to p.host_out; status LEVEL_ABANDONED (or a finished stream without
 // a result) means that no team could start: the level's arrays are untouched.
 // LEVEL_IRREGULAR: the level has rows of more than TEAM_MAX_DEG edges, and too
-// many edges (likewise nothing has changed).
-enum : int32_t { LEVEL_DONE = 0, LEVEL_STALLED = 2, LEVEL_ABANDONED = 3, LEVEL_IRREGULAR = 4 };
+// many edges (likewise nothing has changed). LEVEL_MORE: iter_cap was reached;
+// a launch with `resume` and the published state goes on.
+enum : int32_t { LEVEL_DONE = 0, LEVEL_MORE = 1, LEVEL_STALLED = 2, LEVEL_ABANDONED = 3, LEVEL_IRREGULAR = 4 };
 void launch_refine_team(TeamParams p, hipStream_t s);
 
 }  // namespace jet

@@ -32,7 +32,6 @@ namespace jet {
 // of more than 10,000 vertices (mesh of 65,536: 30 against 22 us an iteration).
 constexpr int TM_BLOCK = 1024;
 constexpr int TM_WAVES = TM_BLOCK / WAVE;
-constexpr int32_t TM_ITER_CAP = 1 << 16;
 constexpr int32_t TM_LANES = 16;             // lanes that build a row of at most TM_SMALL edges
 constexpr int32_t TM_SMALL = 64;
 constexpr int32_t TM_TABLE = 256;            // table slots of a wave: WAVE / TM_LANES * TM_SMALL, and TEAM_MAX_K
@@ -236,16 +235,18 @@ __device__ inline int32_t tm_walk(const int64_t* es, int32_t lo, int32_t hi, int
 
 // The next step of the temperature loop of :1095-1134: `for (fr : temps) {
 // count = 0; while (count++ <= 11) ... }` as the state (temp_idx, count).
-__device__ inline void tm_next_step(TeamShared& L, int32_t ntemps) {
+__device__ inline void tm_next_step(TeamShared& L, int32_t ntemps, int32_t iter_cap) {
     LevelState& S = L.S;
     if (S.count > 11) {
         S.temp_idx++;
         S.count = 0;
     }
     L.done = S.temp_idx >= ntemps ? 1 : 0;
-    if (!L.done && S.iterations >= TM_ITER_CAP) {
-        S.status = LEVEL_STALLED;
+    if (!L.done && S.iterations >= iter_cap) {
+        // the next launch takes this step again, from this state
+        S.status = LEVEL_MORE;
         L.done = 1;
+        return;
     }
     S.count++;
     if (!L.done) S.iterations++;
@@ -259,6 +260,11 @@ __device__ inline void tm_publish(const TeamParams& P, const LevelState& S, int3
     P.host_out[4] = S.changed;
     P.host_out[5] = S.status;
     P.host_out[6] = err;
+    P.host_out[7] = S.curr_cut;
+    P.host_out[8] = S.curr_imb;
+    P.host_out[9] = S.temp_idx;
+    P.host_out[10] = S.count;
+    P.host_out[11] = S.balance_counter;
     __threadfence_system();
     P.host_out[TEAM_OUT_WORDS] = P.seq;  // the host waits for this word
     __threadfence_system();
@@ -267,12 +273,13 @@ __device__ inline void tm_publish(const TeamParams& P, const LevelState& S, int3
 }  // namespace
 
 __global__ void __launch_bounds__(256) k_team_prep(RefineCtl* ctl, int32_t* buckets, int32_t nb, int64_t* sizes,
-                                                  const int64_t* best_sizes, int32_t k) {
+                                                  const int64_t* best_sizes, int32_t k, int32_t resume) {
     const int32_t t = blockIdx.x * 256 + threadIdx.x;
     constexpr int32_t W = sizeof(RefineCtl) / 4;
     if (t < W) reinterpret_cast<int32_t*>(ctl)[t] = 0;
     for (int32_t x = t; x < nb; x += gridDim.x * 256) buckets[x] = 0;
-    for (int32_t x = t; x < k; x += gridDim.x * 256) sizes[x] = best_sizes[x];
+    if (!resume)
+        for (int32_t x = t; x < k; x += gridDim.x * 256) sizes[x] = best_sizes[x];
 }
 
 __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
@@ -297,8 +304,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
             S.status = LEVEL_ABANDONED;
             tm_publish(P, S, 0);
         }
-        S.curr_cut = S.best_cut = P.cut;
-        S.curr_imb = S.best_imb = P.imb;
+        S = P.start;
         S.status = LEVEL_DONE;
         L.S = S;
     }
@@ -316,7 +322,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
     };
 
     // ------------------------------------------------------------ initial state
-    {
+    if (!P.resume) {
         int32_t mx = 0;
         for_own([&](vid_t i, bool in) {
             if (!in) return;
@@ -337,14 +343,14 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
             }
         }
     }
-    for (int32_t p = t; p < k; p += TM_BLOCK) L.sizes[p] = P.best_sizes[p];
-    tm_build_rows(P, P.best_part, false, reinterpret_cast<int2*>(dyn), L.used, T, me);
+    for (int32_t p = t; p < k; p += TM_BLOCK) L.sizes[p] = P.resume ? P.sizes[p] : P.best_sizes[p];
+    if (!P.resume) tm_build_rows(P, P.best_part, false, reinterpret_cast<int2*>(dyn), L.used, T, me);
     if (t < 6) L.cnt[t] = 0;
     for (int32_t p = t; p < k; p += TM_BLOCK) L.delta[p] = 0;
     if (t == 0) {
         L.take = 0;
         L.cc = 0;
-        tm_next_step(L, P.ntemps);
+        tm_next_step(L, P.ntemps, P.iter_cap);
     }
     bool alive = team.sync();
     int b = 0;  // the step's set of sums
@@ -958,7 +964,7 @@ __global__ void __launch_bounds__(TM_BLOCK) k_refine_team(TeamParams P) {
                     S.changed = 1;
                 }
                 L.take = take;
-                tm_next_step(L, P.ntemps);
+                tm_next_step(L, P.ntemps, P.iter_cap);
             }
         }
         if (!(alive = team.sync())) break;
@@ -1031,7 +1037,7 @@ void launch_refine_team(TeamParams p, hipStream_t s) {
     p.own = 64;
     while (p.own > 8 && ceil_div(p.g.n, p.own) < 4 * (int64_t)p.team) p.own /= 2;
     k_team_prep<<<(int)std::max<int64_t>(1, ceil_div(p.nbk + 1, 1024)), 256, 0, s>>>(p.ctl, p.buckets, p.nbk + 1,
-                                                                                    p.sizes, p.best_sizes, p.k);
+                                                                                    p.sizes, p.best_sizes, p.k, p.resume);
     k_refine_team<<<p.team == 1 ? 1 : 8 * p.team, TM_BLOCK, team_lds(p), s>>>(p);
     JET_LAUNCH_CHECK();
 }

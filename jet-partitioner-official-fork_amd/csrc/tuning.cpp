@@ -44,6 +44,7 @@ const Field kFields[] = {
     {"sel_max_blocks", &Tuning::sel_max_blocks, 64, 65536},
     {"sel_copy_wgs", &Tuning::sel_copy_wgs, 1, 65536},
     {"team_start_spins", &Tuning::team_start_spins, 0, 1 << 22},
+    {"team_launch_iters", &Tuning::team_launch_iters, 1, 1 << 16},
 };
 std::mutex g_mu;
 // fields set through jet_tuning_set: the table applied at context creation

@@ -24,6 +24,8 @@ struct Tuning {
     // polls of a team's first workgroup before it gives up waiting for the
     // others (some 0.1 s; 0: every team of more than one workgroup is given up)
     int64_t team_start_spins = 1 << 18;
+    // iterations of a level that one launch of a team runs at most
+    int64_t team_launch_iters = 1 << 16;
     // "small" levels: every connectivity row is built by a wave, the
     // afterburner takes ab_lanes_small times its lanes per candidate, and the
     // rebalancers' select kernels run 128-thread workgroups
