@@ -18,7 +18,9 @@ void copy_i64(int64_t* dst, const int64_t* src, int64_t n, hipStream_t s);
 // Pinned, device-mapped host words owned by the calling thread (allocated on
 // first use, MAILBOX_SLOTS of them). A kernel stores a result there with a
 // system-scope fence and the host reads it after synchronising the stream:
-// no copy command and no staging buffer on the way.
+// no copy command and no staging buffer on the way. Results that the host polls
+// for lie in one 64-byte line (8 words) with the sequence word it waits for:
+// words of another line have been seen older than it.
 constexpr int MAILBOX_SLOTS = 64;
 struct Mailbox {
     int64_t* host = nullptr;

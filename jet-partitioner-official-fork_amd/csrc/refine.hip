@@ -3110,8 +3110,8 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
     P.best_sizes = best_sizes_;
     P.evict_adjust = evict_adjust_;
     P.ctl = team_ctl_;
-    P.host_out = mailbox_->dev + 16;
-    volatile int64_t* out = mailbox_->host + 16;
+    P.host_out = mailbox_->dev + TEAM_MAILBOX;
+    volatile int64_t* out = mailbox_->host + TEAM_MAILBOX;
     P.team = team_size(g.n, g.m);
     P.start_spins = (int32_t)tuning().team_start_spins;
     // A launch ends after team_launch_iters iterations (about a second by
@@ -3125,12 +3125,23 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
         launch_refine_team(P, s_);
         // without a result: no workgroup ran on the wanted XCD
         const bool ran = wait_mailbox(&out[TEAM_OUT_WORDS], P.seq, s_);
-        const int64_t status = ran ? out[5] : LEVEL_ABANDONED, err = ran ? out[6] : 0;
-        if (err) throw DeviceError(refine_error_text((int32_t)err));
+        const int64_t bits = ran ? out[6] : LEVEL_ABANDONED;
+        const int32_t status = (int32_t)(bits & 0xffff), err = ran ? (int32_t)out[5] : 0;
+        if (err) throw DeviceError(refine_error_text(err));
+        if (status == LEVEL_DONE || status == LEVEL_MORE)
+            P.start = LevelState{out[2],
+                                 out[3],
+                                 out[0],
+                                 out[1],
+                                 (int32_t)(bits >> 32 & 0xffff),
+                                 (int32_t)(bits >> 48 & 0xffff),
+                                 (int32_t)(out[5] >> 32),
+                                 (int32_t)out[4],
+                                 (int32_t)(out[4] >> 32),
+                                 (int32_t)(bits >> 16 & 0xffff),
+                                 status};
         if (status == LEVEL_DONE) break;
         if (status == LEVEL_MORE) {
-            P.start = LevelState{out[7],           out[8],           out[0],          out[1],          (int32_t)out[9],
-                                 (int32_t)out[10], (int32_t)out[11], (int32_t)out[2], (int32_t)out[3], (int32_t)out[4]};
             P.resume = 1;
             tries = 0;
             continue;
@@ -3142,12 +3153,13 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
         if (!P.resume && (status == LEVEL_ABANDONED || status == LEVEL_IRREGULAR)) return false;
         throw DeviceError("team refinement made no progress");
     }
-    cut_ = out[0];
-    total_imb_ = out[1];
-    rec.iterations = (int32_t)out[2];
-    rec.lp_iterations = (int32_t)out[3];
+    const LevelState& S = P.start;
+    cut_ = S.best_cut;
+    total_imb_ = S.best_imb;
+    rec.iterations = S.iterations;
+    rec.lp_iterations = S.lp_iterations;
     gen_ += rec.iterations;
-    if (out[4]) changed_ = true;
+    if (S.changed) changed_ = true;
     rec.cut2 = cut_;
     rec.total_imb = total_imb_;
     rec.n = g.n;

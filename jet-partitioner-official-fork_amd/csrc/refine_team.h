@@ -68,10 +68,15 @@ struct TeamParams {
     int64_t seq;
 };
 
-// best cut, best imbalance, iterations, LP iterations, changed, status, error
-// bits; then what a continued level starts from: current cut and imbalance,
-// temperature, count, balance counter
-constexpr int TEAM_OUT_WORDS = 12;
+// Best cut, best imbalance, current cut, current imbalance; then pairs of 32
+// bits (low, high): iterations and LP iterations, error bits and balance
+// counter, and in 16 bits each status, changed, temperature, count. With the
+// sequence word they fill one 64-byte line: the host has seen words of another
+// line older than the sequence word written after them, in spite of the fence
+// between (one in some 300 batches of 24 graphs; none with one line).
+constexpr int TEAM_OUT_WORDS = 7;
+constexpr int TEAM_MAILBOX = 16;  // their place in the thread's mailbox
+static_assert(TEAM_MAILBOX % 8 == 0 && TEAM_OUT_WORDS < 8, "one 64-byte line");
 // Levels of more edges are refined by a team only when no row is longer.
 constexpr int64_t TEAM_REGULAR_M = 100000;
 constexpr int32_t TEAM_MAX_DEG = 128;

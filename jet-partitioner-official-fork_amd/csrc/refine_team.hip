@@ -255,16 +255,11 @@ __device__ inline void tm_next_step(TeamShared& L, int32_t ntemps, int32_t iter_
 __device__ inline void tm_publish(const TeamParams& P, const LevelState& S, int32_t err) {
     P.host_out[0] = S.best_cut;
     P.host_out[1] = S.best_imb;
-    P.host_out[2] = S.iterations;
-    P.host_out[3] = S.lp_iterations;
-    P.host_out[4] = S.changed;
-    P.host_out[5] = S.status;
-    P.host_out[6] = err;
-    P.host_out[7] = S.curr_cut;
-    P.host_out[8] = S.curr_imb;
-    P.host_out[9] = S.temp_idx;
-    P.host_out[10] = S.count;
-    P.host_out[11] = S.balance_counter;
+    P.host_out[2] = S.curr_cut;
+    P.host_out[3] = S.curr_imb;
+    P.host_out[4] = (int64_t)S.lp_iterations << 32 | (uint32_t)S.iterations;
+    P.host_out[5] = (int64_t)S.balance_counter << 32 | (uint32_t)err;
+    P.host_out[6] = (int64_t)S.count << 48 | (int64_t)S.temp_idx << 32 | S.changed << 16 | S.status;
     __threadfence_system();
     P.host_out[TEAM_OUT_WORDS] = P.seq;  // the host waits for this word
     __threadfence_system();
