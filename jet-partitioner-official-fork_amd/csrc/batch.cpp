@@ -81,10 +81,15 @@ struct jet_ctx {
 
 namespace {
 
-// Upper estimate of a job's device memory: the staged input (int64 offsets,
+// Estimate of a job's device memory: the staged input (int64 offsets,
 // int32 columns and weights), the coarse hierarchy (at most the input again),
 // the refiner's tables (8 bytes per slot, slots <= m) and per-vertex arrays,
-// and contraction temporaries (radix keys of the spill path).
+// and contraction temporaries (radix keys of the spill path); the device's
+// coarsening for the initial partition runs without the refiner's and takes
+// less (8 bytes an entry for the rows built and as much for its arrays). Of
+// twelve graphs of 256 to 1,000,000 vertices, eleven held 0.20 to 0.96 of it at
+// most; a hierarchy of many levels that hardly shrink (plain matching of an
+// R-MAT graph) 2.6 times, a graph whose long rows all spill 1.4 times.
 int64_t footprint_of(int64_t n, int64_t m) { return 128 * n + 48 * m + (int64_t(1) << 20); }
 
 void worker_loop(jet_ctx* X, jet::Context* E) {

@@ -460,8 +460,9 @@ bool init_coarsen_device(const DGraph& g, std::vector<int32_t>& vw, uint64_t see
     vid_t* tkey = a.alloc<vid_t>(g.m);
     wgt_t* tval = a.alloc<wgt_t>(g.m);
     if (h[3] > 0) {
-        // at most 1 GB of position and weight arrays
-        const int64_t fit = std::max<int64_t>(1, (int64_t(1) << 30) / (8 * (int64_t)nc));
+        // at most 1 GB of position and weight arrays, and no more than the
+        // level's columns and weights take
+        const int64_t fit = std::max<int64_t>(1, std::min<int64_t>(int64_t(1) << 30, 8 * (int64_t)g.m) / (8 * (int64_t)nc));
         const int G = (int)std::min<int64_t>({(int64_t)h[3], 512, fit});
         ArenaScope sd(a);
         int32_t* dense = a.alloc<int32_t>((int64_t)G * 2 * nc);

@@ -332,7 +332,7 @@ static void uncoarsen_levels(Context& C, const jet_config_t& cfg, const std::vec
     {
         ArenaScope rscope(C.scratch);
         int64_t cap = conn_capacity(fine.n, fine.rowptr, k, C.scratch, s);
-        Refiner ref(C.scratch, s, fine.n, cap, rp);
+        Refiner ref(C.scratch, s, fine.n, fine.m, cap, rp);
         // A level that shares its graph with the level just refined (the
         // coarsening fixed point) starts from that level's output partition
         // and refine_data. When that level changed neither, this level
@@ -508,7 +508,7 @@ static void initial_partition_multilevel(Context& C, const jet_config_t& cfg, co
     rp.ultra = cfg.ultra_settings != 0;
     ArenaScope rscope(C.scratch);
     int64_t cap = conn_capacity(D[0].n, D[0].rowptr, k, C.scratch, s);
-    Refiner ref(C.scratch, s, D[0].n, cap, rp);
+    Refiner ref(C.scratch, s, D[0].n, D[0].m, cap, rp);
     part_t* cur = C.persist.alloc<part_t>(D.back().n);
     JET_HIP(hipMemcpyAsync(cur, hp.data(), sizeof(int32_t) * D.back().n, hipMemcpyHostToDevice, s));
     for (size_t L = D.size(); L-- > 0;) {
@@ -852,7 +852,7 @@ int jet_conn_tables(int64_t n, const int64_t* row_offsets, const int32_t* col, c
         RefineParams rp;
         rp.k = k;
         int64_t cap = conn_capacity(L.n, L.rowptr, k, C.scratch, C.stream);
-        Refiner ref(C.scratch, C.stream, L.n, cap, rp);
+        Refiner ref(C.scratch, C.stream, L.n, L.m, cap, rp);
         std::vector<int64_t> off;
         std::vector<int32_t> sp, sv, sz;
         ref.conn_tables(L, dp, off, sp, sv, sz);
@@ -879,7 +879,7 @@ int jet_refine_step(int32_t kind, int64_t n, const int64_t* row_offsets, const i
         rp.k = k;
         rp.imb = imb;
         int64_t cap = conn_capacity(L.n, L.rowptr, k, C.scratch, C.stream);
-        Refiner ref(C.scratch, C.stream, L.n, cap, rp);
+        Refiner ref(C.scratch, C.stream, L.n, L.m, cap, rp);
         std::vector<int32_t> mv, de;
         ref.single_step(L, dp, kind, filter_ratio, mv, de);
         std::copy(mv.begin(), mv.end(), moves_out);
@@ -917,7 +917,7 @@ int jet_refine_level_trace(int64_t n, const int64_t* row_offsets, const int32_t*
         rp.tol = tol;
         rp.ultra = ultra != 0;
         int64_t cap = conn_capacity(L.n, L.rowptr, k, C.scratch, C.stream);
-        Refiner ref(C.scratch, C.stream, L.n, cap, rp);
+        Refiner ref(C.scratch, C.stream, L.n, L.m, cap, rp);
         std::vector<std::array<int64_t, 6>> tr;
         if (iters_out) ref.trace = &tr;
         LevelRecord rec = ref.refine(L, dp);
@@ -1051,7 +1051,7 @@ int jet_partition_quality(int64_t n, const int64_t* row_offsets, const int32_t* 
         RefineParams rp;
         rp.k = k;
         int64_t cap = conn_capacity(L.n, L.rowptr, k, C.scratch, C.stream);
-        Refiner ref(C.scratch, C.stream, L.n, cap, rp);
+        Refiner ref(C.scratch, C.stream, L.n, L.m, cap, rp);
         int64_t comm = 0;
         std::vector<int64_t> cpp;
         ref.quality(L, dp, comm, cpp);
@@ -1087,7 +1087,7 @@ int jet_cut_heatmap(int64_t n, const int64_t* row_offsets, const int32_t* col, c
         RefineParams rp;
         rp.k = k;
         int64_t cap = conn_capacity(L.n, L.rowptr, k, C.scratch, C.stream);
-        Refiner ref(C.scratch, C.stream, L.n, cap, rp);
+        Refiner ref(C.scratch, C.stream, L.n, L.m, cap, rp);
         ref.heatmap(L, dp, dh);
         from_device(C, heat_out, dh, kk, ptr_space);
     });

@@ -35,7 +35,7 @@ struct BestCopy;
 // and the refine_data persisting across levels (jet_refiner.hpp:100-106).
 class Refiner {
   public:
-    Refiner(Arena& a, hipStream_t s, vid_t finest_n, int64_t finest_conn_cap, const RefineParams& p);
+    Refiner(Arena& a, hipStream_t s, vid_t finest_n, int64_t finest_m, int64_t finest_conn_cap, const RefineParams& p);
     ~Refiner() = default;
     Refiner(const Refiner&) = delete;
     Refiner& operator=(const Refiner&) = delete;
@@ -186,9 +186,7 @@ class Refiner {
     int64_t* bcopies_ = nullptr;  // ncopies_ - 1 more bucket arrays, kept zero between uses
     int32_t ncopies_ = 1;
     int64_t nbuckets_ = 0;
-    // the team kernel's tables (rows at their adjacency's offset), control
-    // words and scratch
-    int2* team_conn_ = nullptr;
+    // the team kernel's control words and scratch
     RefineCtl* team_ctl_ = nullptr;
     int32_t* team_buckets_ = nullptr;
     uint64_t* team_rkey_ = nullptr;

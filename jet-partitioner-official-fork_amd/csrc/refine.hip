@@ -2445,7 +2445,8 @@ static void allow_pull_lds() {
     JET_HIP(rc[dev]);
 }
 
-Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefineParams& p) : a_(a), s_(s), p_(p), nmax_(n) {
+Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t m, int64_t cap, const RefineParams& p)
+    : a_(a), s_(s), p_(p), nmax_(n) {
     if (p.k < 1 || p.k > MAX_K) throw std::invalid_argument("k out of range");
     if (2 * sizeof(int2) * (size_t)p.k > 65536) {
         // dynamic LDS above 64 KB must be allowed per kernel (gfx950 has 160 KB)
@@ -2455,7 +2456,6 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     allow_pull_lds();
     int64_t N = std::max<int64_t>(n, 1);
     conn_off_ = a.alloc<eoff_t>(N + 1);
-    conn_ = a.alloc<int2>(std::max<int64_t>(cap, 1));
     conn_size_ = a.alloc<int32_t>(N);
     dest_cache_ = a.alloc<part_t>(N);
     lock_ = a.alloc<int32_t>(N);
@@ -2496,7 +2496,9 @@ Refiner::Refiner(Arena& a, hipStream_t s, vid_t n, int64_t cap, const RefinePara
     bcopies_ = a.alloc<int64_t>(std::max<int64_t>(1, nbuckets_ * (ncopies_ - 1)));
     moved_bits_ = a.alloc<uint32_t>((N + 31) / 32);
     cand_bits_ = a.alloc<uint64_t>((N + WAVE - 1) / WAVE);
-    team_conn_ = a.alloc<int2>(TEAM_MAX_M);
+    // tables of a level on the kernels (cap slots on the finest) or on a team,
+    // whose rows start at their adjacency's offset: at most m slots either way
+    conn_ = a.alloc<int2>(std::max<int64_t>({cap, std::min<int64_t>(m, TEAM_MAX_M), 1}));
     team_ctl_ = a.alloc<RefineCtl>(1);
     team_buckets_ = a.alloc<int32_t>(TEAM_MAX_NBK + 1);
     team_rkey_ = a.alloc<uint64_t>(std::min<int64_t>(N, TEAM_MAX_N));
@@ -3090,7 +3092,7 @@ bool Refiner::refine_team(const Level& L, part_t* best_part, const std::vector<d
     P.start.curr_imb = P.start.best_imb = total_imb_;
     P.part = cur_part_;
     P.best_part = best_part;
-    P.conn = team_conn_;
+    P.conn = conn_;
     P.conn_size = conn_size_;
     P.dest_cache = dest_cache_;
     P.lock = lock_;
