@@ -611,6 +611,8 @@ def main():
                      "refine": round(st.refine_s, 4), "levels": st.num_levels} if st else None,
         "roofline": roofline,
         "kernel_families": families,
+        "kernel_families_path": "multi-kernel on every level (levels of up to 65,536 vertices of the timed "
+                                "partitions run on one-launch teams)",
         "end_to_end": e2e,
         "cpu_baseline": cpu,
         "pcie_inclusive": pcie,

@@ -394,9 +394,9 @@ int jet_partition_batch(jet_ctx_t* ctx, int32_t count, const jet_config_t* cfgs,
  *   wider afterburner lane groups, 128-thread rebalancer select workgroups);
  * "ab_lanes_small", "upd_lanes": lane-group multipliers (1-4) of the
  *   afterburner on small levels and of the update passes;
- * "upd_big_slices": moves and candidates of degree above 128 times this (1-64)
- *   are taken by a whole workgroup in the update passes and the afterburner,
- *   others of degree above 64 by a wave;
+ * "upd_big_slices": rows of degree above 128 times this (1-64) are taken by a
+ *   whole workgroup in the afterburner and by a wave per 1024 edges in the
+ *   update passes, others of degree above 64 by a wave;
  * "lp_one_pass_n": LP select runs one pass per wave up to this level size;
  * "ct_wave_max", "ct_block_max": contraction rows of up to this many fine
  *   entries take the one-wave (<= 128) or one-workgroup (<= 4096) LDS table;
@@ -405,7 +405,8 @@ int jet_partition_batch(jet_ctx_t* ctx, int32_t count, const jet_config_t* cfgs,
  * "sel_max_blocks": the rebalancers' select kernels run at most this many
  *   workgroups (64-65536), each over a contiguous range of vertices;
  * "sel_copy_wgs": and flush their bucket sums into one copy of the bucket
- *   array per this many workgroups (1-65536; at most 16 copies).
+ *   array per this many workgroups (1-65536; at most 16 copies), with up to 64
+ *   parts per at most 32 to 64 workgroups.
  * jet_tuning_set / jet_tuning_get return JET_EINVAL for an unknown name or a
  * value out of range; jet_tuning_load applies a table file ("name value"
  * lines, '#' comments) and returns JET_EINVAL, applying nothing, when it

@@ -417,10 +417,12 @@ __global__ void __launch_bounds__(BB_BLOCK)
 // kernels, one after another of its lanes' long tables: a lane that reads 256
 // slots alone takes 64 dependent trips to memory, for which its wave waits.
 // That pays where the waves wait for memory anyway: R-MAT 22 (k = 256), LP
-// select 1.06 -> 0.86 ms on 4,194,304 vertices, 0.49 -> 0.31 on 756,505 and
-// 0.19 -> 0.15 on 438,484, but 98 -> 141 us on 370,878; strong select 0.90 ->
-// 0.37, 0.15 -> 0.10, 0.08 -> 0.06 ms and 70 -> 82 us. The weak select's four
-// vertices a lane hide the trips as they are (0.15 -> 0.20 ms on 756,505).
+// select 1.06 -> 0.86 ms on 4,194,304 vertices and 0.49 -> 0.31 on 756,505, but
+// 98 -> 141 us on 370,878; strong select 0.90 -> 0.37, 0.15 -> 0.10 and, on
+// 438,484 vertices, 0.08 -> 0.06 ms, but 70 -> 82 us on 370,878. (LP select has
+// the variant in its two-pass shape only, above lp_one_pass_n vertices.) The
+// weak select's four vertices a lane hide the trips as they are (0.15 -> 0.20 ms
+// on 756,505).
 constexpr int32_t SEL_LONG = 16;
 constexpr int64_t SEL_LONG_N = 400000;
 

@@ -51,7 +51,8 @@ struct Tuning {
     // contiguous range of vertices)
     int64_t sel_max_blocks = 1024;
     // and flush their bucket maps into one copy of the bucket array per this
-    // many workgroups (at most 16 copies)
+    // many workgroups (at most 16 copies; up to 64 parts, per at most 32 to 64:
+    // Refiner::rebalance)
     int64_t sel_copy_wgs = 256;
 };
 
